@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "sd_internal.hpp"
+#include "sd_readback.hpp"
 
 namespace sd {
 
@@ -152,6 +153,7 @@ struct sd_ctx {
     int* pcounters = nullptr;
     hipStream_t hside = nullptr;
     hipEvent_t hev_fork = nullptr, hev_join = nullptr;
+    HostStage stage;  // pinned staging of the read-backs
 };
 
 namespace {
@@ -165,6 +167,7 @@ void drop_graphs(sd_ctx* c) {
 
 void release(sd_ctx* c) {
     drop_graphs(c);
+    stage_release(c->stage);
     void* bufs[] = {c->pos[0], c->pos[1], c->vel[0], c->vel[1], c->omg[0], c->omg[1], c->ids[0], c->ids[1],
                     c->posB, c->k32[0], c->k32[1], c->v32[0], c->v32[1], c->k64[0], c->k64[1], c->sort_tmp,
                     c->cell_start, c->hcount[0], c->hcount[1], c->hist[0], c->hist[1], c->overflow, c->diag,
@@ -1000,29 +1003,11 @@ extern "C" sd_status sd_ctx_download_spheres(sd_ctx* c, float* x, float* y, floa
                                              float* wx, float* wy, float* wz) {
     SD_REQUIRE(c, "sd_ctx_download_spheres: NULL context");
     if (c->n == 0) return set_error(SD_ERR_STATE, "sd_ctx_download_spheres: no spheres uploaded");
-    const int n = c->n;
-    std::vector<float4> pos(n), vel(n), omg(n);
-    std::vector<int> ids(n);
     const int cs = c->cur_state;
-    SD_HIP(hipMemcpyAsync(pos.data(), c->pos[cs], n * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    SD_HIP(hipMemcpyAsync(vel.data(), c->vel[cs], n * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    SD_HIP(hipMemcpyAsync(omg.data(), c->omg[cs], n * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    SD_HIP(hipMemcpyAsync(ids.data(), c->ids[cs], n * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SD_HIP(hipStreamSynchronize(c->stream));
-    for (int s = 0; s < n; ++s) {
-        const int i = ids[s];
-        if (i < 0 || i >= n) return set_error(SD_ERR_STATE, "sd_ctx_download_spheres: corrupt id %d", i);
-        if (x) x[i] = pos[s].x;
-        if (y) y[i] = pos[s].y;
-        if (z) z[i] = pos[s].z;
-        if (vx) vx[i] = vel[s].x;
-        if (vy) vy[i] = vel[s].y;
-        if (vz) vz[i] = vel[s].z;
-        if (wx) wx[i] = omg[s].x;
-        if (wy) wy[i] = omg[s].y;
-        if (wz) wz[i] = omg[s].z;
-    }
-    return SD_OK;
+    float* const out[9] = {x, y, z, vx, vy, vz, wx, wy, wz};
+    // the other state buffer holds nothing between steps: its ids serve as scratch
+    return readback_spheres(c->stage, c->pos[cs], c->vel[cs], c->omg[cs], c->ids[cs], c->n, c->ids[1 - cs], out,
+                            c->stream);
 }
 
 static sd_status diag_values(sd_ctx* c, double out[DIAG_VALUES]) {
