@@ -237,12 +237,14 @@ sd_status sd_ctx_step(sd_ctx* ctx, int nsteps);
  * every cell), [2] permute, [3] fused contact + integrate + next keys. With u64
  * keys, [0] is the re-sort from the previous order (positions permuted and
  * cell starts updated in the same pass; [1] is empty) when at most 1024
- * spheres changed cell in the previous step, else the radix sort (all passes),
+ * spheres (one in 256, up to 16384, of more than 262,144) changed cell in the
+ * previous step, else the radix sort (all passes),
  * and the positions are then permuted within [1]; [2] is empty. */
 sd_status sd_ctx_profile(sd_ctx* ctx, int nsteps, float* stage_ms, int nstages);
 /* Spheres that changed cell in the last step (u64 keys; 0 with u32 keys):
  * *full_next = 1 if the next step uses the full radix sort (more than 1024
- * changes, or after upload / load), else 0. Diagnostic with no counterpart in
+ * changes, or one in 256 up to 16384 of more than 262,144 spheres, or after
+ * upload / load), else 0. Diagnostic with no counterpart in
  * the reference, whose sort does not depend on the previous order. */
 sd_status sd_ctx_cell_changes(sd_ctx* ctx, int* count, int* full_next);
 /* Host arrays in particle-id order (any pointer may be NULL). */

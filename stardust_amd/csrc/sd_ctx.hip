@@ -113,7 +113,7 @@ struct sd_ctx {
     int cur_hist = 0;
     int* overflow = nullptr;
     // spheres that changed cell in the last step (u64 keys): count (set above
-    // RESORT_CAP to force the full sort), new and old keys, and the same sorted
+    // the cap to force the full sort), new and old keys, and the same sorted
     int* mcount = nullptr;
     uint64_t* mnew = nullptr;
     uint64_t* mold = nullptr;
@@ -209,7 +209,7 @@ sd_status dalloc(T** p, size_t count) {
 // Enqueues one step on the context stream. If ev is given, ev[0..4] are
 // recorded before the sort and after the sort, cell-start, permute and contact stages.
 // full (u64 keys): the radix sort instead of the re-sort from the previous
-// order. A re-sort step that finds more than RESORT_CAP changed cells is given
+// order. A re-sort step that finds more than resort_cap(n) changed cells is given
 // up on the device (step_ctl[0]), together with every later step of the same
 // launch sequence; the host then redoes it as a full step (run_steps).
 sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
@@ -261,7 +261,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
                                            c->items, nullptr, 0);
         } else {
             // also updates the cell starts and sets mc_write = 0
-            st = launch_resort_u64(mc_read, c->mnew, c->mold, c->msn, c->mso, K, n, c->cell_start, c->n_cells,
+            st = launch_resort_u64(mc_read, resort_cap(n), c->mnew, c->mold, c->msn, c->mso, K, n, c->cell_start, c->n_cells,
                                    c->pos[so], c->posB, Ka, mc_write, c->step_ctl, s);
             uint64_t* t = K;
             K = Ka;
@@ -280,7 +280,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
         a.mcount = mc_write;
         a.mnew = c->mnew;
         a.mold = c->mold;
-        a.mcap = RESORT_CAP;
+        a.mcap = resort_cap(n);
         a.step_ctl = c->step_ctl;
         a.scenes = c->scenes_d;
         a.scene_of = c->scene_of;
@@ -444,7 +444,7 @@ sd_status run_steps(sd_ctx* c, int nsteps) {
             int m = 0;
             SD_HIP(hipMemcpyAsync(&m, c->mcount + c->cur_hist, sizeof(int), hipMemcpyDeviceToHost, c->stream));
             SD_HIP(hipStreamSynchronize(c->stream));
-            c->dense = m > RESORT_CAP;
+            c->dense = m > resort_cap(c->n);
         }
     }
     return SD_OK;
@@ -613,10 +613,10 @@ sd_status upload_state(sd_ctx* c, int n, const float* x, const float* y, const f
     ALLOC(c->hist[1], (size_t)maxc * n);
     ALLOC(c->overflow, 1);
     ALLOC(c->mcount, 2);
-    ALLOC(c->mnew, RESORT_CAP);
-    ALLOC(c->mold, RESORT_CAP);
-    ALLOC(c->msn, RESORT_CAP);
-    ALLOC(c->mso, RESORT_CAP);
+    ALLOC(c->mnew, resort_cap(n));
+    ALLOC(c->mold, resort_cap(n));
+    ALLOC(c->msn, resort_cap(n));
+    ALLOC(c->mso, resort_cap(n));
     ALLOC(c->step_ctl, 2);
     c->diag_blocks = div_up(n, DIAG_BLOCK) < 1024 ? div_up(n, DIAG_BLOCK) : 1024;
     ALLOC(c->diag, (size_t)c->diag_blocks * DIAG_VALUES);
@@ -827,7 +827,7 @@ extern "C" sd_status sd_ctx_profile(sd_ctx* c, int nsteps, float* stage_ms, int 
                 st = set_error(SD_ERR_HIP, "sd_ctx_profile: counter read failed");
                 break;
             }
-            full = m > RESORT_CAP;
+            full = m > resort_cap(c->n);
         }
         c->need_full = false;
         st = enqueue_step(c, ev, full);
@@ -1054,7 +1054,7 @@ extern "C" sd_status sd_ctx_cell_changes(sd_ctx* c, int* count, int* full_next) 
     int m = 0;  // written by the last step, read by the next one
     SD_HIP(hipMemcpyAsync(&m, c->mcount + c->cur_hist, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     SD_HIP(hipStreamSynchronize(c->stream));
-    *full_next = m > RESORT_CAP ? 1 : 0;
+    *full_next = m > resort_cap(c->n) ? 1 : 0;
     *count = m == 0x7fffffff ? 0 : m;
     return SD_OK;
 }

@@ -166,9 +166,15 @@ sd_status launch_contacts_straddle(const ContactArgs& a, hipStream_t s);
 // the spheres that changed cell (see sd_resort.hip): writes the sorted keys to
 // keys_out and the positions in that order to posB, turns cell_start (the
 // previous order's cell starts, n_cells + 1 entries) into the new order's and
-// sets *next_count = 0. With *mcount > RESORT_CAP it gives the step up instead
+// sets *next_count = 0. With *mcount > cap (= resort_cap(n)) it gives the step up instead
 // (step_ctl[0] = 1).
-constexpr int RESORT_CAP = 1024;
+// Most changed cells a re-sort takes: 1,024, and one sphere in 256 of larger
+// scenes up to 16,384. Ranking the movers grows with their square and the
+// radix sort it saves with n: at 4,194,304 spheres a re-sort of 1,000 movers
+// takes 38 us and the full sort with its cell starts 147; at 250,007 spheres 12
+// and 41. A fixed 1,024 sent a 4,194,304-sphere column whose spheres move at 0.5 m/s
+// to the full sort every few steps.
+inline int resort_cap(int n) { return n / 256 < 1024 ? 1024 : (n / 256 > 16384 ? 16384 : n / 256); }
 // sd_lbvh_build, and with pnode (2 per node) also the packed tree of a
 // stackless walk: (box low corner, left child or leaf index), (box high corner, rope)
 sd_status lbvh_build(const uint64_t* sorted_keys, int n, const float* lo4, const float* hi4, int* left, int* right,
@@ -177,7 +183,7 @@ sd_status lbvh_build(const uint64_t* sorted_keys, int n, const float* lo4, const
 // keys[i] = (morton30 of box i's centroid with its drop_bits lowest bits cleared) << 32 | i
 sd_status launch_morton(const float* lo4, const float* hi4, int n, const float* domain6, uint64_t* keys,
                         int drop_bits, hipStream_t s);
-sd_status launch_resort_u64(const int* mcount, const uint64_t* mnew, const uint64_t* mold, uint64_t* msorted_new,
+sd_status launch_resort_u64(const int* mcount, int cap, const uint64_t* mnew, const uint64_t* mold, uint64_t* msorted_new,
                             uint64_t* msorted_old, const uint64_t* keys, int n, int* cell_start, int n_cells,
                             const float4* pos_state, float4* posB, uint64_t* keys_out, int* next_count,
                             int* step_ctl, hipStream_t s);

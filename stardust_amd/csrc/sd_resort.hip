@@ -15,13 +15,13 @@
 //              the first read off the previous step's cell starts.
 // The result is the same array a stable radix sort of the keys produces, and
 // the positions are permuted into that order in the same pass. With more than
-// RESORT_CAP changes the step is given up: step_ctl[0] is set, every later
+// resort_cap(n) changes the step is given up: step_ctl[0] is set, every later
 // kernel of the launch sequence returns at once (the state is untouched), and
 // the host redoes that step with the full radix sort.
 //
 // Replaces nothing in the reference (which re-sorts from scratch every step,
 // src/engine/cuda/sh_collision_detection.cu:310-360); the full radix sort runs
-// instead whenever more than RESORT_CAP spheres changed cell, and after every
+// instead whenever more than resort_cap(n) spheres changed cell, and after every
 // upload, load or restore.
 #include "sd_grid_dev.hpp"
 #include "sd_internal.hpp"
@@ -29,49 +29,75 @@
 namespace sd {
 
 constexpr int RESORT_MERGE_BLOCK = 512;
+constexpr int RANK_MOVERS = 64;  // movers ranked by one block
+constexpr int RANK_BLOCK = 256;  // four waves share the comparisons of 64 movers
+constexpr int MERGE_SLICE = 1024;  // new keys of one merge block held in LDS
 
-// One workgroup: sorts the movers' new and old keys (rank by counting, keys are
-// distinct) and places every mover.
-__global__ __launch_bounds__(RESORT_CAP) void k_resort_movers(
-    const int* __restrict__ mcount, const uint64_t* __restrict__ mnew, const uint64_t* __restrict__ mold,
+// Ranks the movers' new and old keys by counting (keys are distinct) and places
+// every mover, 64 movers a block. Counting is M^2 comparisons, so it is spread
+// over M / 64 blocks; what remains is the latency of dependent loads that miss
+// the cache after the contact kernel (count, keys, cell starts, positions). In
+// a 128-scene batch of 1.83M spheres with 900 movers a step one block for all
+// of them took 39 us, this form 12; a handful of movers 4.4 us in either.
+__global__ __launch_bounds__(RANK_BLOCK) void k_resort_movers(
+    const int* __restrict__ mcount, int cap, const uint64_t* __restrict__ mnew, const uint64_t* __restrict__ mold,
     uint64_t* __restrict__ msn, uint64_t* __restrict__ mso, int n, const int* __restrict__ cell_start,
     const float4* __restrict__ pos_state, float4* __restrict__ posB, uint64_t* __restrict__ keys_out,
     int* __restrict__ step_ctl) {
-    if (step_ctl[0]) return;  // an earlier step of this launch sequence was given up
-    const int M = *mcount;
-    if (M > RESORT_CAP) {  // too many changes: this step is given up (the host redoes it with the full sort)
-        if (threadIdx.x == 0) step_ctl[0] = 1;
+    const int given_up = step_ctl[0], M = *mcount;
+    if (given_up) return;  // an earlier step of this launch sequence was given up
+    if (M > cap) {  // too many changes: this step is given up (the host redoes it with the full sort)
+        if (blockIdx.x == 0 && threadIdx.x == 0) step_ctl[0] = 1;
         return;
     }
-    __shared__ uint64_t sn[RESORT_CAP], so[RESORT_CAP];
-    const int i = threadIdx.x;
-    if (i < M) {
-        sn[i] = mnew[i];
-        so[i] = mold[i];
-    }
-    __syncthreads();
-    if (i >= M) return;
-    const uint64_t x = sn[i];
-    const uint64_t o = so[i];
+    const int first = blockIdx.x * RANK_MOVERS;
+    if (first >= M) return;
+    __shared__ uint64_t tn[RANK_BLOCK], to[RANK_BLOCK];
+    __shared__ int part[3][RANK_BLOCK];
+    const int lane = lane_id(), seg = (int)threadIdx.x >> 6;
+    const int i = first + lane;
+    const uint64_t x = i < M ? mnew[i] : 0u;
+    const uint64_t o = i < M ? mold[i] : 0u;
+    // the starts of x's cell and its position, their latency behind the counting
+    const uint32_t cell = (uint32_t)(x >> 32);  // < the cell count: written from a clamped cell
+    const int c0 = cell_start[cell], c1 = cell_start[cell + 1];
+    const float4 px = pos_state[min((uint32_t)x, (uint32_t)(n - 1))];
     int rn = 0, ro = 0, old_less = 0;
-    for (int j = 0; j < M; ++j) {
-        const uint64_t a = sn[j], b = so[j];
-        rn += a < x ? 1 : 0;
-        ro += b < o ? 1 : 0;
-        old_less += b < x ? 1 : 0;
+    for (int j0 = 0; j0 < M; j0 += RANK_BLOCK) {
+        const int j = j0 + (int)threadIdx.x;
+        tn[threadIdx.x] = j < M ? mnew[j] : ~0ull;  // (past the end: smaller than no key)
+        to[threadIdx.x] = j < M ? mold[j] : ~0ull;
+        __syncthreads();
+#pragma unroll 8
+        for (int k = 0; k < RANK_MOVERS; ++k) {
+            const uint64_t a = tn[seg * RANK_MOVERS + k], b = to[seg * RANK_MOVERS + k];
+            rn += a < x ? 1 : 0;
+            ro += b < o ? 1 : 0;
+            old_less += b < x ? 1 : 0;
+        }
+        __syncthreads();
+    }
+    part[0][threadIdx.x] = rn;
+    part[1][threadIdx.x] = ro;
+    part[2][threadIdx.x] = old_less;
+    __syncthreads();
+    if (seg != 0 || i >= M) return;
+#pragma unroll
+    for (int w = 1; w < RANK_BLOCK / 64; ++w) {
+        rn += part[0][w * 64 + lane];
+        ro += part[1][w * 64 + lane];
+        old_less += part[2][w * 64 + lane];
     }
     msn[rn] = x;
     mso[ro] = o;
     // previous positions with a smaller key: those of the cells before x's
     // cell, and those of x's cell below x's position
-    const uint32_t cell = (uint32_t)(x >> 32);  // < the cell count: written from a clamped cell
     const int sx = (int)(uint32_t)x;
-    const int c0 = cell_start[cell], c1 = cell_start[cell + 1];
     const int all_less = c0 + (sx < c0 ? 0 : (sx > c1 ? c1 - c0 : sx - c0));
     const int dest = all_less - old_less + rn;
     if (dest >= 0 && dest < n && (uint32_t)x < (uint32_t)n) {  // (always, for consistent keys)
         keys_out[dest] = x;
-        posB[dest] = pos_state[(uint32_t)x];
+        posB[dest] = px;
     }
 }
 
@@ -84,89 +110,144 @@ __device__ __forceinline__ int lower_bound_u64(const uint64_t* a, int lo, int hi
     return lo;
 }
 
+// Entries of the ascending a[0, M) below key, by a whole wave: 64 probes a
+// round, so three dependent loads for up to 262,144 entries. low: the entries'
+// low halves (old positions, ascending too) are compared.
+template <bool low>
+__device__ __forceinline__ int wave_lower_bound(const uint64_t* __restrict__ a, int M, uint64_t key) {
+    int lo = 0, hi = M;
+    while (hi - lo > 64) {
+        const int step = (hi - lo + 63) / 64;
+        const int at = lo + (lane_id() + 1) * step - 1;
+        bool less = false;
+        if (at < hi) less = low ? (uint32_t)a[at] < (uint32_t)key : a[at] < key;
+        const int k = __popcll(__ballot(less));
+        lo = lo + k * step;
+        hi = min(hi, lo + step);
+    }
+    const int at = lo + lane_id();
+    bool less = false;
+    if (at < hi) less = low ? (uint32_t)a[at] < (uint32_t)key : a[at] < key;
+    return lo + __popcll(__ballot(less));
+}
+
 // Every stayer: its place, key and position. Also the new order's cell starts,
 // in place: start[c] counts the keys below c << 32, so it changes by the
 // movers' new keys below c << 32 minus their old keys below c << 32. Each
-// block updates cells_per_block consecutive cells, RESORT_MERGE_BLOCK at a
-// time; a run of cells that holds no mover key has one change for all its
-// cells (most runs: none). Sets *next_count = 0 for the next step's movers.
+// block updates cells_per_block consecutive cells; a run of cells that holds no
+// mover key has one change for all its cells (most runs: none). Sets
+// *next_count = 0 for the next step's movers.
+//
+// A block's positions and cells meet few movers: each wave finds one bound of
+// them in the sorted lists, and only that slice is held in LDS (all the movers'
+// keys were before, which set their limit and cost 16 KB of LDS a block).
 __global__ __launch_bounds__(RESORT_MERGE_BLOCK) void k_resort_merge(
-    const int* __restrict__ mcount, const uint64_t* __restrict__ msn, const uint64_t* __restrict__ mso,
+    const int* __restrict__ mcount, int cap, const uint64_t* __restrict__ msn, const uint64_t* __restrict__ mso,
     const uint64_t* __restrict__ keys, int n, const float4* __restrict__ pos_state, float4* __restrict__ posB,
     uint64_t* __restrict__ keys_out, int* __restrict__ cell_start, int n_cells, int cells_per_block,
     int* __restrict__ next_count, const int* __restrict__ step_ctl) {
-    if (step_ctl[0]) return;
-    const int M = *mcount;
-    if (M > RESORT_CAP) return;
+    const int given_up = step_ctl[0], M = *mcount;
+    if (given_up || M > cap) return;
     // this thread's key and position, loaded first: their latency overlaps the
-    // movers' staging and the searches below
-    const int s = blockIdx.x * RESORT_MERGE_BLOCK + (int)threadIdx.x;
+    // searches below
+    const int s0 = blockIdx.x * RESORT_MERGE_BLOCK;
+    const int s = s0 + (int)threadIdx.x;
     uint64_t y = 0u;
     float4 ps = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (s < n) {
         y = keys[s];
         ps = pos_state[s];
     }
-    __shared__ uint64_t sn[RESORT_CAP], so[RESORT_CAP];
-    for (int j = threadIdx.x; j < M; j += RESORT_MERGE_BLOCK) {
-        sn[j] = msn[j];
-        so[j] = mso[j];
-    }
-    __syncthreads();
     if (blockIdx.x == 0 && threadIdx.x == 0) *next_count = 0;
-    const int c0 = blockIdx.x * cells_per_block;
-    const int c1 = min(c0 + cells_per_block, n_cells);
-    if (M > 0 && c0 < c1) {
-        // mover keys below the run start (new: alo, old: blo); the runs are
-        // consecutive, so each next bound is a short scan from the last one
-        int alo = lower_bound_u64(sn, 0, M, (uint64_t)c0 << 32);
-        int blo = lower_bound_u64(so, 0, M, (uint64_t)c0 << 32);
-        for (int cs = c0; cs < c1; cs += RESORT_MERGE_BLOCK) {
-            const int ce = min(cs + RESORT_MERGE_BLOCK, c1);
-            const uint64_t khi = (uint64_t)ce << 32;
-            int ahi = alo, bhi = blo;
-            while (ahi < M && sn[ahi] < khi) ++ahi;
-            while (bhi < M && so[bhi] < khi) ++bhi;
-            const int c = cs + (int)threadIdx.x;
-            if (c < ce) {
-                int d = alo - blo;
-                if (alo != ahi || blo != bhi) {
-                    const uint64_t k = (uint64_t)c << 32;
-                    d = lower_bound_u64(sn, alo, ahi, k) - lower_bound_u64(so, blo, bhi, k);
+    int d = s;
+    if (M > 0) {
+        constexpr int NW = RESORT_MERGE_BLOCK / 64;
+        static_assert(NW == 8, "one search per wave below");
+        __shared__ uint64_t so[RESORT_MERGE_BLOCK], sn[MERGE_SLICE];
+        __shared__ int bound[NW];
+        __shared__ uint64_t ymin[NW], ymax[NW];
+        const int w = (int)threadIdx.x >> 6;
+        const int c0 = (int)min((long long)blockIdx.x * cells_per_block, (long long)n_cells);
+        const int c1 = (int)min((long long)c0 + cells_per_block, (long long)n_cells);
+        const uint64_t k0 = (uint64_t)(uint32_t)c0 << 32, k1 = (uint64_t)(uint32_t)c1 << 32;
+        int b;
+        if (w == 0) b = wave_lower_bound<true>(mso, M, (uint64_t)(uint32_t)s0);
+        else if (w == 1) b = wave_lower_bound<true>(mso, M, (uint64_t)(uint32_t)(s0 + RESORT_MERGE_BLOCK));
+        else if (w == 2) b = wave_lower_bound<false>(msn, M, k0);
+        else if (w == 3) b = wave_lower_bound<false>(msn, M, k1);
+        else if (w == 4) b = wave_lower_bound<false>(mso, M, k0);
+        else if (w == 5) b = wave_lower_bound<false>(mso, M, k1);
+        else b = 0;
+        if (lane_id() == 0) bound[w] = b;
+        __syncthreads();
+        const int olo = bound[0], on = bound[1] - olo;  // at most one old key per position: on <= 512
+        const int alo = bound[2], ahi = bound[3], blo = bound[4], bhi = bound[5];
+        if ((int)threadIdx.x < on) so[threadIdx.x] = mso[olo + threadIdx.x];
+        __syncthreads();
+        // cell starts of this block's cells
+        if (alo != blo || ahi != alo || bhi != blo) {
+            for (int c = c0 + (int)threadIdx.x; c < c1; c += RESORT_MERGE_BLOCK) {
+                int dd = alo - blo;
+                if (ahi != alo || bhi != blo) {
+                    const uint64_t k = (uint64_t)(uint32_t)c << 32;
+                    dd = lower_bound_u64(msn, alo, ahi, k) - lower_bound_u64(mso, blo, bhi, k);
                 }
-                if (d != 0) cell_start[c] += d;
+                if (dd != 0) cell_start[c] += dd;
             }
-            alo = ahi;
-            blo = bhi;
         }
+        // movers before s: old keys ascend with their positions (the low halves)
+        int lo = 0, hi = on;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if ((uint32_t)so[mid] < (uint32_t)s) lo = mid + 1;
+            else hi = mid;
+        }
+        const bool stays = s < n && !(lo < on && (uint32_t)so[lo] == (uint32_t)s);  // (movers are placed already)
+        // the stayers' keys ascend: their range, and the new keys inside it
+        const uint64_t m = __ballot(stays);
+        const int fl = m ? __builtin_ctzll(m) : 0, ll = m ? 63 - __builtin_clzll(m) : 0;
+        if (m && lane_id() == fl) ymin[w] = y;
+        if (m && lane_id() == ll) ymax[w] = y;
+        if (!m && lane_id() == 0) {
+            ymin[w] = ~0ull;
+            ymax[w] = 0u;
+        }
+        __syncthreads();
+        uint64_t y0 = ~0ull, y1 = 0u;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            y0 = ymin[q] < y0 ? ymin[q] : y0;
+            y1 = ymax[q] > y1 ? ymax[q] : y1;
+        }
+        if (w == 0) b = wave_lower_bound<false>(msn, M, y0);
+        else if (w == 1) b = wave_lower_bound<false>(msn, M, y1);
+        if (w < 2 && lane_id() == 0) bound[6 + w] = b;
+        __syncthreads();
+        const int nlo = bound[6], nn = max(bound[7] - nlo, 0);  // new keys in [y0, y1)
+        const bool held = nn <= MERGE_SLICE;
+        if (held)
+            for (int j = threadIdx.x; j < nn; j += RESORT_MERGE_BLOCK) sn[j] = msn[nlo + j];
+        __syncthreads();
+        if (!stays) return;
+        const int a = held ? nlo + lower_bound_u64(sn, 0, nn, y) : lower_bound_u64(msn, nlo, nlo + nn, y);
+        d = s - (olo + lo) + a;
     }
-    if (s >= n) return;
-    // movers before s: old keys ascend with their positions (the low halves)
-    int lo = 0, hi = M;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if ((uint32_t)so[mid] < (uint32_t)s) lo = mid + 1;
-        else hi = mid;
-    }
-    if (lo < M && (uint32_t)so[lo] == (uint32_t)s) return;  // a mover, placed by k_resort_movers
-    const int a = lower_bound_u64(sn, 0, M, y);
-    const int d = s - lo + a;
-    if (d < 0 || d >= n) return;  // (never, for consistent keys)
+    if (s >= n || d < 0 || d >= n) return;  // (d is inside for consistent keys)
     keys_out[d] = y;
     posB[d] = ps;
 }
 
-sd_status launch_resort_u64(const int* mcount, const uint64_t* mnew, const uint64_t* mold, uint64_t* msorted_new,
-                            uint64_t* msorted_old, const uint64_t* keys, int n, int* cell_start, int n_cells,
-                            const float4* pos_state, float4* posB, uint64_t* keys_out, int* next_count,
-                            int* step_ctl, hipStream_t s) {
+sd_status launch_resort_u64(const int* mcount, int cap, const uint64_t* mnew, const uint64_t* mold,
+                            uint64_t* msorted_new, uint64_t* msorted_old, const uint64_t* keys, int n,
+                            int* cell_start, int n_cells, const float4* pos_state, float4* posB, uint64_t* keys_out,
+                            int* next_count, int* step_ctl, hipStream_t s) {
     if (n <= 0) return SD_OK;
-    hipLaunchKernelGGL(k_resort_movers, dim3(1), dim3(RESORT_CAP), 0, s, mcount, mnew, mold, msorted_new,
-                       msorted_old, n, (const int*)cell_start, pos_state, posB, keys_out, step_ctl);
+    hipLaunchKernelGGL(k_resort_movers, dim3(div_up(cap, RANK_MOVERS)), dim3(RANK_BLOCK), 0, s, mcount, cap, mnew,
+                       mold, msorted_new, msorted_old, n, (const int*)cell_start, pos_state, posB, keys_out, step_ctl);
     SD_LAUNCH_CHECK();
     const int nblocks = div_up(n, RESORT_MERGE_BLOCK);
     const int cells_per_block = div_up(div_up(n_cells, nblocks), RESORT_MERGE_BLOCK) * RESORT_MERGE_BLOCK;
-    hipLaunchKernelGGL(k_resort_merge, dim3(nblocks), dim3(RESORT_MERGE_BLOCK), 0, s, mcount,
+    hipLaunchKernelGGL(k_resort_merge, dim3(nblocks), dim3(RESORT_MERGE_BLOCK), 0, s, mcount, cap,
                        (const uint64_t*)msorted_new, (const uint64_t*)msorted_old, keys, n, pos_state, posB, keys_out,
                        cell_start, n_cells, cells_per_block, next_count, (const int*)step_ctl);
     SD_LAUNCH_CHECK();
