@@ -209,7 +209,8 @@ sd_status sd_permute_spheres(const int* perm, int n,
 typedef struct sd_sphere_params {
     sd_grid grid;
     sd_contact_params contact;
-    int key64;           /* 0: u32 cell keys + u32 index values; 1: packed u64 (cell<<32 | index) */
+    int key64;           /* keys of a saved state: 0: u32 cells and u32 indices; 1: packed u64 (cell<<32 | index);
+                          * both step alike */
     int use_graph;       /* 1: replay steps from a captured hipGraph */
     int tile_items;      /* sort items per thread (0 = autotuned) */
 } sd_sphere_params;
@@ -234,8 +235,8 @@ sd_status sd_ctx_step(sd_ctx* ctx, int nsteps);
 /* Runs nsteps steps without graph replay, recording HIP events on the context
  * stream around each stage, and adds the time of each stage summed over the
  * steps to stage_ms: [0] sort, [1] cell starts (first sorted position of
- * every cell), [2] permute, [3] fused contact + integrate + next keys. With u64
- * keys, [0] is the re-sort from the previous order (positions permuted and
+ * every cell), [2] permute, [3] fused contact + integrate + next keys. [0] is
+ * the re-sort from the previous order (positions permuted and
  * cell starts updated in the same pass; [1] is empty) when at most 1024
  * spheres (one in 256, up to 16384, of more than 262,144) changed cell in the
  * previous step, else the radix sort (all passes),

@@ -73,7 +73,6 @@ __device__ __forceinline__ void integrate_sphere(const ContactDev& c, float4& p,
 
 __device__ __forceinline__ int old_slot_of(const ContactArgs& a, int s) {
     if (a.old_slot_i32) return a.old_slot_i32[s];
-    if (a.old_slot_u32) return (int)a.old_slot_u32[s];
     return (int)(uint32_t)a.old_slot_u64[s];
 }
 
@@ -395,10 +394,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
         a.vel_o[s] = v;
         a.omg_o[s] = w;
         a.ids_o[s] = myid;
-        if (MODE == CONTACT_FUSED_U32) {
-            a.keys_o32[s] = cell_id(g, p.x, p.y, p.z);
-            a.vals_o32[s] = (uint32_t)s;
-        } else {
+        {
             const uint32_t cell_new = cbase + cell_id(g, p.x, p.y, p.z);
             const uint64_t key_new = ((uint64_t)cell_new << 32) | (uint64_t)(uint32_t)s;
             a.keys_o64[s] = key_new;
@@ -492,8 +488,6 @@ sd_status launch_contacts(int mode, const ContactArgs& a, hipStream_t s, int blo
     const size_t lds = (size_t)(block / WAVE) * CONTACT_STAGE * sizeof(float4);
     if (mode == CONTACT_FORCES)
         hipLaunchKernelGGL((k_contacts<CONTACT_FORCES, false>), grid, dim3(block), lds, s, a);
-    else if (mode == CONTACT_FUSED_U32)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U32, true>), grid, dim3(block), lds, s, a);
     else if (mode == CONTACT_FUSED_U64)
         hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U64, true>), grid, dim3(block), lds, s, a);
     else

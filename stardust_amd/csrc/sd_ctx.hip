@@ -6,8 +6,8 @@
 //
 // One step, all on the context stream, no host synchronisation:
 //   sort(keys)            keys were written by the previous step (or upload):
-//                         the radix sort, or with u64 keys the re-sort from
-//                         the previous order (which also permutes positions)
+//                         the re-sort from the previous order (which also
+//                         permutes positions), or the radix sort
 //   cell starts           first sorted position of every cell
 //   permute positions     sorted positions gathered from the current state
 //   fused contact kernel  reads sorted positions, the current state (through the
@@ -101,8 +101,10 @@ struct sd_ctx {
     int* ids[2] = {nullptr, nullptr};
     int cur_state = 0;
     float4* posB = nullptr;
-    uint32_t* k32[2] = {nullptr, nullptr};
-    uint32_t* v32[2] = {nullptr, nullptr};
+    // cell << 32 | slot, whatever the width of the keys that the caller chose
+    // (p.key64): 32-bit keys and values would need a full sort every step. At
+    // 65,536 spheres its nine launches and the cell starts and permutation
+    // after it took 40 of 51 us per step; the re-sort takes 9.
     uint64_t* k64[2] = {nullptr, nullptr};
     int cur_keys = 0;
     void* sort_tmp = nullptr;
@@ -169,7 +171,7 @@ void release(sd_ctx* c) {
     drop_graphs(c);
     stage_release(c->stage);
     void* bufs[] = {c->pos[0], c->pos[1], c->vel[0], c->vel[1], c->omg[0], c->omg[1], c->ids[0], c->ids[1],
-                    c->posB, c->k32[0], c->k32[1], c->v32[0], c->v32[1], c->k64[0], c->k64[1], c->sort_tmp,
+                    c->posB, c->k64[0], c->k64[1], c->sort_tmp,
                     c->cell_start, c->hcount[0], c->hcount[1], c->hist[0], c->hist[1], c->overflow, c->diag,
                     c->scenes_d, c->scene_of, c->straddle, c->mcount, c->mnew, c->mold, c->msn, c->mso,
                     c->step_ctl};
@@ -180,7 +182,6 @@ void release(sd_ctx* c) {
         c->ids[k] = nullptr;
     }
     c->posB = nullptr;
-    c->k32[0] = c->k32[1] = c->v32[0] = c->v32[1] = nullptr;
     c->k64[0] = c->k64[1] = nullptr;
     c->sort_tmp = nullptr;
     c->cell_start = nullptr;
@@ -208,7 +209,7 @@ sd_status dalloc(T** p, size_t count) {
 
 // Enqueues one step on the context stream. If ev is given, ev[0..4] are
 // recorded before the sort and after the sort, cell-start, permute and contact stages.
-// full (u64 keys): the radix sort instead of the re-sort from the previous
+// full: the radix sort instead of the re-sort from the previous
 // order. A re-sort step that finds more than resort_cap(n) changed cells is given
 // up on the device (step_ctl[0]), together with every later step of the same
 // launch sequence; the host then redoes it as a full step (run_steps).
@@ -246,87 +247,64 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
         if (st != SD_OK) return st;
         SD_HIP(hipEventRecord(c->hev_join, c->hside));
     }
-    if (c->p.key64) {
-        // sorted keys: the radix sort (full), or the re-sort from the previous
-        // order and the spheres that changed cell, with the positions permuted
-        // in the same pass. Either leaves them in the other key buffer.
-        uint64_t* K = c->k64[c->cur_keys];
-        uint64_t* Ka = c->k64[1 - c->cur_keys];
-        // changed-cell counters alternate with the history buffers: this step
-        // reads [ho] (written by the previous step) and appends to [hn]
-        int* mc_read = c->mcount + ho;
-        int* mc_write = c->mcount + hn;
-        if (full) {
-            st = radix_sort_keys_u64_gated(&K, &Ka, n, 32, 32 + c->key_bits, c->sort_tmp, c->sort_tmp_bytes, s,
-                                           c->items, nullptr, 0);
-        } else {
-            // also updates the cell starts and sets mc_write = 0
-            st = launch_resort_u64(mc_read, resort_cap(n), c->mnew, c->mold, c->msn, c->mso, K, n, c->cell_start, c->n_cells,
-                                   c->pos[so], c->posB, Ka, mc_write, c->step_ctl, s);
-            uint64_t* t = K;
-            K = Ka;
-            Ka = t;
-        }
-        if (st != SD_OK) return st;
-        MARK(1);
-        // after the full sort: cell starts, the permutation, mc_write = 0
-        if (full) st = launch_step_starts_u64(K, n, c->n_cells, c->cell_start, c->step_ctl, true, c->pos[so],
-                                              c->posB, mc_write, s);
-        if (st != SD_OK) return st;
-        MARK(2);
-        MARK(3);
-        a.old_slot_u64 = K;
-        a.keys_o64 = Ka;
-        a.mcount = mc_write;
-        a.mnew = c->mnew;
-        a.mold = c->mold;
-        a.mcap = resort_cap(n);
-        a.step_ctl = c->step_ctl;
-        a.scenes = c->scenes_d;
-        a.scene_of = c->scene_of;
-        a.straddle = c->straddle;
-        a.n_straddle = c->n_straddle;
-        // waves spanning two scenes: their own launch, beside the main one
-        // (disjoint spheres; shared counters are atomics)
-        const bool fork = c->batch && c->n_straddle > 0;
-        if (fork) {
-            SD_HIP(hipEventRecord(c->ev_fork, s));
-            SD_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-            st = launch_contacts_straddle(a, c->side);
-            if (st != SD_OK) return st;
-            SD_HIP(hipEventRecord(c->ev_join, c->side));
-        }
-        if (c->persistent)
-            st = launch_contacts_persistent(c->batch ? CONTACT_FUSED_BATCH : CONTACT_FUSED_U64, a, s,
-                                            c->contact_block, c->pcounters);
-        else
-            st = launch_contacts(c->batch ? CONTACT_FUSED_BATCH : CONTACT_FUSED_U64, a, s, c->contact_block);
-        if (st != SD_OK) return st;
-        if (fork) SD_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
-        MARK(4);
-        c->cur_keys = (Ka == c->k64[0]) ? 0 : 1;
+    // sorted keys: the radix sort (full), or the re-sort from the previous
+    // order and the spheres that changed cell, with the positions permuted
+    // in the same pass. Either leaves them in the other key buffer.
+    uint64_t* K = c->k64[c->cur_keys];
+    uint64_t* Ka = c->k64[1 - c->cur_keys];
+    // changed-cell counters alternate with the history buffers: this step
+    // reads [ho] (written by the previous step) and appends to [hn]
+    int* mc_read = c->mcount + ho;
+    int* mc_write = c->mcount + hn;
+    if (full) {
+        st = radix_sort_keys_u64_gated(&K, &Ka, n, 32, 32 + c->key_bits, c->sort_tmp, c->sort_tmp_bytes, s,
+                                       c->items, nullptr, 0);
     } else {
-        uint32_t* K = c->k32[c->cur_keys];
-        uint32_t* V = c->v32[c->cur_keys];
-        uint32_t* Ka = c->k32[1 - c->cur_keys];
-        uint32_t* Va = c->v32[1 - c->cur_keys];
-        st = radix_sort_pairs_u32(&K, &V, &Ka, &Va, n, 0, c->key_bits, c->sort_tmp, c->sort_tmp_bytes, s, c->items);
-        if (st != SD_OK) return st;
-        MARK(1);
-        st = launch_cell_starts_u32(K, n, c->n_cells, c->cell_start, s);
-        if (st != SD_OK) return st;
-        MARK(2);
-        st = launch_permute_pos(V, nullptr, n, c->pos[so], c->posB, s);
-        if (st != SD_OK) return st;
-        MARK(3);
-        a.old_slot_u32 = V;
-        a.keys_o32 = Ka;
-        a.vals_o32 = Va;
-        st = launch_contacts(CONTACT_FUSED_U32, a, s, c->contact_block);
-        if (st != SD_OK) return st;
-        MARK(4);
-        c->cur_keys = (Ka == c->k32[0]) ? 0 : 1;
+        // also updates the cell starts and sets mc_write = 0
+        st = launch_resort_u64(mc_read, resort_cap(n), c->mnew, c->mold, c->msn, c->mso, K, n, c->cell_start, c->n_cells,
+                               c->pos[so], c->posB, Ka, mc_write, c->step_ctl, s);
+        uint64_t* t = K;
+        K = Ka;
+        Ka = t;
     }
+    if (st != SD_OK) return st;
+    MARK(1);
+    // after the full sort: cell starts, the permutation, mc_write = 0
+    if (full) st = launch_step_starts_u64(K, n, c->n_cells, c->cell_start, c->step_ctl, true, c->pos[so],
+                                          c->posB, mc_write, s);
+    if (st != SD_OK) return st;
+    MARK(2);
+    MARK(3);
+    a.old_slot_u64 = K;
+    a.keys_o64 = Ka;
+    a.mcount = mc_write;
+    a.mnew = c->mnew;
+    a.mold = c->mold;
+    a.mcap = resort_cap(n);
+    a.step_ctl = c->step_ctl;
+    a.scenes = c->scenes_d;
+    a.scene_of = c->scene_of;
+    a.straddle = c->straddle;
+    a.n_straddle = c->n_straddle;
+    // waves spanning two scenes: their own launch, beside the main one
+    // (disjoint spheres; shared counters are atomics)
+    const bool fork = c->batch && c->n_straddle > 0;
+    if (fork) {
+        SD_HIP(hipEventRecord(c->ev_fork, s));
+        SD_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
+        st = launch_contacts_straddle(a, c->side);
+        if (st != SD_OK) return st;
+        SD_HIP(hipEventRecord(c->ev_join, c->side));
+    }
+    if (c->persistent)
+        st = launch_contacts_persistent(c->batch ? CONTACT_FUSED_BATCH : CONTACT_FUSED_U64, a, s,
+                                        c->contact_block, c->pcounters);
+    else
+        st = launch_contacts(c->batch ? CONTACT_FUSED_BATCH : CONTACT_FUSED_U64, a, s, c->contact_block);
+    if (st != SD_OK) return st;
+    if (fork) SD_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
+    MARK(4);
+    c->cur_keys = (Ka == c->k64[0]) ? 0 : 1;
 #undef MARK
     if (c->hulls) SD_HIP(hipStreamWaitEvent(s, c->hev_join, 0));
     c->cur_hist = hn;
@@ -368,7 +346,7 @@ sd_status run_graph_pair(sd_ctx* c, bool full = false) {
     return SD_OK;
 }
 
-// Runs nsteps steps. u64 keys: re-sort steps (graph-replayed in pairs when
+// Runs nsteps steps: re-sort steps (graph-replayed in pairs when
 // use_graph), and a full step first whenever the keys are not from a step of
 // this order, or a re-sort step was given up. The device counts the steps that
 // ran, which sets the buffer roles; one synchronisation per launch sequence.
@@ -377,21 +355,6 @@ sd_status run_steps(sd_ctx* c, int nsteps) {
     if (c->hulls && hull_generation(c->hulls) != c->hull_gen) {
         drop_graphs(c);  // captured with the attached bodies' previous step
         c->hull_gen = hull_generation(c->hulls);
-    }
-    if (!c->p.key64) {
-        int left = nsteps;
-        if (c->p.use_graph) {
-            while (left >= 2) {
-                st = run_graph_pair(c);
-                if (st != SD_OK) return st;
-                left -= 2;
-            }
-        }
-        for (; left > 0; --left) {
-            st = enqueue_step(c);
-            if (st != SD_OK) return st;
-        }
-        return SD_OK;
     }
     int left = nsteps;
     while (left > 0) {
@@ -595,15 +558,8 @@ sd_status upload_state(sd_ctx* c, int n, const float* x, const float* y, const f
         ALLOC(c->ids[k], n);
     }
     ALLOC(c->posB, (size_t)n + CONTACT_POS_PAD);
-    if (c->p.key64) {
-        ALLOC(c->k64[0], n);
-        ALLOC(c->k64[1], n);
-    } else {
-        ALLOC(c->k32[0], n);
-        ALLOC(c->k32[1], n);
-        ALLOC(c->v32[0], n);
-        ALLOC(c->v32[1], n);
-    }
+    ALLOC(c->k64[0], n);
+    ALLOC(c->k64[1], n);
     c->sort_tmp_bytes = radix_temp_bytes(n);
     ALLOC(*(char**)&c->sort_tmp, c->sort_tmp_bytes);
     ALLOC(c->cell_start, (size_t)c->n_cells + 1);
@@ -670,8 +626,7 @@ extern "C" sd_status sd_ctx_upload_spheres(sd_ctx* c, int n, const float* x, con
         return st;
     }
     const GridDev g = to_dev(c->p.grid);
-    st = c->p.key64 ? launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], c->stream)
-                    : launch_hash_keys_u32(c->pos[0], n, g, c->k32[0], c->v32[0], c->stream);
+    st = launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], c->stream);
     if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(c->stream));
     return SD_OK;
@@ -819,7 +774,7 @@ extern "C" sd_status sd_ctx_profile(sd_ctx* c, int nsteps, float* stage_ms, int 
     sd_status st = SD_OK;
     for (int i = 0; i < nsteps && st == SD_OK; ++i) {
         bool full = c->need_full;
-        if (c->p.key64 && !full) {  // full sort when the re-sort would give the step up
+        if (!full) {  // full sort when the re-sort would give the step up
             int m = 0;
             if (hipMemcpyAsync(&m, c->mcount + c->cur_hist, sizeof(int), hipMemcpyDeviceToHost, c->stream) !=
                     hipSuccess ||
@@ -869,13 +824,13 @@ namespace {
 
 struct Snapshot {
     char* buf = nullptr;
-    size_t off[8] = {};
-    size_t sz[8] = {};
+    size_t off[7] = {};
+    size_t sz[7] = {};
     int roles[3] = {0, 0, 0};
 };
 
-// Role buffers of the current state: pos, vel, omg, ids, keys (k64 or k32), v32, hcount, hist.
-void role_buffers(sd_ctx* c, void* b[8], size_t sz[8]) {
+// Role buffers of the current state: pos, vel, omg, ids, keys, hcount, hist.
+void role_buffers(sd_ctx* c, void* b[7], size_t sz[7]) {
     const size_t n = (size_t)c->n;
     const int cs = c->cur_state, ck = c->cur_keys, ch = c->cur_hist;
     b[0] = c->pos[cs];
@@ -886,26 +841,24 @@ void role_buffers(sd_ctx* c, void* b[8], size_t sz[8]) {
     sz[2] = n * sizeof(float4);
     b[3] = c->ids[cs];
     sz[3] = n * sizeof(int);
-    b[4] = c->p.key64 ? (void*)c->k64[ck] : (void*)c->k32[ck];
-    sz[4] = n * (c->p.key64 ? sizeof(uint64_t) : sizeof(uint32_t));
-    b[5] = c->p.key64 ? nullptr : (void*)c->v32[ck];
-    sz[5] = c->p.key64 ? 0 : n * sizeof(uint32_t);
-    b[6] = c->hcount[ch];
-    sz[6] = n * sizeof(int);
-    b[7] = c->hist[ch];
-    sz[7] = (size_t)c->p.contact.max_contacts * n * sizeof(float4);
+    b[4] = c->k64[ck];
+    sz[4] = n * sizeof(uint64_t);
+    b[5] = c->hcount[ch];
+    sz[5] = n * sizeof(int);
+    b[6] = c->hist[ch];
+    sz[6] = (size_t)c->p.contact.max_contacts * n * sizeof(float4);
 }
 
 sd_status snapshot_take(sd_ctx* c, Snapshot& sn) {
-    void* b[8];
+    void* b[7];
     size_t total = 0;
     role_buffers(c, b, sn.sz);
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < 7; ++k) {
         sn.off[k] = total;
         total += (sn.sz[k] + 255) & ~(size_t)255;
     }
     SD_HIP(hipMalloc((void**)&sn.buf, total));
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < 7; ++k)
         if (sn.sz[k]) SD_HIP(hipMemcpyAsync(sn.buf + sn.off[k], b[k], sn.sz[k], hipMemcpyDeviceToDevice, c->stream));
     sn.roles[0] = c->cur_keys;
     sn.roles[1] = c->cur_hist;
@@ -917,10 +870,10 @@ sd_status snapshot_restore(sd_ctx* c, const Snapshot& sn) {
     c->cur_keys = sn.roles[0];
     c->cur_hist = sn.roles[1];
     c->cur_state = sn.roles[2];
-    void* b[8];
-    size_t sz[8];
+    void* b[7];
+    size_t sz[7];
     role_buffers(c, b, sz);
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < 7; ++k)
         if (sz[k]) SD_HIP(hipMemcpyAsync(b[k], sn.buf + sn.off[k], sz[k], hipMemcpyDeviceToDevice, c->stream));
     sd_status st = force_full_sort(c);
     if (st != SD_OK) return st;
@@ -1166,8 +1119,7 @@ sd_status write_rows(sd_ctx* c, const HostRows& r) {
     SD_HIP(hipMemcpyAsync(c->hcount[0], r.hcount.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, s));
     SD_HIP(hipMemcpyAsync(c->hist[0], r.hist.data(), maxc * n * sizeof(float4), hipMemcpyHostToDevice, s));
     const GridDev g = to_dev(c->p.grid);
-    st = c->p.key64 ? launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], s)
-                    : launch_hash_keys_u32(c->pos[0], n, g, c->k32[0], c->v32[0], s);
+    st = launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], s);
     if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(s));
     c->steps_done = steps;
@@ -1304,16 +1256,21 @@ extern "C" sd_status sd_ctx_save(sd_ctx* c, void* buffer, size_t bytes) {
     if (st == SD_OK) st = d2h(c->vel[cs], n * sizeof(float4));
     if (st == SD_OK) st = d2h(c->omg[cs], n * sizeof(float4));
     if (st == SD_OK) st = d2h(c->ids[cs], n * sizeof(int));
-    if (c->p.key64) {
-        if (st == SD_OK) st = d2h(c->k64[c->cur_keys], n * sizeof(uint64_t));
-    } else {
-        if (st == SD_OK) st = d2h(c->k32[c->cur_keys], n * sizeof(uint32_t));
-        if (st == SD_OK) st = d2h(c->v32[c->cur_keys], n * sizeof(uint32_t));
-    }
+    char* const keys = b;
+    if (st == SD_OK) st = d2h(c->k64[c->cur_keys], n * sizeof(uint64_t));
     if (st == SD_OK) st = d2h(c->hcount[c->cur_hist], n * sizeof(int));
     if (st == SD_OK) st = d2h(c->hist[c->cur_hist], (size_t)c->p.contact.max_contacts * n * sizeof(float4));
     if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(c->stream));
+    if (!c->p.key64) {  // 32-bit keys: the cells, then the slots
+        std::vector<uint64_t> k(n);
+        memcpy(k.data(), keys, n * sizeof(uint64_t));
+        for (size_t i = 0; i < n; ++i) {
+            const uint32_t cell = (uint32_t)(k[i] >> 32), slot = (uint32_t)k[i];
+            memcpy(keys + i * sizeof(uint32_t), &cell, sizeof cell);
+            memcpy(keys + (n + i) * sizeof(uint32_t), &slot, sizeof slot);
+        }
+    }
     return SD_OK;
 }
 
@@ -1346,11 +1303,22 @@ extern "C" sd_status sd_ctx_load(sd_ctx* c, const void* buffer, size_t bytes) {
     if (st == SD_OK) st = h2d(c->vel[0], n * sizeof(float4));
     if (st == SD_OK) st = h2d(c->omg[0], n * sizeof(float4));
     if (st == SD_OK) st = h2d(c->ids[0], n * sizeof(int));
+    std::vector<uint64_t> k;  // lives until the synchronisation below
     if (c->p.key64) {
         if (st == SD_OK) st = h2d(c->k64[0], n * sizeof(uint64_t));
-    } else {
-        if (st == SD_OK) st = h2d(c->k32[0], n * sizeof(uint32_t));
-        if (st == SD_OK) st = h2d(c->v32[0], n * sizeof(uint32_t));
+    } else {  // 32-bit keys: the cells, then the slots
+        k.resize(n);
+        for (size_t i = 0; i < n; ++i) {
+            uint32_t cell, slot;
+            memcpy(&cell, b + i * sizeof(uint32_t), sizeof cell);
+            memcpy(&slot, b + (n + i) * sizeof(uint32_t), sizeof slot);
+            k[i] = (uint64_t)cell << 32 | slot;
+        }
+        b += n * sizeof(uint64_t);
+        if (st == SD_OK)
+            st = hipMemcpyAsync(c->k64[0], k.data(), n * sizeof(uint64_t), hipMemcpyHostToDevice, c->stream) == hipSuccess
+                     ? SD_OK
+                     : set_error(SD_ERR_HIP, "sd_ctx_load: key copy failed");
     }
     if (st == SD_OK) st = h2d(c->hcount[0], n * sizeof(int));
     if (st == SD_OK) st = h2d(c->hist[0], (size_t)c->p.contact.max_contacts * n * sizeof(float4));

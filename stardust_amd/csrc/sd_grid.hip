@@ -61,28 +61,11 @@ __global__ void k_hash_xyz_u64(const float* __restrict__ x, const float* __restr
     keys[i] = ((uint64_t)cell_id(g, x[i], y[i], z[i]) << 32) | (uint64_t)(uint32_t)i;
 }
 
-__global__ void k_hash_pos4_u32(const float4* __restrict__ p, int n, GridDev g, uint32_t* __restrict__ keys,
-                                uint32_t* __restrict__ vals) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 q = p[i];
-    keys[i] = cell_id(g, q.x, q.y, q.z);
-    vals[i] = (uint32_t)i;
-}
-
 __global__ void k_hash_pos4_u64(const float4* __restrict__ p, int n, GridDev g, uint64_t* __restrict__ keys) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4 q = p[i];
     keys[i] = ((uint64_t)cell_id(g, q.x, q.y, q.z) << 32) | (uint64_t)(uint32_t)i;
-}
-
-sd_status launch_hash_keys_u32(const float4* pos4, int n, const GridDev& g, uint32_t* keys, uint32_t* vals,
-                               hipStream_t s) {
-    if (n <= 0) return SD_OK;
-    hipLaunchKernelGGL(k_hash_pos4_u32, dim3(div_up(n, 256)), dim3(256), 0, s, pos4, n, g, keys, vals);
-    SD_LAUNCH_CHECK();
-    return SD_OK;
 }
 
 sd_status launch_hash_keys_u64(const float4* pos4, int n, const GridDev& g, uint64_t* keys, hipStream_t s) {
@@ -218,10 +201,6 @@ static sd_status launch_cell_starts(const K* keys, int n, int n_cells, int* star
     return SD_OK;
 }
 
-sd_status launch_cell_starts_u32(const uint32_t* keys, int n, int n_cells, int* start, hipStream_t s) {
-    return launch_cell_starts<uint32_t, 0>(keys, n, n_cells, start, nullptr, false, nullptr, nullptr, nullptr, s);
-}
-
 sd_status launch_step_starts_u64(const uint64_t* keys, int n, int n_cells, int* start, const int* skip, bool permute,
                                  const float4* pos, float4* pos_o, int* next_count, hipStream_t s) {
     return launch_cell_starts<uint64_t, 32>(keys, n, n_cells, start, skip, permute, pos, pos_o, next_count, s);
@@ -249,26 +228,6 @@ sd_status launch_permute(const uint32_t* perm32, const uint64_t* perm64, int n, 
     if (n <= 0) return SD_OK;
     hipLaunchKernelGGL(k_permute, dim3(div_up(n, 256)), dim3(256), 0, s, perm32, perm64, n, pos, vel, omg, ids, pos_o,
                        vel_o, omg_o, ids_o);
-    SD_LAUNCH_CHECK();
-    return SD_OK;
-}
-
-__global__ void k_permute_pos(const uint32_t* __restrict__ perm32, const uint64_t* __restrict__ perm64, int n,
-                              const float4* __restrict__ pos, float4* __restrict__ pos_o,
-                              const int* __restrict__ gate, int gate_cap) {
-    if (gate && *gate <= gate_cap) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const uint32_t src = perm32 ? perm32[t] : (uint32_t)perm64[t];
-    if (src >= (uint32_t)n) return;
-    pos_o[t] = pos[src];
-}
-
-sd_status launch_permute_pos(const uint32_t* perm32, const uint64_t* perm64, int n, const float4* pos, float4* pos_o,
-                             hipStream_t s, const int* gate, int gate_cap) {
-    if (n <= 0) return SD_OK;
-    hipLaunchKernelGGL(k_permute_pos, dim3(div_up(n, 256)), dim3(256), 0, s, perm32, perm64, n, pos, pos_o, gate,
-                       gate_cap);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }

@@ -49,8 +49,6 @@ sd_status check_grid(const sd_grid* g);
 
 sd_status launch_fill_u32(uint32_t* dst, uint32_t value, size_t count, hipStream_t s);
 sd_status launch_copy_u32(uint32_t* dst, const uint32_t* src, size_t count, hipStream_t s);
-sd_status launch_hash_keys_u32(const float4* pos4, int n, const GridDev& g, uint32_t* keys, uint32_t* vals,
-                               hipStream_t s);
 sd_status launch_hash_keys_u64(const float4* pos4, int n, const GridDev& g, uint64_t* keys, hipStream_t s);
 struct SceneDev;
 // keys[i] = (scene cbase + cell of pos4[i] in the scene grid) << 32 | i
@@ -59,20 +57,15 @@ sd_status launch_hash_keys_batch(const float4* pos4, int n, const SceneDev* scen
 sd_status launch_cell_ranges_u32(const uint32_t* keys, int n, int n_cells, int* ranges, hipStream_t s);
 sd_status launch_cell_ranges_u64(const uint64_t* keys, int n, int n_cells, int* ranges, hipStream_t s);
 // Cell starts of sorted keys: start[c] = number of keys whose cell is below c,
-// c = 0 .. n_cells (n_cells + 1 entries), every entry written. The u64 form
-// also gathers pos into sorted order (pos_o) with permute and sets
-// *next_count = 0; it does nothing while *skip.
-sd_status launch_cell_starts_u32(const uint32_t* keys, int n, int n_cells, int* start, hipStream_t s);
+// c = 0 .. n_cells (n_cells + 1 entries), every entry written. Also gathers pos
+// into sorted order (pos_o) with permute and sets *next_count = 0; does
+// nothing while *skip.
 sd_status launch_step_starts_u64(const uint64_t* keys, int n, int n_cells, int* start, const int* skip, bool permute,
                                  const float4* pos, float4* pos_o, int* next_count, hipStream_t s);
 // perm is either u32 values (perm32) or the low halves of u64 keys (perm64).
 sd_status launch_permute(const uint32_t* perm32, const uint64_t* perm64, int n, const float4* pos, const float4* vel,
                          const float4* omg, const int* ids, float4* pos_o, float4* vel_o, float4* omg_o, int* ids_o,
                          hipStream_t s);
-
-// gate (nullable): skipped on the device while *gate <= gate_cap.
-sd_status launch_permute_pos(const uint32_t* perm32, const uint64_t* perm64, int n, const float4* pos, float4* pos_o,
-                             hipStream_t s, const int* gate = nullptr, int gate_cap = 0);
 
 // ------------------------------------------------------------------ contacts
 struct ContactDev {
@@ -91,7 +84,7 @@ constexpr int CONTACT_POS_PAD = 4;
 
 // Fused step kernel modes. CONTACT_FUSED_BATCH: packed u64 keys, every sphere
 // takes its grid, contact law and cell-id base from its scene's SceneDev.
-enum { CONTACT_FORCES = 0, CONTACT_FUSED_U32 = 1, CONTACT_FUSED_U64 = 2, CONTACT_FUSED_BATCH = 3 };
+enum { CONTACT_FORCES = 0, CONTACT_FUSED_U64 = 1, CONTACT_FUSED_BATCH = 2 };
 
 // One scene of a batch: its grid, its contact law, the first global cell id of
 // its cells and its slot range [first, first + n) (sorted positions of a batch
@@ -115,9 +108,8 @@ struct ContactArgs {
     const int* ranges;      // CONTACT_FORCES: (start, end) per cell, empty cells (0, 0)
     const int* cell_start;  // fused modes: first sorted position of every cell (n_cells + 1 entries)
     ContactDev c;
-    // old order: either an int array, u32 sort values or packed u64 keys
+    // old order: either an int array or packed u64 keys
     const int* old_slot_i32;
-    const uint32_t* old_slot_u32;
     const uint64_t* old_slot_u64;
     const int* hcount_old;
     const float4* hist_old;
@@ -132,8 +124,6 @@ struct ContactArgs {
     float4* vel_o;
     float4* omg_o;
     int* ids_o;
-    uint32_t* keys_o32;
-    uint32_t* vals_o32;
     uint64_t* keys_o64;
     // fused u64 modes: spheres whose cell changed this step, appended as
     // (new key, old key) while *mcount < mcap (nullable: not recorded)

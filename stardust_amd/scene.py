@@ -40,7 +40,7 @@ class SphereScene:
     def profile(self, nsteps):
         """Per-stage GPU time in ms summed over nsteps eager steps:
         sort, ranges (the cell starts), permute, contact (HIP events on the
-        context stream). With u64 keys "sort" is the re-sort, positions permuted
+        context stream). "sort" is the re-sort, positions permuted
         and cell starts updated in the same pass, unless the full radix sort ran
         (then "ranges" holds the cell starts and the permutation)."""
         out = np.zeros(4, np.float32)
