@@ -103,7 +103,15 @@ __device__ __forceinline__ void find_history(const ContactArgs& a, int os, int o
 constexpr int XCDS = 8;       // gfx950: 8 accelerator complex dies, one L2 each
 constexpr int CAND_UNROLL = 4; // candidate positions loaded per batch (loads in flight)
 static_assert(CAND_UNROLL - 1 <= CONTACT_POS_PAD, "sorted positions must be padded for a whole batch");
-constexpr int CONTACT_STAGE = 256;  // staged candidate positions per wave (4 KiB of LDS)
+constexpr int CONTACT_STAGE = 224;  // staged candidate positions per wave (3.5 KiB of LDS)
+constexpr int CONTACT_ITEMS = 128;  // contacts of a wave handed out at a time (their places in the same LDS)
+constexpr int CONTACT_PASS = 12;    // contacts of one sphere spread over the wave
+// float4s of LDS per wave: the stage of a search, or only what shares it, and
+// the contacts found by each lane
+constexpr int CONTACT_SHARED = CONTACT_ITEMS / 2 + 6 * WAVE / 4;
+constexpr int contact_lds(bool listed) { return (listed ? CONTACT_SHARED : CONTACT_STAGE) + CONTACT_PASS * WAVE / 4; }
+static_assert(LIST_CAP % CAND_UNROLL == 0, "whole batches of a list are read");
+static_assert(CONTACT_SHARED <= CONTACT_STAGE, "items and results fit the stage");
 
 // Orders one wave's LDS writes and reads (the lanes of a wave only).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -119,6 +127,24 @@ __device__ __forceinline__ int xcd_logical_block(int nblocks) {
     const int per = (nblocks + XCDS - 1) / XCDS;
     const int lb = (int)(blockIdx.x % XCDS) * per + (int)(blockIdx.x / XCDS);
     return lb < nblocks ? lb : -1;
+}
+
+// Largest of the wave's squared displacements into one of the step's maxima
+// (non-negative floats and not-a-numbers order as their bits do). The active
+// lanes are a prefix of the wave: DPP steps leave lane i the largest of lanes
+// 0 .. i.
+__device__ __forceinline__ void note_displacement(StepCtl* L, float d2) {
+    uint32_t u = __float_as_uint(d2);
+#define SD_STEP(ctrl, rows)                                                                                     \
+    {                                                                                                           \
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)u, (int)u, ctrl, rows, 0xf, false);       \
+        u = o > u ? o : u;                                                                                      \
+    }
+    SD_STEP(0x111, 0xf) SD_STEP(0x112, 0xf) SD_STEP(0x114, 0xf) SD_STEP(0x118, 0xf)  // row_shr 1, 2, 4, 8
+    SD_STEP(0x142, 0xa) SD_STEP(0x143, 0xc)                                          // row_bcast 15, 31
+#undef SD_STEP
+    const uint64_t m = __ballot(1);
+    if (lane_id() == 63 - __builtin_clzll(m)) atomicMax(&L->dmax[((blockIdx.x * 4u + (threadIdx.x >> 6)) & 63u) * 16u], u);
 }
 
 // MODE: CONTACT_FORCES writes force/torque; CONTACT_FUSED_* integrates and writes
@@ -142,24 +168,50 @@ __device__ __forceinline__ T uniform_copy(const T& src) {
 
 // STRADDLE (batch mode only): one 64-thread block per listed wave whose slots
 // span more than one scene; every lane then takes its own scene's parameters.
-// The work of one sphere slot s of a wave (its lanes are consecutive slots
-// of one wave, or the lanes of a straddling wave): everything the kernel does
-// once the slot is known.
-template <int MODE, bool INDIRECT, bool STRADDLE>
-__device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
+// The work of the 64 consecutive slots of one wave, slot the lane's: everything
+// the kernel does once the slot is known.
+//
+// In three parts. (1) Every lane finds its sphere's contacts, in ascending
+// sorted position: among its near list (LISTED), or by a search of the cells
+// around it (which also makes the list). (2) The wave's contacts, as one
+// sequence, are spread over its lanes, one contact a lane, so that a wave's
+// time goes with its number of contacts and not with the largest number of one
+// sphere, and the loads of 64 contacts are in flight together. (3) Every lane
+// adds up its sphere's forces in order.
+//
+// A step on lists moves about 200 bytes a sphere (state in and out, keys,
+// history count, a list row or two) and is bound by that in a dilute scene:
+// 4,194,304 spheres 181 us, where the search of every step took 312 (VALU
+// issue, 97 candidate tests a sphere). With 2 to 3 contacts a sphere the chain
+// of loads of a contact counts: 1,048,576 spheres 154 us (215 when each lane
+// went through its own contacts), 1,000 spheres 18 us (51). A step that makes
+// lists takes 416, 222 and 43 us, every 40th step or so.
+//
+// Two kernels: with the search as a branch of one, the steps on lists ran at 4
+// waves a SIMD or with spills (4,194,304 spheres 265 and 395 us).
+template <int MODE, bool INDIRECT, bool STRADDLE, bool LISTED>
+__device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
     constexpr bool BATCH = MODE == CONTACT_FUSED_BATCH;
-    constexpr bool PADDED = MODE != CONTACT_FORCES;  // fused modes read a context's padded buffer
-    if (s >= a.n) return;
+    constexpr bool FUSED = MODE != CONTACT_FORCES;
+    constexpr bool PADDED = FUSED;  // fused modes read a context's padded buffer
+    const int lane = lane_id();
+    const bool live = slot < a.n;  // lanes past the end take part in the wave's shared work
+    const int first = __builtin_amdgcn_readfirstlane(slot - lane);  // the wave's first slot
+    if (first >= a.n) return;
+    const int s = min(first + lane, a.n - 1);
     GridDev g;
     ContactDev c;
     const int* ranges;  // CONTACT_FORCES: (start, end) per cell; fused modes: cell starts
     uint32_t cbase = 0u;
+    float rmax = 0.0f;
     if constexpr (STRADDLE) {
-        const SceneDev& S = a.scenes[a.scene_of[s]];
+        const int sid = a.scene_of[s];
+        const SceneDev& S = a.scenes[sid];
         g = S.g;
         c = S.c;
         cbase = S.cbase;
         ranges = a.cell_start + cbase;
+        rmax = a.scene_rmax[sid];
     } else if constexpr (BATCH) {
         // one scene in the wave (the waves spanning two are in a.straddle and
         // run by the straddle launch): its parameters are wave-uniform
@@ -171,128 +223,239 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
         c = S.c;
         cbase = S.cbase;
         ranges = a.cell_start + cbase;
+        rmax = a.scene_rmax[sid];
     } else {
         g = a.g;
         c = a.c;
         ranges = MODE == CONTACT_FORCES ? a.ranges : a.cell_start;
+        rmax = a.rmax;
     }
-    float4 p = a.pos[s];
     const int os = old_slot_of(a, s);
-    const int self = INDIRECT ? os : s;
-    float4 v = a.vel[self];
-    float4 w = a.omg[self];
-    const int myid = a.ids[self];
+    const int self = INDIRECT ? os : s;  // the sphere's row: of the previous order, or the sorted one
+    const float4* const rowpos = INDIRECT ? a.pos_rows : a.pos;
+    // the velocity and spin are read where they are needed, after the
+    // contacts: held from here they cost a wave a SIMD
+    float4 p = rowpos[self];
+    const float inv_m = a.vel[self].w, inv_i = a.omg[self].w;
+    const int myid = FUSED ? a.ids[self] : 0;
     int oc = a.hcount_old[os];
     oc = oc < c.maxc ? oc : c.maxc;
+    int lcount = 0;      // LISTED: the sphere's list
+    float sigma = 0.0f;  // a search that makes lists: their margin
+    if constexpr (LISTED) lcount = live ? a.lcount_old[os] : 0;
+    else if (FUSED && a.lists == LIST_BUILD) sigma = a.ctl->sigma;
 
     int cx, cy, cz;
     cell_coords(g, p.x, p.y, p.z, cx, cy, cz);
+    const uint32_t cell_old = cbase + (uint32_t)((cz * g.ny + cy) * g.nx + cx);
     float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx = 0.0f, ty = 0.0f, tz = 0.0f;
     int nc = 0;
 
-    // one sphere-sphere contact with the sphere at sorted position t; the
-    // sphere itself and coincident spheres (d2 == 0) are not contacts
-    auto visit = [&](int t, const float4* sl) {
-        const float4 q = sl[t];  // the staged copy (LDS) of position t
-        const float dx = p.x - q.x;
-        const float dyy = p.y - q.y;
-        const float dzz = p.z - q.z;
-        const float d2 = dx * dx + dyy * dyy + dzz * dzz;
-        const float rs = p.w + q.w;
-        if (!(d2 < rs * rs) || d2 == 0.0f) return;
-        const int ot = INDIRECT ? old_slot_of(a, t) : t;
-        const float4 vq = a.vel[ot];
-        if (v.w + vq.w == 0.0f) return;  // two static spheres
-        const float4 wq = a.omg[ot];
-        const int pid = a.ids[ot];
-        const float d = sqrtf(d2);
-        const float inv_d = 1.0f / d;
-        const float nx = dx * inv_d, ny = dyy * inv_d, nz = dzz * inv_d;
-        float hx, hy, hz;
-        find_history(a, os, oc, pid, nc, hx, hy, hz);
-        const PairForce f = contact_law(c, nx, ny, nz, rs - d, p.w, q.w, v.w, vq.w, v.x - vq.x, v.y - vq.y,
-                                        v.z - vq.z, w.x, w.y, w.z, wq.x, wq.y, wq.z, hx, hy, hz);
-        fx = fx + f.fx;
-        fy = fy + f.fy;
-        fz = fz + f.fz;
-        tx = tx + f.tx;
-        ty = ty + f.ty;
-        tz = tz + f.tz;
-        if (nc < c.maxc) a.hist_new[(size_t)nc * a.n + s] = make_float4(hx, hy, hz, __int_as_float(pid));
-        ++nc;
+    // LDS of the wave: staged candidates of a search, later the contacts of the
+    // wave (row, owning lane and number) and 64 results; the rows of each
+    // lane's contacts (entry k of a lane at k * 64 + lane)
+    extern __shared__ float4 cstage[];
+    float4* const stg = cstage + (threadIdx.x >> 6) * contact_lds(LISTED);
+    int2* const items = reinterpret_cast<int2*>(stg);
+    float* const res = reinterpret_cast<float*>(stg + CONTACT_ITEMS / 2);
+    int* const pend = reinterpret_cast<int*>(stg + (LISTED ? CONTACT_SHARED : CONTACT_STAGE)) + lane;
+
+    // Whether the sphere at row `row`, closer than the radii, (dx, dy, dz) away
+    // and not coincident (the sphere itself, too), is a contact: not both
+    // static, and in the 27 cells around the sphere. Rounding of the cell of a
+    // sphere at a boundary can put a pair as far apart along an axis as the
+    // cell is wide two cells apart, which is no contact (nearer pairs cannot
+    // be, by far, on grids of up to 65,536 cells a side): a search of the 27
+    // cells does not meet it.
+    const float near = FUSED && a.lists != LIST_NONE
+                           ? (max(g.nx, max(g.ny, g.nz)) > 65536 ? 0.0f : 0.9f * g.cell)
+                           : 3.4e38f;
+    auto is_contact = [&](int row, float dx, float dyy, float dzz) -> bool {
+        if (fmaxf(fabsf(dx), fmaxf(fabsf(dyy), fabsf(dzz))) > near) {
+            const float4 q = rowpos[row];
+            int qx, qy, qz;
+            cell_coords(g, q.x, q.y, q.z, qx, qy, qz);
+            if (abs(qx - cx) > 1 || abs(qy - cy) > 1 || abs(qz - cz) > 1) return false;
+        }
+        return inv_m > 0.0f || a.vel[row].w > 0.0f;
     };
 
-    // Distance test of the candidates at sorted positions t0 .. t0+3 (q), then
-    // the contacts among them in ascending position order. Only the distance
-    // is tested per candidate; a batch with a possible contact in any lane
-    // (rare, and always the batch holding the sphere itself) then drops
-    // positions past hi and the sphere itself (position s, without a memory
-    // access), and visit() drops coincident spheres (d2 == 0).
-    auto test_batch = [&](const float4 (&q)[CAND_UNROLL], int t0, int hi, const float4* sl) {
-        bool h[CAND_UNROLL];
-        uint64_t any = 0u;  // lanes with a possible contact (scalar masks)
+    int hc = 0;     // contacts found; the first CONTACT_PASS of them are in pend
+    int pc = 0;     // contacts in pend
+    int after = -1; // LISTED: the place of the last one in pend
+    int ln = 0;     // listed neighbours
+    if (LISTED) {
+        // The listed spheres, in any order; their contacts in ascending
+        // new position: the order of the search, so of the sums and of the
+        // history. A list made by a search is ascending; only a sphere that
+        // changed cell moves in one. Positions come from the previous
+        // order's rows, so that the place of a sphere in the new order is
+        // off the chain of loads.
+        int k0 = 0;
+        do {  // (the first batch does not wait for the list's length)
+            int t[CAND_UNROLL], tn[CAND_UNROLL];
+            float4 q[CAND_UNROLL];
 #pragma unroll
-        for (int k = 0; k < CAND_UNROLL; ++k) {
-            const float dx = p.x - q[k].x;
-            const float dyy = p.y - q[k].y;
-            const float dzz = p.z - q[k].z;
-            const float d2 = dx * dx + dyy * dyy + dzz * dzz;
-            const float rs = p.w + q[k].w;
-            h[k] = d2 < rs * rs;
-            any |= __builtin_amdgcn_ballot_w64(h[k]);
-        }
-        if (any) {
-            uint32_t hit = 0u;
+            for (int k = 0; k < CAND_UNROLL; ++k) t[k] = a.list_old[(size_t)(k0 + k) * a.n + os];
 #pragma unroll
-            for (int k = 0; k < CAND_UNROLL; ++k) hit |= h[k] ? (1u << k) : 0u;
-            while (hit) {
-                const int k = __builtin_ctz(hit);
-                hit &= hit - 1u;
-                if (t0 + k < hi && t0 + k != s) visit(t0 + k, sl);
+            for (int k = 0; k < CAND_UNROLL; ++k) {
+                if (k0 + k >= lcount) t[k] = self;  // (past the list: whatever the row held)
+                q[k] = rowpos[t[k]];
+                tn[k] = a.newpos[t[k]];
+            }
+#pragma unroll
+            for (int k = 0; k < CAND_UNROLL; ++k) {
+                if (k0 + k >= lcount) break;
+                const int row = t[k], place = tn[k];
+                a.list_new[(size_t)(k0 + k) * a.n + s] = place;
+                const float dx = p.x - q[k].x;
+                const float dyy = p.y - q[k].y;
+                const float dzz = p.z - q[k].z;
+                const float d2 = dx * dx + dyy * dyy + dzz * dzz;
+                const float rs = p.w + q[k].w;
+                if (!(d2 < rs * rs) || d2 == 0.0f ||
+                    !is_contact(row, dx, dyy, dzz))
+                    continue;
+                ++hc;
+                const bool full = pc == CONTACT_PASS;
+                if (full) {
+                    if (place > after) continue;
+                    --pc;  // (the furthest one is left out)
+                }
+                int m = pc++;
+                if (place > after) {
+                    after = place;
+                } else {
+                    for (; m > 0; --m) {
+                        const int b = pend[(m - 1) * WAVE];
+                        if (a.newpos[b] < place) break;
+                        pend[m * WAVE] = b;
+                    }
+                }
+                pend[m * WAVE] = row;
+                if (full) after = a.newpos[pend[(pc - 1) * WAVE]];
+            }
+            k0 += CAND_UNROLL;
+        } while (k0 < lcount);
+    }
+    if (!LISTED && live) {
+        // Distance test of the candidates at sorted positions t0 .. t0+3
+        // (q). Only the distance is tested per candidate; a batch with a
+        // possible contact in any lane (rare, and always the batch holding
+        // the sphere itself) then drops positions past hi and the sphere
+        // itself (position s, without a memory access). While lists are
+        // built, the distance is the contact's plus the margin, and every
+        // sphere within it is listed.
+        const float reach = p.w + sigma;
+        auto test_batch = [&](const float4 (&q)[CAND_UNROLL], int t0, int hi, const float4* sl) {
+            bool h[CAND_UNROLL];
+            uint64_t any = 0u;  // lanes with a possible contact (scalar masks)
+#pragma unroll
+            for (int k = 0; k < CAND_UNROLL; ++k) {
+                const float dx = p.x - q[k].x;
+                const float dyy = p.y - q[k].y;
+                const float dzz = p.z - q[k].z;
+                const float d2 = dx * dx + dyy * dyy + dzz * dzz;
+                const float rs = reach + q[k].w;
+                h[k] = d2 < rs * rs;
+                any |= __builtin_amdgcn_ballot_w64(h[k]);
+            }
+            if (any) {
+                uint32_t hit = 0u;
+#pragma unroll
+                for (int k = 0; k < CAND_UNROLL; ++k) hit |= h[k] ? (1u << k) : 0u;
+                while (hit) {
+                    const int t = t0 + __builtin_ctz(hit);
+                    hit &= hit - 1u;
+                    if (t >= hi || t == s) continue;
+                    if constexpr (FUSED) {
+                        if (ln < LIST_CAP && a.lists == LIST_BUILD) a.list_new[(size_t)ln * a.n + s] = t;
+                        ++ln;
+                    }
+                    const float4 qt = sl[t];  // (the staged copy)
+                    const float dx = p.x - qt.x;
+                    const float dyy = p.y - qt.y;
+                    const float dzz = p.z - qt.z;
+                    const float d2 = dx * dx + dyy * dyy + dzz * dzz;
+                    const float rs = p.w + qt.w;
+                    if (!(d2 < rs * rs) || d2 == 0.0f) continue;
+                    const int row = INDIRECT ? old_slot_of(a, t) : t;
+                    if (!is_contact(row, dx, dyy, dzz)) continue;
+                    if (hc < CONTACT_PASS) pend[hc * WAVE] = row;
+                    ++hc;
+                }
+            }
+        };
+
+        // Candidate staging. The lanes of a wave are consecutive sorted
+        // spheres, so for one stencil row offset (dz, dy) their windows
+        // ascend with the lane (rows and cells are in sorted order). The
+        // lanes in the first active lane's grid row (segment A) and the
+        // others (segment B, normally the next row) each have a compact
+        // union of windows. The two unions, each followed by the 3
+        // positions a batch may read past a window, form one staged
+        // sequence: sorted position t of a lane is entry t + off of it.
+        // The wave copies the sequence into its LDS region with coalesced
+        // loads (in chunks of CONTACT_STAGE entries; one chunk unless the
+        // wave spans several sparse rows) and every lane tests its
+        // candidates in the chunk from LDS.
+        const uint64_t amask = __ballot(1);  // the searching lanes
+        const int arank = __popcll(amask & lanemask_lt());
+        const int nact = __popcll(amask);
+        const uint32_t rowid = cell_old - (uint32_t)cx;
+        const bool segB = rowid != (uint32_t)__builtin_amdgcn_readfirstlane((int)rowid);
+        const uint64_t bmask = __ballot(segB);
+        constexpr int PAD = CAND_UNROLL - 1;        // a batch reads up to 3 positions past its window
+        constexpr int CHUNK = CONTACT_STAGE - PAD;  // sequence entries tested per chunk
+        const char* const pos_bytes = reinterpret_cast<const char*>(a.pos);
+
+        // Rows of the search, in ascending order: the 27 cells around the
+        // sphere, or, while lists are built, the rows that a sphere within
+        // reach of it can lie in (the cell of a coordinate grows with it,
+        // so the cells of both ends of the reach bound them): fewer than
+        // nine for most spheres, one further out for a sphere near a cell
+        // boundary. e: cells on either side in x, the same for the wave
+        // (windows ascend with the lane).
+        int y0 = max(cy - 1, 0), y1 = min(cy + 1, g.ny - 1), z0 = max(cz - 1, 0), z1 = min(cz + 1, g.nz - 1);
+        int e = 1;
+        if constexpr (FUSED) {
+            if (a.lists == LIST_BUILD) {
+                const float R = (reach + rmax) * 1.0001f;
+                y0 = axis_cell(p.y - R, g.loy, g.cell, g.ny);
+                y1 = axis_cell(p.y + R, g.loy, g.cell, g.ny);
+                z0 = axis_cell(p.z - R, g.loz, g.cell, g.nz);
+                z1 = axis_cell(p.z + R, g.loz, g.cell, g.nz);
+                const int x0 = axis_cell(p.x - R, g.lox, g.cell, g.nx);
+                const int x1 = axis_cell(p.x + R, g.lox, g.cell, g.nx);
+                e = __ballot(cx - x0 > 1 || x1 - cx > 1) ? 2 : 1;
             }
         }
-    };
-
-    // Candidate staging. The lanes of a wave are consecutive sorted spheres, so
-    // for one stencil row offset (dz, dy) their windows ascend with the lane
-    // (rows and cells are in sorted order). The lanes in the first active
-    // lane's grid row (segment A) and the others (segment B, normally the next
-    // row) each have a compact union of windows. The two unions, each followed
-    // by the 3 positions a batch may read past a window, form one staged
-    // sequence: sorted position t of a lane is entry t + off of it. The wave
-    // copies the sequence into its LDS region with coalesced loads (in chunks
-    // of CONTACT_STAGE entries; one chunk unless the wave spans several sparse
-    // rows) and every lane tests its candidates in the chunk from LDS.
-    extern __shared__ float4 cstage[];
-    float4* const stg = cstage + (threadIdx.x >> 6) * CONTACT_STAGE;
-    const uint64_t amask = __ballot(1);  // active lanes: a prefix of the wave
-    const int arank = __popcll(amask & lanemask_lt());
-    const int nact = __popcll(amask);
-    const uint32_t rowid = cbase + (uint32_t)((cz * g.ny + cy) * g.nx);
-    const bool segB = rowid != (uint32_t)__builtin_amdgcn_readfirstlane((int)rowid);
-    const uint64_t bmask = __ballot(segB);
-    constexpr int PAD = CAND_UNROLL - 1;        // a batch reads up to 3 positions past its window
-    constexpr int CHUNK = CONTACT_STAGE - PAD;  // sequence entries tested per chunk
-    const char* const pos_bytes = reinterpret_cast<const char*>(a.pos);
-
-    // window of stencil row r (rows (dz, dy) in ascending order); the next
-    // row's window is loaded while a row is copied and tested
-    auto window = [&](int r, int& lo, int& hi) {
-        const int z = cz + r / 3 - 1, y = cy + r % 3 - 1;
-        lo = 0;
-        hi = 0;
-        if (z >= 0 && z < g.nz && y >= 0 && y < g.ny) {
-            if constexpr (MODE == CONTACT_FORCES) row_range(g, ranges, cx, y, z, lo, hi);
-            else row_window(g, ranges, cx, y, z, lo, hi);
-        }
-    };
-    int next_lo, next_hi;
-    window(0, next_lo, next_hi);
+        // row offsets (dz, dy) that some lane of the wave has
+        const int dz0 = __ballot(z0 < cz - 1) ? -2 : (__ballot(z0 < cz) ? -1 : 0);
+        const int dz1 = __ballot(z1 > cz + 1) ? 2 : (__ballot(z1 > cz) ? 1 : 0);
+        const int dy0 = __ballot(y0 < cy - 1) ? -2 : (__ballot(y0 < cy) ? -1 : 0);
+        const int dy1 = __ballot(y1 > cy + 1) ? 2 : (__ballot(y1 > cy) ? 1 : 0);
+        // window of a row; the next row's window is loaded while a row is
+        // copied and tested
+        auto window = [&](int dz, int dy, int& lo, int& hi) {
+            const int z = cz + dz, y = cy + dy;
+            lo = 0;
+            hi = 0;
+            if (z >= z0 && z <= z1 && y >= y0 && y <= y1) {
+                if constexpr (MODE == CONTACT_FORCES) row_range(g, ranges, cx, y, z, lo, hi);
+                else row_window(g, ranges, cx, e, y, z, lo, hi);
+            }
+        };
+        int next_lo, next_hi, dz = dz0, dy = dy0;
+        window(dz, dy, next_lo, next_hi);
 #pragma unroll 1
-    for (int r = 0; r < 9; ++r) {
-        {
+        while (dz <= dz1) {
             const int lo = next_lo, hi = next_hi;
-            if (r + 1 < 9) window(r + 1, next_lo, next_hi);
+            if (++dy > dy1) {
+                dy = dy0;
+                ++dz;
+            }
+            if (dz <= dz1) window(dz, dy, next_lo, next_hi);
             const uint64_t ne = __ballot(hi > lo);
             if (ne == 0u) continue;
             const uint64_t ma = ne & ~bmask, mb = ne & bmask;
@@ -341,10 +504,151 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
         }
     }
 
+    asm volatile("" ::"v"(inv_i));  // (the row is in the cache by now; not held further)
+
+    // the wave's contacts: lane l's are [off, off + pc)
+    if (!LISTED) pc = min(hc, CONTACT_PASS);
+    const int inc = (int)wave_inclusive_scan((uint32_t)pc);
+    const int off = inc - pc;
+    const int total = __builtin_amdgcn_readlane(inc, 63);
+    for (int c0 = 0; c0 < total; c0 += CONTACT_ITEMS) {
+        for (int j = max(c0 - off, 0); j < pc && off + j < c0 + CONTACT_ITEMS; ++j)
+            items[off + j - c0] = make_int2(pend[j * WAVE], lane | (j << 8));
+        wave_lds_sync();
+        const int ce = min(total - c0, CONTACT_ITEMS);
+        for (int i0 = 0; i0 < ce; i0 += WAVE) {
+            const bool on = i0 + lane < ce;
+            const int2 it = items[on ? i0 + lane : 0];
+            const int row = it.x, ow = it.y & 63;
+            // the owner's row, old slot, history entries and entry of this contact
+            const int oself = __shfl(self, ow);
+            const int oos = INDIRECT ? oself : __shfl(os, ow);
+            const int ooc = __shfl(oc, ow);
+            const int k = __shfl(nc, ow) + (it.y >> 8);
+            ContactDev lc = c;
+            if constexpr (STRADDLE) {
+                lc.kn = __shfl(c.kn, ow);
+                lc.kt = __shfl(c.kt, ow);
+                lc.c2z = __shfl(c.c2z, ow);
+                lc.mu = __shfl(c.mu, ow);
+            }
+            if (on) {
+                const float4 pi = rowpos[oself], pj = rowpos[row];
+                const float4 vi = a.vel[oself], vj = a.vel[row];
+                const float4 wi = a.omg[oself], wj = a.omg[row];
+                const int pid = a.ids[row];
+                const float dx = pi.x - pj.x;
+                const float dyy = pi.y - pj.y;
+                const float dzz = pi.z - pj.z;
+                const float d2 = dx * dx + dyy * dyy + dzz * dzz;
+                const float d = sqrtf(d2);
+                const float inv_d = 1.0f / d;
+                const float nx = dx * inv_d, ny = dyy * inv_d, nz = dzz * inv_d;
+                float hx, hy, hz;
+                find_history(a, oos, ooc, pid, k, hx, hy, hz);
+                const PairForce f =
+                    contact_law(lc, nx, ny, nz, (pi.w + pj.w) - d, pi.w, pj.w, vi.w, vj.w, vi.x - vj.x,
+                                vi.y - vj.y, vi.z - vj.z, wi.x, wi.y, wi.z, wj.x, wj.y, wj.z, hx, hy, hz);
+                res[lane] = f.fx;
+                res[64 + lane] = f.fy;
+                res[128 + lane] = f.fz;
+                res[192 + lane] = f.tx;
+                res[256 + lane] = f.ty;
+                res[320 + lane] = f.tz;
+                if (k < lc.maxc)
+                    a.hist_new[(size_t)k * a.n + (first + ow)] = make_float4(hx, hy, hz, __int_as_float(pid));
+            }
+            wave_lds_sync();
+            // this lane's results, in order
+            const int f0 = c0 + i0;
+            for (int j = max(f0 - off, 0); j < pc && off + j < f0 + WAVE; ++j) {
+                const float* const r = res + (off + j - f0);
+                fx = fx + r[0];
+                fy = fy + r[64];
+                fz = fz + r[128];
+                tx = tx + r[192];
+                ty = ty + r[256];
+                tz = tz + r[320];
+            }
+            wave_lds_sync();
+        }
+    }
+    nc += pc;
+
+    // A sphere with more contacts than that (one large sphere among many small
+    // ones): the others one after the other. A second pass of the code above
+    // instead, in a loop around it, took 25 registers more.
+    if (__ballot(hc > CONTACT_PASS) != 0u && hc > CONTACT_PASS) {
+        auto add = [&](int row) {
+            const float4 q = rowpos[row], vi = a.vel[self], vj = a.vel[row], wi = a.omg[self], wj = a.omg[row];
+            const int pid = a.ids[row];
+            const float dx = p.x - q.x;
+            const float dyy = p.y - q.y;
+            const float dzz = p.z - q.z;
+            const float d = sqrtf(dx * dx + dyy * dyy + dzz * dzz);
+            const float inv_d = 1.0f / d;
+            float hx, hy, hz;
+            find_history(a, os, oc, pid, nc, hx, hy, hz);
+            const PairForce f = contact_law(c, dx * inv_d, dyy * inv_d, dzz * inv_d, (p.w + q.w) - d, p.w, q.w, vi.w,
+                                            vj.w, vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, wi.x, wi.y, wi.z, wj.x, wj.y,
+                                            wj.z, hx, hy, hz);
+            fx = fx + f.fx;
+            fy = fy + f.fy;
+            fz = fz + f.fz;
+            tx = tx + f.tx;
+            ty = ty + f.ty;
+            tz = tz + f.tz;
+            if (nc < c.maxc) a.hist_new[(size_t)nc * a.n + s] = make_float4(hx, hy, hz, __int_as_float(pid));
+            ++nc;
+        };
+        auto touches = [&](int row) -> bool {
+            const float4 q = rowpos[row];
+            const float dx = p.x - q.x;
+            const float dyy = p.y - q.y;
+            const float dzz = p.z - q.z;
+            const float d2 = dx * dx + dyy * dyy + dzz * dzz;
+            const float rs = p.w + q.w;
+            return d2 < rs * rs && d2 != 0.0f && is_contact(row, dx, dyy, dzz);
+        };
+        if constexpr (LISTED) {
+            while (nc < hc) {  // the next one in ascending place
+                int best = 0x7fffffff, row = 0;
+                for (int k = 0; k < lcount; ++k) {
+                    const int t = a.list_old[(size_t)k * a.n + os], place = a.newpos[t];
+                    if (place > after && place < best && touches(t)) {
+                        best = place;
+                        row = t;
+                    }
+                }
+                after = best;
+                add(row);
+            }
+        } else {
+            int skip = CONTACT_PASS;
+            for (int r = 0; r < 9 && nc < hc; ++r) {
+                const int z = cz + r / 3 - 1, y = cy + r % 3 - 1;
+                if (z < 0 || z >= g.nz || y < 0 || y >= g.ny) continue;
+                int lo, hi;
+                if constexpr (MODE == CONTACT_FORCES) row_range(g, ranges, cx, y, z, lo, hi);
+                else row_window(g, ranges, cx, 1, y, z, lo, hi);
+                for (int t = lo; t < hi && nc < hc; ++t) {
+                    if (t == s) continue;
+                    const int row = INDIRECT ? old_slot_of(a, t) : t;
+                    if (!touches(row)) continue;
+                    if (skip > 0) --skip;
+                    else add(row);
+                }
+            }
+        }
+    }
+
+    float4 v = a.vel[self];
+    float4 w = a.omg[self];
+
     // walls: the touched ones first, so that the contact-law set-up of a wall
     // contact runs only where some lane of the wave touches a wall
     uint32_t touch = 0u;
-    if (c.walls && v.w > 0.0f) {
+    if (c.walls && v.w > 0.0f && live) {
 #pragma unroll
         for (int wl = 0; wl < 6; ++wl) {
             const int ax = wl >> 1;
@@ -355,13 +659,15 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
         }
     }
     if (touch) {
-#pragma unroll
-        for (int wl = 0; wl < 6; ++wl) {
-            if (!((touch >> wl) & 1u)) continue;
+#pragma unroll 1
+        for (; touch; touch &= touch - 1u) {
+            const int wl = __builtin_ctz(touch);
             const int ax = wl >> 1;
             const bool upper = wl & 1;
             const float pc = ax == 0 ? p.x : (ax == 1 ? p.y : p.z);
-            const float dist = upper ? c.whi[ax] - pc : pc - c.wlo[ax];
+            const float wlo = ax == 0 ? c.wlo[0] : (ax == 1 ? c.wlo[1] : c.wlo[2]);
+            const float whi = ax == 0 ? c.whi[0] : (ax == 1 ? c.whi[1] : c.whi[2]);
+            const float dist = upper ? whi - pc : pc - wlo;
             const float sgn = upper ? -1.0f : 1.0f;
             const float nx = ax == 0 ? sgn : 0.0f;
             const float ny = ax == 1 ? sgn : 0.0f;
@@ -382,26 +688,40 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
         }
     }
 
-    a.hcount_new[s] = nc < c.maxc ? nc : c.maxc;
+    if (live) a.hcount_new[s] = nc < c.maxc ? nc : c.maxc;
     if (nc > c.maxc) atomicMax(a.overflow, nc);
 
     if (MODE == CONTACT_FORCES) {
-        a.force[s] = make_float4(fx, fy, fz, 0.0f);
-        a.torque[s] = make_float4(tx, ty, tz, 0.0f);
+        if (live) {
+            a.force[s] = make_float4(fx, fy, fz, 0.0f);
+            a.torque[s] = make_float4(tx, ty, tz, 0.0f);
+        }
     } else {
+        if constexpr (LISTED) {
+            if (live) a.lcount_new[s] = (uint8_t)lcount;
+        } else if (a.lists == LIST_BUILD) {
+            if (live) a.lcount_new[s] = (uint8_t)min(ln, LIST_CAP);
+            if (__ballot(live && ln > LIST_CAP) != 0u && lane == 0) a.ctl->over = 1;
+        }
+        const float ox = p.x, oy = p.y, oz = p.z;
         integrate_sphere(c, p, v, w, fx, fy, fz, tx, ty, tz);
-        a.pos_o[s] = p;
-        a.vel_o[s] = v;
-        a.omg_o[s] = w;
-        a.ids_o[s] = myid;
+        {
+            const float dx = p.x - ox, dyy = p.y - oy, dzz = p.z - oz;
+            note_displacement(a.ctl, live ? dx * dx + dyy * dyy + dzz * dzz : 0.0f);
+        }
+        if (live) {
+            a.pos_o[s] = p;
+            a.vel_o[s] = v;
+            a.omg_o[s] = w;
+            a.ids_o[s] = myid;
+        }
         {
             const uint32_t cell_new = cbase + cell_id(g, p.x, p.y, p.z);
             const uint64_t key_new = ((uint64_t)cell_new << 32) | (uint64_t)(uint32_t)s;
-            a.keys_o64[s] = key_new;
+            if (live) a.keys_o64[s] = key_new;
             // a sphere that left the cell it was sorted in: listed for the next
             // step's re-sort (one atomic per wave)
-            const uint32_t cell_old = cbase + (uint32_t)((cz * g.ny + cy) * g.nx + cx);
-            const bool moved = a.mcount != nullptr && cell_new != cell_old;
+            const bool moved = a.mcount != nullptr && live && cell_new != cell_old;
             const uint64_t m = __ballot(moved);
             if (moved) {
                 const int leader = __ffsll((long long)m) - 1;
@@ -419,12 +739,13 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int s) {
 }
 
 
-template <int MODE, bool INDIRECT, bool STRADDLE = false>
+template <int MODE, bool INDIRECT, bool STRADDLE, bool LISTED>
 __global__ __launch_bounds__(256) void k_contacts(ContactArgs a) {
     static_assert(!STRADDLE || MODE == CONTACT_FUSED_BATCH, "k_contacts: straddling waves exist in batch mode only");
-    if (a.step_ctl) {
-        if (a.step_ctl[0]) return;  // the step was given up
-        if (!STRADDLE && blockIdx.x == 0 && threadIdx.x == 0) a.step_ctl[1] += 1;
+    static_assert(!LISTED || INDIRECT, "k_contacts: only a context's steps have lists");
+    if (MODE != CONTACT_FORCES) {
+        if (a.ctl->given_up) return;
+        if (!STRADDLE && blockIdx.x == 0 && threadIdx.x == 0) a.ctl->ran += 1;
     }
     int s;
     if constexpr (STRADDLE) {
@@ -434,7 +755,7 @@ __global__ __launch_bounds__(256) void k_contacts(ContactArgs a) {
         if (lb < 0) return;
         s = lb * (int)blockDim.x + (int)threadIdx.x;
     }
-    contact_wave<MODE, INDIRECT, STRADDLE>(a, s);
+    contact_wave<MODE, INDIRECT, STRADDLE, LISTED>(a, s);
 }
 
 constexpr int PERSIST_CLAIM = 8;    // tiles a wave claims at a time
@@ -445,13 +766,11 @@ constexpr int PERSIST_STRIDE = 64;  // ints between the XCDs' counters
 // x-th eighth of the slots, so an XCD's L2 still holds neighbouring cells)
 // until its range is exhausted; the results are those of k_contacts (every
 // tile computes the same slots the same way). counters[0..7] start at 0.
-template <int MODE, bool INDIRECT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_contacts_persistent(
+template <int MODE, bool LISTED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_contacts_persistent(
     ContactArgs a, int* __restrict__ counters) {
-    if (a.step_ctl) {
-        if (a.step_ctl[0]) return;  // the step was given up
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.step_ctl[1] += 1;
-    }
+    if (a.ctl->given_up) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->ran += 1;
     const int ntiles = (a.n + WAVE - 1) / WAVE;
     const int per = (ntiles + XCDS - 1) / XCDS;
     const int x = (int)(blockIdx.x % XCDS);
@@ -463,7 +782,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         t = t0 + __shfl(t, 0);
         if (t >= t1) break;
         const int te = min(t + PERSIST_CLAIM, t1);
-        for (; t < te; ++t) contact_wave<MODE, INDIRECT, false>(a, t * WAVE + lane_id());
+        for (; t < te; ++t) contact_wave<MODE, true, false, LISTED>(a, t * WAVE + lane_id());
     }
 }
 
@@ -485,13 +804,18 @@ sd_status launch_contacts(int mode, const ContactArgs& a, hipStream_t s, int blo
     SD_REQUIRE(block % WAVE == 0 && block <= 256, "contact kernel: block must be a multiple of 64, <= 256");
     const int nblocks = div_up(a.n, block);
     const dim3 grid(div_up(nblocks, XCDS) * XCDS);  // padded for the XCD remap
-    const size_t lds = (size_t)(block / WAVE) * CONTACT_STAGE * sizeof(float4);
+    const bool listed = mode != CONTACT_FORCES && a.lists == LIST_USE;
+    const size_t lds = (size_t)(block / WAVE) * contact_lds(listed) * sizeof(float4);
     if (mode == CONTACT_FORCES)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FORCES, false>), grid, dim3(block), lds, s, a);
+        hipLaunchKernelGGL((k_contacts<CONTACT_FORCES, false, false, false>), grid, dim3(block), lds, s, a);
+    else if (mode == CONTACT_FUSED_U64 && listed)
+        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U64, true, false, true>), grid, dim3(block), lds, s, a);
     else if (mode == CONTACT_FUSED_U64)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U64, true>), grid, dim3(block), lds, s, a);
+        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U64, true, false, false>), grid, dim3(block), lds, s, a);
+    else if (listed)
+        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, false, true>), grid, dim3(block), lds, s, a);
     else
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true>), grid, dim3(block), lds, s, a);
+        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, false, false>), grid, dim3(block), lds, s, a);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }
@@ -502,16 +826,17 @@ sd_status launch_contacts_persistent(int mode, const ContactArgs& a, hipStream_t
     SD_REQUIRE(block % WAVE == 0 && block <= 256, "contact kernel: block must be a multiple of 64, <= 256");
     SD_REQUIRE(mode == CONTACT_FUSED_U64 || mode == CONTACT_FUSED_BATCH,
                "contact kernel: the persistent form is for packed 64-bit keys");
-    const size_t lds = (size_t)(block / WAVE) * CONTACT_STAGE * sizeof(float4);
+    const bool listed = a.lists == LIST_USE;
+    void (*const kernel)(ContactArgs, int*) =
+        mode == CONTACT_FUSED_U64 ? (listed ? &k_contacts_persistent<CONTACT_FUSED_U64, true>
+                                            : &k_contacts_persistent<CONTACT_FUSED_U64, false>)
+                                  : (listed ? &k_contacts_persistent<CONTACT_FUSED_BATCH, true>
+                                            : &k_contacts_persistent<CONTACT_FUSED_BATCH, false>);
+    const size_t lds = (size_t)(block / WAVE) * contact_lds(listed) * sizeof(float4);
     int dev = 0, cus = 0, per_cu = 0;
     SD_HIP(hipGetDevice(&dev));
     SD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    if (mode == CONTACT_FUSED_U64)
-        SD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(&k_contacts_persistent<CONTACT_FUSED_U64, true>), block, lds));
-    else
-        SD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(&k_contacts_persistent<CONTACT_FUSED_BATCH, true>), block, lds));
+    SD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), block, lds));
     // every resident block, at most one per tile, a multiple of the XCD count
     const int tiles = div_up(a.n, WAVE);
     int nb = std::max(1, per_cu) * std::max(1, cus);
@@ -519,12 +844,7 @@ sd_status launch_contacts_persistent(int mode, const ContactArgs& a, hipStream_t
     nb = std::max(XCDS, nb / XCDS * XCDS);
     sd_status st = launch_fill_u32((uint32_t*)counters, 0u, (size_t)PERSIST_STRIDE * XCDS, s);
     if (st != SD_OK) return st;
-    if (mode == CONTACT_FUSED_U64)
-        hipLaunchKernelGGL((k_contacts_persistent<CONTACT_FUSED_U64, true>), dim3(nb), dim3(block), lds, s, a,
-                           counters);
-    else
-        hipLaunchKernelGGL((k_contacts_persistent<CONTACT_FUSED_BATCH, true>), dim3(nb), dim3(block), lds, s, a,
-                           counters);
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(block), lds, s, a, counters);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }
@@ -532,8 +852,14 @@ sd_status launch_contacts_persistent(int mode, const ContactArgs& a, hipStream_t
 sd_status launch_contacts_straddle(const ContactArgs& a, hipStream_t s) {
     if (a.n <= 0 || a.n_straddle <= 0) return SD_OK;
     SD_REQUIRE(a.straddle && a.scenes && a.scene_of, "contact kernel: straddle launch without its lists");
-    const size_t lds = (size_t)CONTACT_STAGE * sizeof(float4);
-    hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, true>), dim3(a.n_straddle), dim3(WAVE), lds, s, a);
+    const bool listed = a.lists == LIST_USE;
+    const size_t lds = (size_t)contact_lds(listed) * sizeof(float4);
+    if (listed)
+        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, true, true>), dim3(a.n_straddle), dim3(WAVE), lds, s,
+                           a);
+    else
+        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, true, false>), dim3(a.n_straddle), dim3(WAVE), lds,
+                           s, a);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }

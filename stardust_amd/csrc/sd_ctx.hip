@@ -68,17 +68,22 @@ __global__ __launch_bounds__(DIAG_BLOCK) void k_diag_partial(const float4* __res
 struct GraphKey {
     int keys, hist, state;
     bool full;  // two steps with the full radix sort (dense runs)
+    int lists;  // what they do with the near lists
     bool operator<(const GraphKey& o) const {
         if (keys != o.keys) return keys < o.keys;
         if (hist != o.hist) return hist < o.hist;
         if (state != o.state) return state < o.state;
-        return full < o.full;
+        if (full != o.full) return full < o.full;
+        return lists < o.lists;
     }
 };
 
 // Full-sort steps run between two reads of the changed-cell count while a
 // scene is dense (more changed cells per step than the re-sort takes).
 constexpr int DENSE_CHUNK = 16;
+// Steps run between two looks at how long the near lists last, or whether they
+// would do.
+constexpr int LIST_REST = 64;
 
 }  // namespace sd
 
@@ -113,7 +118,7 @@ struct sd_ctx {
     int* hcount[2] = {nullptr, nullptr};
     float4* hist[2] = {nullptr, nullptr};
     int cur_hist = 0;
-    int* overflow = nullptr;
+    StepCtl* ctl = nullptr;
     // spheres that changed cell in the last step (u64 keys): count (set above
     // the cap to force the full sort), new and old keys, and the same sorted
     int* mcount = nullptr;
@@ -121,8 +126,18 @@ struct sd_ctx {
     uint64_t* mold = nullptr;
     uint64_t* msn = nullptr;
     uint64_t* mso = nullptr;
-    // [0] != 0: a re-sort step was given up; [1] steps run since the last reset
-    int* step_ctl = nullptr;
+    // near lists, alternating with the history buffers (sd_internal.hpp)
+    uint8_t* lcount[2] = {nullptr, nullptr};
+    int* list[2] = {nullptr, nullptr};
+    int* newpos = nullptr;
+    float list_cell = 0.0f;  // smallest cell edge; 0: no lists (spheres larger than their cell)
+    float rmax = 0.0f;
+    float* scene_rmax = nullptr;
+    int list_steps = 0;     // steps that the lists are expected to last (0: build them next)
+    int list_rest = 0;      // steps to run without lists before they are tried again
+    float last_move = -1.0f; // largest displacement of a step, as last read back (negative: not known)
+    bool crowded = false;    // the last lists did not hold some sphere's neighbours
+    int last_ovf = 0;        // StepCtl::overflow as last read back
     bool need_full = true;  // the next step's keys are not from a step of this order
     bool dense = false;     // the last full-sort step had more changed cells than the re-sort takes
     double* diag = nullptr;
@@ -172,9 +187,10 @@ void release(sd_ctx* c) {
     stage_release(c->stage);
     void* bufs[] = {c->pos[0], c->pos[1], c->vel[0], c->vel[1], c->omg[0], c->omg[1], c->ids[0], c->ids[1],
                     c->posB, c->k64[0], c->k64[1], c->sort_tmp,
-                    c->cell_start, c->hcount[0], c->hcount[1], c->hist[0], c->hist[1], c->overflow, c->diag,
+                    c->cell_start, c->hcount[0], c->hcount[1], c->hist[0], c->hist[1], c->ctl, c->diag,
                     c->scenes_d, c->scene_of, c->straddle, c->mcount, c->mnew, c->mold, c->msn, c->mso,
-                    c->step_ctl};
+                    c->lcount[0], c->lcount[1], c->list[0], c->list[1], c->newpos,
+                    c->scene_rmax};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (int k = 0; k < 2; ++k) {
@@ -187,10 +203,13 @@ void release(sd_ctx* c) {
     c->cell_start = nullptr;
     c->hcount[0] = c->hcount[1] = nullptr;
     c->hist[0] = c->hist[1] = nullptr;
-    c->overflow = nullptr;
+    c->ctl = nullptr;
     c->mcount = nullptr;
     c->mnew = c->mold = c->msn = c->mso = nullptr;
-    c->step_ctl = nullptr;
+    c->lcount[0] = c->lcount[1] = nullptr;
+    c->list[0] = c->list[1] = nullptr;
+    c->newpos = nullptr;
+    c->scene_rmax = nullptr;
     c->diag = nullptr;
     c->scenes_d = nullptr;
     c->scene_of = nullptr;
@@ -211,9 +230,10 @@ sd_status dalloc(T** p, size_t count) {
 // recorded before the sort and after the sort, cell-start, permute and contact stages.
 // full: the radix sort instead of the re-sort from the previous
 // order. A re-sort step that finds more than resort_cap(n) changed cells is given
-// up on the device (step_ctl[0]), together with every later step of the same
-// launch sequence; the host then redoes it as a full step (run_steps).
-sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
+// up on the device (StepCtl::given_up), together with every later step of the
+// same launch sequence; the host then redoes it as a full step (run_steps).
+// lists: what the step does with the near lists (LIST_USE only on a re-sort).
+sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev, bool full, int lists) {
     hipStream_t s = c->stream;
 #define MARK(i) \
     if (ev) SD_HIP(hipEventRecord(ev[i], s))
@@ -222,6 +242,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
     const int so = c->cur_state, sn = 1 - c->cur_state;
     ContactArgs a = {};
     a.pos = c->posB;
+    a.pos_rows = c->pos[so];
     a.vel = c->vel[so];
     a.omg = c->omg[so];
     a.ids = c->ids[so];
@@ -233,7 +254,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
     a.hist_old = c->hist[ho];
     a.hcount_new = c->hcount[hn];
     a.hist_new = c->hist[hn];
-    a.overflow = c->overflow;
+    a.overflow = &c->ctl->overflow;
     a.pos_o = c->pos[sn];
     a.vel_o = c->vel[sn];
     a.omg_o = c->omg[sn];
@@ -262,7 +283,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
     } else {
         // also updates the cell starts and sets mc_write = 0
         st = launch_resort_u64(mc_read, resort_cap(n), c->mnew, c->mold, c->msn, c->mso, K, n, c->cell_start, c->n_cells,
-                               c->pos[so], c->posB, Ka, mc_write, c->step_ctl, s);
+                               c->pos[so], c->posB, Ka, mc_write, c->ctl, c->newpos, lists, c->list_cell, s);
         uint64_t* t = K;
         K = Ka;
         Ka = t;
@@ -270,8 +291,8 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
     if (st != SD_OK) return st;
     MARK(1);
     // after the full sort: cell starts, the permutation, mc_write = 0
-    if (full) st = launch_step_starts_u64(K, n, c->n_cells, c->cell_start, c->step_ctl, true, c->pos[so],
-                                          c->posB, mc_write, s);
+    if (full) st = launch_step_starts_u64(K, n, c->n_cells, c->cell_start, &c->ctl->given_up, true, c->pos[so],
+                                          c->posB, mc_write, nullptr, c->ctl, lists, c->list_cell, s);
     if (st != SD_OK) return st;
     MARK(2);
     MARK(3);
@@ -281,11 +302,19 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
     a.mnew = c->mnew;
     a.mold = c->mold;
     a.mcap = resort_cap(n);
-    a.step_ctl = c->step_ctl;
+    a.ctl = c->ctl;
+    a.lists = lists;
     a.scenes = c->scenes_d;
     a.scene_of = c->scene_of;
     a.straddle = c->straddle;
     a.n_straddle = c->n_straddle;
+    a.lcount_old = c->lcount[ho];
+    a.list_old = c->list[ho];
+    a.lcount_new = c->lcount[hn];
+    a.list_new = c->list[hn];
+    a.newpos = c->newpos;
+    a.rmax = c->rmax;
+    a.scene_rmax = c->scene_rmax;
     // waves spanning two scenes: their own launch, beside the main one
     // (disjoint spheres; shared counters are atomics)
     const bool fork = c->batch && c->n_straddle > 0;
@@ -312,14 +341,14 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev = nullptr, bool full = false) {
     return SD_OK;
 }
 
-sd_status run_graph_pair(sd_ctx* c, bool full = false) {
-    const GraphKey key{c->cur_keys, c->cur_hist, c->cur_state, full};
+sd_status run_graph_pair(sd_ctx* c, bool full, int lists) {
+    const GraphKey key{c->cur_keys, c->cur_hist, c->cur_state, full, lists};
     auto it = c->graphs.find(key);
     if (it == c->graphs.end()) {
         const int k0 = c->cur_keys, h0 = c->cur_hist, s0 = c->cur_state;
         SD_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        sd_status st = enqueue_step(c, nullptr, full);
-        if (st == SD_OK) st = enqueue_step(c, nullptr, full);
+        sd_status st = enqueue_step(c, nullptr, full, lists);
+        if (st == SD_OK) st = enqueue_step(c, nullptr, full, lists);
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         if (st != SD_OK) {
@@ -346,6 +375,22 @@ sd_status run_graph_pair(sd_ctx* c, bool full = false) {
     return SD_OK;
 }
 
+// Steps that lists of margin sigma are expected to last from `displaced` on, a
+// tenth short of what the last displacement says (a shortfall costs a given-up
+// launch sequence, a surplus a build a few steps early).
+int list_life(float displaced, float sigma, float last) {
+    const float steps = 0.9f * (0.49f * sigma - displaced) / fmaxf(last, 1e-30f);
+    return steps >= (float)LIST_REST ? LIST_REST : (steps > 0.0f ? (int)steps : 0);  // (not a number: 0)
+}
+
+// Whether near lists pay at the scene's speed: not where even the largest
+// margin would last fewer than 4 steps, nor in dense runs (whose spheres cross
+// cells). Steps with rigid bodies attached keep none: a given-up sphere step
+// would not take the bodies' step back.
+bool lists_pay(const sd_ctx* c) {
+    return !c->dense && !c->hulls && c->list_cell > 0.0f && 8.0f * c->last_move <= LIST_MAX * c->list_cell;
+}
+
 // Runs nsteps steps: re-sort steps (graph-replayed in pairs when
 // use_graph), and a full step first whenever the keys are not from a step of
 // this order, or a re-sort step was given up. The device counts the steps that
@@ -356,53 +401,66 @@ sd_status run_steps(sd_ctx* c, int nsteps) {
         drop_graphs(c);  // captured with the attached bodies' previous step
         c->hull_gen = hull_generation(c->hulls);
     }
+    // steps of one kind: graph pairs, then singly
+    auto run = [&](int l, bool full, int lists) -> sd_status {
+        sd_status e = SD_OK;
+        for (; c->p.use_graph && l >= 2 && e == SD_OK; l -= 2) e = run_graph_pair(c, full, lists);
+        for (; l > 0 && e == SD_OK; --l) e = enqueue_step(c, nullptr, full, lists);
+        return e;
+    };
     int left = nsteps;
     while (left > 0) {
-        st = launch_fill_u32((uint32_t*)c->step_ctl, 0u, 2, c->stream);
+        st = launch_fill_u32((uint32_t*)c->ctl, 0u, 2, c->stream);  // given_up, ran
         if (st != SD_OK) return st;
         const int h0 = c->cur_hist, s0 = c->cur_state;
         const bool full = c->need_full || c->dense;
-        if (full) {
-            // one full-sort step after a given-up step or an upload; while the
-            // scene is dense, DENSE_CHUNK of them (graph pairs) before the
-            // changed-cell count is read again
-            int l = c->dense ? std::min(left, DENSE_CHUNK) : 1;
-            if (c->p.use_graph) {
-                while (l >= 2) {
-                    st = run_graph_pair(c, true);
-                    if (st != SD_OK) return st;
-                    l -= 2;
-                }
-            }
-            for (; l > 0; --l) {
-                st = enqueue_step(c, nullptr, true);
-                if (st != SD_OK) return st;
-            }
-            c->need_full = false;
+        // lists, unless they were found not to hold some sphere's neighbours
+        const bool use = lists_pay(c) && c->list_rest == 0;
+        int rest = 0;
+        if (!use) {
+            // full-sort steps: one after a given-up step or an upload, DENSE_CHUNK
+            // of them while the scene is dense, before the changed-cell count is
+            // read again
+            rest = full ? (c->dense ? std::min(left, DENSE_CHUNK) : 1) : std::min(left, LIST_REST);
+            st = run(rest, full, LIST_NONE);
+            c->list_steps = 0;
         } else {
             int l = left;
-            if (c->p.use_graph) {
-                while (l >= 2) {
-                    st = run_graph_pair(c);
-                    if (st != SD_OK) return st;
-                    l -= 2;
-                }
+            if (full || c->list_steps < std::min(left, 2)) {
+                st = enqueue_step(c, nullptr, full, LIST_BUILD);
+                // (one that was too full for lists, or of unknown speed: a look first)
+                c->list_steps = c->crowded || c->last_move < 0.0f
+                                    ? 2
+                                    : list_life(0.0f, list_sigma(c->last_move, c->list_cell), c->last_move);
+                --l;
             }
-            for (; l > 0; --l) {
-                st = enqueue_step(c);
-                if (st != SD_OK) return st;
-            }
+            if (st == SD_OK) st = run(std::min(l, c->list_steps), false, LIST_USE);
         }
-        int ctl[2] = {0, 0};
-        SD_HIP(hipMemcpyAsync(ctl, c->step_ctl, sizeof ctl, hipMemcpyDeviceToHost, c->stream));
+        if (st != SD_OK) return st;
+        c->need_full = false;
+        StepCtl ctl;
+        SD_HIP(hipMemcpyAsync(&ctl, c->ctl, STEP_CTL_READ * sizeof(int), hipMemcpyDeviceToHost, c->stream));
         SD_HIP(hipStreamSynchronize(c->stream));
-        const int ran = ctl[1];
-        if (ran < 0 || ran > left || (ran == 0 && ctl[0] == 0))
+        const int ran = ctl.ran;
+        if (ran < 0 || ran > left || (ran == 0 && ctl.given_up == 0))
             return set_error(SD_ERR_STATE, "step: %d of %d steps ran", ran, left);
         c->cur_hist = h0 ^ (ran & 1);  // the roles of the steps that ran
         c->cur_state = s0 ^ (ran & 1);
         left -= ran;
-        if (ctl[0]) c->need_full = true;  // redo the given-up step with the full sort
+        c->last_ovf = ctl.overflow;
+        c->last_move = isfinite(ctl.last) ? ctl.last : 3.4e38f;
+        // the displacement of the last step is not in yet: count it as the one before
+        c->list_steps = ctl.given_up ? 0 : list_life(ctl.displaced + ctl.last, ctl.sigma, ctl.last);
+        if (ctl.given_up == GIVEN_UP_SORT) c->need_full = true;  // redo the given-up step with the full sort
+        if (use) {
+            c->crowded = ctl.over != 0;
+            if (c->crowded) {
+                c->list_steps = 0;
+                c->list_rest = 4 * LIST_REST;
+            }
+        } else {
+            c->list_rest = std::max(0, c->list_rest - ran);
+        }
         if (full) {  // still dense: the last full-sort step's changed cells exceed the re-sort's cap
             int m = 0;
             SD_HIP(hipMemcpyAsync(&m, c->mcount + c->cur_hist, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -533,9 +591,40 @@ sd_status check_spheres(const char* who, int n, const float* x, const float* y, 
 sd_status force_full_sort(sd_ctx* c) {
     c->need_full = true;
     c->dense = false;
-    sd_status st = launch_fill_u32((uint32_t*)c->step_ctl, 0u, 2, c->stream);
+    c->list_steps = 0;
+    c->list_rest = 0;
+    c->last_move = -1.0f;
+    // nothing run, no lists (displaced infinite), no displacements
+    sd_status st = launch_fill_u32((uint32_t*)c->ctl, 0u, sizeof(StepCtl) / 4, c->stream);
+    if (st == SD_OK) st = launch_fill_u32((uint32_t*)&c->ctl->displaced, 0x7f800000u, 1, c->stream);
     if (st != SD_OK) return st;
     return launch_fill_u32((uint32_t*)(c->mcount + c->cur_hist), 0x7fffffffu, 1, c->stream);
+}
+
+// The grid and radii that the near lists depend on: the largest radius of every
+// scene (r: radii in slot order, stride floats apart), no lists where a
+// diameter exceeds its cell (a loaded state's may).
+sd_status set_list_bounds(sd_ctx* c, const float* r, int stride) {
+    const int scenes = c->batch ? c->nscenes : 1;
+    std::vector<float> rm((size_t)scenes, 0.0f);
+    c->list_cell = 3.4e38f;
+    for (int k = 0; k < scenes; ++k) {
+        const size_t i0 = c->batch ? (size_t)c->scenes_h[k].first : 0;
+        const size_t m = c->batch ? (size_t)c->scenes_h[k].n : (size_t)c->n;
+        const float cell = c->batch ? c->scenes_h[k].g.cell : c->p.grid.cell;
+        for (size_t i = i0; i < i0 + m; ++i) rm[k] = r[i * stride] > rm[k] ? r[i * stride] : rm[k];
+        c->list_cell = std::min(c->list_cell, 2.0f * rm[k] <= cell ? cell : 0.0f);
+    }
+    c->rmax = rm[0];
+    if (c->batch) {
+        if (!c->scene_rmax) {
+            sd_status st = dalloc(&c->scene_rmax, (size_t)scenes);
+            if (st != SD_OK) return st;
+        }
+        SD_HIP(hipMemcpyAsync(c->scene_rmax, rm.data(), scenes * sizeof(float), hipMemcpyHostToDevice, c->stream));
+        SD_HIP(hipStreamSynchronize(c->stream));
+    }
+    return SD_OK;
 }
 
 // Allocates the device state for n spheres and uploads it (slot = particle id);
@@ -567,13 +656,17 @@ sd_status upload_state(sd_ctx* c, int n, const float* x, const float* y, const f
     ALLOC(c->hcount[1], n);
     ALLOC(c->hist[0], (size_t)maxc * n);
     ALLOC(c->hist[1], (size_t)maxc * n);
-    ALLOC(c->overflow, 1);
+    ALLOC(c->ctl, 1);
     ALLOC(c->mcount, 2);
     ALLOC(c->mnew, resort_cap(n));
     ALLOC(c->mold, resort_cap(n));
     ALLOC(c->msn, resort_cap(n));
     ALLOC(c->mso, resort_cap(n));
-    ALLOC(c->step_ctl, 2);
+    for (int k = 0; k < 2; ++k) {
+        ALLOC(c->lcount[k], n);
+        ALLOC(c->list[k], (size_t)LIST_CAP * n);
+    }
+    ALLOC(c->newpos, n);
     c->diag_blocks = div_up(n, DIAG_BLOCK) < 1024 ? div_up(n, DIAG_BLOCK) : 1024;
     ALLOC(c->diag, (size_t)c->diag_blocks * DIAG_VALUES);
 #undef ALLOC
@@ -598,7 +691,6 @@ sd_status upload_state(sd_ctx* c, int n, const float* x, const float* y, const f
     st = launch_fill_u32((uint32_t*)c->hcount[0], 0u, n, c->stream);
     if (st == SD_OK) st = launch_fill_u32((uint32_t*)c->hcount[1], 0u, n, c->stream);
     if (st == SD_OK) st = launch_fill_u32((uint32_t*)(c->posB + n), 0u, 4 * (size_t)CONTACT_POS_PAD, c->stream);
-    if (st == SD_OK) st = launch_fill_u32((uint32_t*)c->overflow, 0u, 1, c->stream);
     if (st != SD_OK) return st;
     c->cur_keys = 0;
     c->cur_hist = 0;
@@ -626,7 +718,8 @@ extern "C" sd_status sd_ctx_upload_spheres(sd_ctx* c, int n, const float* x, con
         return st;
     }
     const GridDev g = to_dev(c->p.grid);
-    st = launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], c->stream);
+    st = set_list_bounds(c, radius, 1);
+    if (st == SD_OK) st = launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], c->stream);
     if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(c->stream));
     return SD_OK;
@@ -735,7 +828,8 @@ extern "C" sd_status sd_batch_upload(sd_ctx* c, int nscenes, const sd_scene_desc
     c->n_straddle = (int)straddle.size();
     SD_HIP(hipMemcpyAsync(c->scenes_d, table.data(), nscenes * sizeof(SceneDev), hipMemcpyHostToDevice, c->stream));
     SD_HIP(hipMemcpyAsync(c->scene_of, sof.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    st = launch_hash_keys_batch(c->pos[0], (int)n, c->scenes_d, c->scene_of, c->k64[0], c->stream);
+    st = set_list_bounds(c, radius, 1);
+    if (st == SD_OK) st = launch_hash_keys_batch(c->pos[0], (int)n, c->scenes_d, c->scene_of, c->k64[0], c->stream);
     if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(c->stream));
     return SD_OK;
@@ -745,13 +839,12 @@ extern "C" sd_status sd_ctx_step(sd_ctx* c, int nsteps) {
     SD_REQUIRE(c, "sd_ctx_step: NULL context");
     SD_REQUIRE(nsteps >= 0, "sd_ctx_step: nsteps < 0");
     if (c->n == 0) return set_error(SD_ERR_STATE, "sd_ctx_step: no spheres uploaded");
-    sd_status st = launch_fill_u32((uint32_t*)c->overflow, 0u, 1, c->stream);
+    sd_status st = launch_fill_u32((uint32_t*)&c->ctl->overflow, 0u, 1, c->stream);
     if (st != SD_OK) return st;
+    c->last_ovf = 0;
     st = run_steps(c, nsteps);
     if (st != SD_OK) return st;
-    int ovf = 0;
-    SD_HIP(hipMemcpyAsync(&ovf, c->overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SD_HIP(hipStreamSynchronize(c->stream));
+    const int ovf = c->last_ovf;
     c->steps_done += nsteps;
     if (c->hulls) {
         hull_count_steps(c->hulls, nsteps);
@@ -785,8 +878,29 @@ extern "C" sd_status sd_ctx_profile(sd_ctx* c, int nsteps, float* stage_ms, int 
             full = m > resort_cap(c->n);
         }
         c->need_full = false;
-        st = enqueue_step(c, ev, full);
+        // near lists as a run would use them, the step redone if they ran out
+        const bool use = lists_pay(c);
+        const int lists = !use ? LIST_NONE : (full || c->list_steps < 1 || c->crowded ? LIST_BUILD : LIST_USE);
+        const int keys0 = c->cur_keys, hist0 = c->cur_hist, state0 = c->cur_state;
+        StepCtl ctl;
+        st = launch_fill_u32((uint32_t*)c->ctl, 0u, 2, c->stream);
+        if (st == SD_OK) st = enqueue_step(c, ev, full, lists);
         if (st != SD_OK) break;
+        if (hipMemcpyAsync(&ctl, c->ctl, STEP_CTL_READ * sizeof(int), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+            hipStreamSynchronize(c->stream) != hipSuccess) {
+            st = set_error(SD_ERR_HIP, "sd_ctx_profile: control read failed");
+            break;
+        }
+        c->last_move = isfinite(ctl.last) ? ctl.last : 3.4e38f;
+        c->crowded = use && ctl.over != 0;
+        c->list_steps = ctl.given_up ? 0 : list_life(ctl.displaced + ctl.last, ctl.sigma, ctl.last);
+        if (ctl.given_up == GIVEN_UP_LIST) {
+            c->cur_keys = keys0;
+            c->cur_hist = hist0;
+            c->cur_state = state0;
+            --i;
+            continue;
+        }
         hipError_t e = hipEventSynchronize(ev[4]);
         if (e != hipSuccess) {
             st = hip_error(e, "hipEventSynchronize", __FILE__, __LINE__);
@@ -877,7 +991,7 @@ sd_status snapshot_restore(sd_ctx* c, const Snapshot& sn) {
         if (sz[k]) SD_HIP(hipMemcpyAsync(b[k], sn.buf + sn.off[k], sz[k], hipMemcpyDeviceToDevice, c->stream));
     sd_status st = force_full_sort(c);
     if (st != SD_OK) return st;
-    return launch_fill_u32((uint32_t*)c->overflow, 0u, 1, c->stream);
+    return launch_fill_u32((uint32_t*)&c->ctl->overflow, 0u, 1, c->stream);
 }
 
 }  // namespace
@@ -1119,7 +1233,8 @@ sd_status write_rows(sd_ctx* c, const HostRows& r) {
     SD_HIP(hipMemcpyAsync(c->hcount[0], r.hcount.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, s));
     SD_HIP(hipMemcpyAsync(c->hist[0], r.hist.data(), maxc * n * sizeof(float4), hipMemcpyHostToDevice, s));
     const GridDev g = to_dev(c->p.grid);
-    st = launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], s);
+    st = set_list_bounds(c, rad.data(), 1);
+    if (st == SD_OK) st = launch_hash_keys_u64(c->pos[0], n, g, c->k64[0], s);
     if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(s));
     c->steps_done = steps;
@@ -1289,7 +1404,18 @@ extern "C" sd_status sd_ctx_load(sd_ctx* c, const void* buffer, size_t bytes) {
     SD_REQUIRE(h.nscenes == c->nscenes && h.layout_hash == layout_hash(c),
                "sd_ctx_load: state was saved from a context with a different scene table or grid");
     const size_t n = (size_t)c->n;
+    sd_status st0;
+    const float cell0 = c->list_cell, rmax0 = c->rmax;
     const char* b = (const char*)buffer + sizeof h;
+    if ((uintptr_t)b % alignof(float)) {  // (rows of an unaligned buffer)
+        std::vector<float4> rows(n);
+        memcpy(rows.data(), b, n * sizeof(float4));
+        st0 = set_list_bounds(c, &rows[0].w, 4);
+    } else {
+        st0 = set_list_bounds(c, (const float*)b + 3, 4);
+    }
+    if (st0 != SD_OK) return st0;
+    if (c->list_cell != cell0 || c->rmax != rmax0) drop_graphs(c);  // captured with the previous bounds
     c->cur_keys = 0;
     c->cur_hist = 0;
     c->cur_state = 0;

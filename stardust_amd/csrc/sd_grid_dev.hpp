@@ -55,16 +55,42 @@ __device__ __forceinline__ void row_range(const GridDev& g, const int* __restric
     if (hi == 0) lo = 0;
 }
 
-// Sorted-position window of cells (cx-1 .. cx+1, y, z) from the cell starts
+// Sorted-position window of cells (cx-e .. cx+e, y, z) from the cell starts
 // (every cell has one, empty or not): [start of the first cell, start of the
 // cell after the last). Empty window: lo == hi.
-__device__ __forceinline__ void row_window(const GridDev& g, const int* __restrict__ start, int cx, int y, int z,
-                                           int& lo, int& hi) {
+__device__ __forceinline__ void row_window(const GridDev& g, const int* __restrict__ start, int cx, int e, int y,
+                                           int z, int& lo, int& hi) {
     const int base = (z * g.ny + y) * g.nx;
-    const int xa = cx > 0 ? cx - 1 : cx;
-    const int xe = cx < g.nx - 1 ? cx + 2 : cx + 1;
+    const int xa = max(cx - e, 0);
+    const int xe = min(cx + e + 1, g.nx);
     lo = start[(size_t)(base + xa)];
     hi = start[(size_t)(base + xe)];
+}
+
+// By the first wave of one block, once per step, before the contact kernel.
+// cell: the smallest cell edge of the context's grids. A step that was to use
+// lists that have run out is given up, and nothing else is changed.
+__device__ __forceinline__ void list_begin_step(StepCtl* L, int lists, float cell) {
+    uint32_t u = L->dmax[(threadIdx.x & 63) * 16];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        const uint32_t o = __shfl_xor(u, d);
+        u = o > u ? o : u;
+    }
+    const float m = sqrtf(__uint_as_float(u)) * 1.00001f;
+    const float D = L->displaced + m;  // (not a number: the lists have run out)
+    if (lists == LIST_USE && (!(2.0f * D <= 0.98f * L->sigma) || L->over)) {
+        if ((threadIdx.x & 63) == 0) L->given_up = GIVEN_UP_LIST;
+        return;
+    }
+    L->dmax[(threadIdx.x & 63) * 16] = 0u;
+    if ((threadIdx.x & 63) != 0) return;
+    L->last = m;
+    L->displaced = lists == LIST_USE ? D : (lists == LIST_BUILD ? 0.0f : __builtin_inff());
+    if (lists == LIST_BUILD) {
+        L->over = 0;
+        L->sigma = fminf(fmaxf(LIST_LIFE * m, LIST_MIN * cell), LIST_MAX * cell);
+    }
 }
 
 }  // namespace sd

@@ -2,6 +2,8 @@
 // libstardust_hip.so (not part of the C ABI).
 #pragma once
 
+#include <math.h>
+
 #include "sd_common.hpp"
 
 namespace sd {
@@ -51,6 +53,7 @@ sd_status launch_fill_u32(uint32_t* dst, uint32_t value, size_t count, hipStream
 sd_status launch_copy_u32(uint32_t* dst, const uint32_t* src, size_t count, hipStream_t s);
 sd_status launch_hash_keys_u64(const float4* pos4, int n, const GridDev& g, uint64_t* keys, hipStream_t s);
 struct SceneDev;
+struct StepCtl;
 // keys[i] = (scene cbase + cell of pos4[i] in the scene grid) << 32 | i
 sd_status launch_hash_keys_batch(const float4* pos4, int n, const SceneDev* scenes, const int* scene_of,
                                  uint64_t* keys, hipStream_t s);
@@ -58,10 +61,12 @@ sd_status launch_cell_ranges_u32(const uint32_t* keys, int n, int n_cells, int* 
 sd_status launch_cell_ranges_u64(const uint64_t* keys, int n, int n_cells, int* ranges, hipStream_t s);
 // Cell starts of sorted keys: start[c] = number of keys whose cell is below c,
 // c = 0 .. n_cells (n_cells + 1 entries), every entry written. Also gathers pos
-// into sorted order (pos_o) with permute and sets *next_count = 0; does
+// into sorted order (pos_o) with permute, sets *next_count = 0 and
+// newpos[slot] = sorted position, and begins the step's near lists; does
 // nothing while *skip.
 sd_status launch_step_starts_u64(const uint64_t* keys, int n, int n_cells, int* start, const int* skip, bool permute,
-                                 const float4* pos, float4* pos_o, int* next_count, hipStream_t s);
+                                 const float4* pos, float4* pos_o, int* next_count, int* newpos, StepCtl* ctl,
+                                 int lists, float list_cell, hipStream_t s);
 // perm is either u32 values (perm32) or the low halves of u64 keys (perm64).
 sd_status launch_permute(const uint32_t* perm32, const uint64_t* perm64, int n, const float4* pos, const float4* vel,
                          const float4* omg, const int* ids, float4* pos_o, float4* vel_o, float4* omg_o, int* ids_o,
@@ -82,6 +87,44 @@ sd_status check_contact(const sd_contact_params* c);
 // contact kernel's batched candidate loads need no clamping.
 constexpr int CONTACT_POS_PAD = 4;
 
+// Near lists of a stepping context. A step that builds them records, for every
+// sphere, the spheres within reach of a contact plus a margin sigma; the steps
+// after it test only those, until the spheres may have used the margin up. The
+// bound is exact: displaced sums the largest displacement of any sphere per
+// step since the build (and grows by each step's before the next one), and a
+// pair outside the lists stays apart while 2 displaced < sigma. A step of a
+// dilute scene then reads a list entry per sphere or so instead of testing 97
+// candidates, one of a packing about 7.
+//
+// The host says what a step does: it builds lists, then runs as many steps on
+// them as the last displacement lets expect, in one launch sequence. A step
+// that was to use lists that have run out is given up on the device, as a
+// re-sort of too many changes is, and redone.
+constexpr int LIST_CAP = 24;  // entries per sphere; a scene with a fuller sphere searches in every step
+constexpr int LIST_SLOTS = 64;  // displacement maxima, a 64-byte line each: the waves' atomics spread over them
+enum { LIST_USE = 0, LIST_BUILD = 1, LIST_NONE = 2 };
+enum { GIVEN_UP_SORT = 1, GIVEN_UP_LIST = 2 };
+// State of a context's launch sequence that the host reads back (the first
+// eight words) and its kernels share.
+struct StepCtl {
+    int given_up;     // != 0: a step was given up, every later kernel of the sequence returns at once
+    int ran;          // steps that ran
+    int overflow;     // most contacts of a sphere beyond the history's capacity
+    int over;         // a sphere had more neighbours than its list holds when the lists were built
+    float displaced;  // infinite: no lists
+    float sigma;
+    float last;       // largest displacement of the step before the current one
+    int pad;
+    int pad2[8];
+    uint32_t dmax[LIST_SLOTS * 16];  // squared displacements of the current step (float bits), slot k at 16 k
+};
+constexpr int STEP_CTL_READ = 8;
+// The margin lasts for LIST_LIFE / 2 steps of the last step's largest
+// displacement, within [LIST_MIN, LIST_MAX] cells. 40 steps spread the cost of a
+// build (about twice a step without lists at most) and keep the lists short.
+constexpr float LIST_LIFE = 80.0f, LIST_MIN = 0.01f, LIST_MAX = 0.08f;
+inline float list_sigma(float last, float cell) { return fminf(fmaxf(LIST_LIFE * last, LIST_MIN * cell), LIST_MAX * cell); }
+
 // Fused step kernel modes. CONTACT_FUSED_BATCH: packed u64 keys, every sphere
 // takes its grid, contact law and cell-id base from its scene's SceneDev.
 enum { CONTACT_FORCES = 0, CONTACT_FUSED_U64 = 1, CONTACT_FUSED_BATCH = 2 };
@@ -99,7 +142,8 @@ struct SceneDev {
 };
 
 struct ContactArgs {
-    const float4* pos;  // sorted state
+    const float4* pos;  // sorted state; positions only where a sphere searches (fused modes)
+    const float4* pos_rows;  // fused modes: positions in the previous order, as vel, omg and ids
     const float4* vel;
     const float4* omg;
     const int* ids;
@@ -131,9 +175,7 @@ struct ContactArgs {
     uint64_t* mnew;
     uint64_t* mold;
     int mcap;
-    // nullable: [0] != 0 -> the step was given up, return at once; [1] counts
-    // the steps that ran
-    int* step_ctl;
+    StepCtl* ctl;  // fused modes
     // CONTACT_FUSED_BATCH: scene table and scene of every slot
     const SceneDev* scenes;
     const int* scene_of;
@@ -143,6 +185,18 @@ struct ContactArgs {
     // registers); launch_contacts_straddle runs them with per-lane parameters.
     const int* straddle;
     int n_straddle;
+    // fused modes: near lists (entry k of slot s at k * n + s; the old ones in
+    // the previous step's order, with newpos[old position] = position), what
+    // the step does with them (LIST_*), and the largest radius (per scene in
+    // batch mode)
+    int lists;
+    const uint8_t* lcount_old;
+    const int* list_old;
+    uint8_t* lcount_new;
+    int* list_new;
+    const int* newpos;
+    float rmax;
+    const float* scene_rmax;
 };
 sd_status launch_contacts(int mode, const ContactArgs& a, hipStream_t s, int block);
 // Persistent form of the fused u64 / batch step kernel (same results): a
@@ -176,7 +230,7 @@ sd_status launch_morton(const float* lo4, const float* hi4, int n, const float* 
 sd_status launch_resort_u64(const int* mcount, int cap, const uint64_t* mnew, const uint64_t* mold, uint64_t* msorted_new,
                             uint64_t* msorted_old, const uint64_t* keys, int n, int* cell_start, int n_cells,
                             const float4* pos_state, float4* posB, uint64_t* keys_out, int* next_count,
-                            int* step_ctl, hipStream_t s);
+                            StepCtl* ctl, int* newpos, int lists, float list_cell, hipStream_t s);
 sd_status launch_integrate(float4* pos, float4* vel, float4* omg, const float4* f, const float4* t, int n,
                            const ContactDev& c, hipStream_t s);
 

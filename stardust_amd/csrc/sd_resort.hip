@@ -15,7 +15,7 @@
 //              the first read off the previous step's cell starts.
 // The result is the same array a stable radix sort of the keys produces, and
 // the positions are permuted into that order in the same pass. With more than
-// resort_cap(n) changes the step is given up: step_ctl[0] is set, every later
+// resort_cap(n) changes the step is given up: StepCtl::given_up is set, every later
 // kernel of the launch sequence returns at once (the state is untouched), and
 // the host redoes that step with the full radix sort.
 //
@@ -33,8 +33,8 @@ constexpr int RANK_MOVERS = 64;  // movers ranked by one block
 constexpr int RANK_BLOCK = 256;  // four waves share the comparisons of 64 movers
 constexpr int MERGE_SLICE = 1024;  // new keys of one merge block held in LDS
 
-// Ranks the movers' new and old keys by counting (keys are distinct) and places
-// every mover, 64 movers a block. Counting is M^2 comparisons, so it is spread
+// Begins the step's near lists, ranks the movers' new and old keys by counting
+// (keys are distinct) and places every mover, 64 movers a block. Counting is M^2 comparisons, so it is spread
 // over M / 64 blocks; what remains is the latency of dependent loads that miss
 // the cache after the contact kernel (count, keys, cell starts, positions). In
 // a 128-scene batch of 1.83M spheres with 900 movers a step one block for all
@@ -43,13 +43,14 @@ __global__ __launch_bounds__(RANK_BLOCK) void k_resort_movers(
     const int* __restrict__ mcount, int cap, const uint64_t* __restrict__ mnew, const uint64_t* __restrict__ mold,
     uint64_t* __restrict__ msn, uint64_t* __restrict__ mso, int n, const int* __restrict__ cell_start,
     const float4* __restrict__ pos_state, float4* __restrict__ posB, uint64_t* __restrict__ keys_out,
-    int* __restrict__ step_ctl) {
-    const int given_up = step_ctl[0], M = *mcount;
+    StepCtl* __restrict__ ctl, int* __restrict__ newpos, int lists, float list_cell) {
+    const int given_up = ctl->given_up, M = *mcount;
     if (given_up) return;  // an earlier step of this launch sequence was given up
     if (M > cap) {  // too many changes: this step is given up (the host redoes it with the full sort)
-        if (blockIdx.x == 0 && threadIdx.x == 0) step_ctl[0] = 1;
+        if (blockIdx.x == 0 && threadIdx.x == 0) ctl->given_up = GIVEN_UP_SORT;
         return;
     }
+    if (blockIdx.x == 0 && threadIdx.x < 64) list_begin_step(ctl, lists, list_cell);
     const int first = blockIdx.x * RANK_MOVERS;
     if (first >= M) return;
     __shared__ uint64_t tn[RANK_BLOCK], to[RANK_BLOCK];
@@ -97,7 +98,8 @@ __global__ __launch_bounds__(RANK_BLOCK) void k_resort_movers(
     const int dest = all_less - old_less + rn;
     if (dest >= 0 && dest < n && (uint32_t)x < (uint32_t)n) {  // (always, for consistent keys)
         keys_out[dest] = x;
-        posB[dest] = px;
+        if (lists != LIST_USE) posB[dest] = px;
+        else newpos[(uint32_t)x] = dest;
     }
 }
 
@@ -136,7 +138,8 @@ __device__ __forceinline__ int wave_lower_bound(const uint64_t* __restrict__ a, 
 // movers' new keys below c << 32 minus their old keys below c << 32. Each
 // block updates cells_per_block consecutive cells; a run of cells that holds no
 // mover key has one change for all its cells (most runs: none). Sets
-// *next_count = 0 for the next step's movers.
+// *next_count = 0 for the next step's movers, newpos (old position to new, as
+// k_resort_movers does for the movers).
 //
 // A block's positions and cells meet few movers: each wave finds one bound of
 // them in the sorted lists, and only that slice is held in LDS (all the movers'
@@ -145,9 +148,12 @@ __global__ __launch_bounds__(RESORT_MERGE_BLOCK) void k_resort_merge(
     const int* __restrict__ mcount, int cap, const uint64_t* __restrict__ msn, const uint64_t* __restrict__ mso,
     const uint64_t* __restrict__ keys, int n, const float4* __restrict__ pos_state, float4* __restrict__ posB,
     uint64_t* __restrict__ keys_out, int* __restrict__ cell_start, int n_cells, int cells_per_block,
-    int* __restrict__ next_count, const int* __restrict__ step_ctl) {
-    const int given_up = step_ctl[0], M = *mcount;
+    int* __restrict__ next_count, const StepCtl* __restrict__ ctl, int* __restrict__ newpos, int lists) {
+    const int given_up = ctl->given_up, M = *mcount;
     if (given_up || M > cap) return;
+    // a step on lists needs no sorted positions, the others no places of the
+    // previous order
+    const bool use = lists == LIST_USE, sorted = !use;
     // this thread's key and position, loaded first: their latency overlaps the
     // searches below
     const int s0 = blockIdx.x * RESORT_MERGE_BLOCK;
@@ -156,7 +162,7 @@ __global__ __launch_bounds__(RESORT_MERGE_BLOCK) void k_resort_merge(
     float4 ps = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (s < n) {
         y = keys[s];
-        ps = pos_state[s];
+        if (sorted) ps = pos_state[s];
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) *next_count = 0;
     int d = s;
@@ -234,22 +240,25 @@ __global__ __launch_bounds__(RESORT_MERGE_BLOCK) void k_resort_merge(
     }
     if (s >= n || d < 0 || d >= n) return;  // (d is inside for consistent keys)
     keys_out[d] = y;
-    posB[d] = ps;
+    if (sorted) posB[d] = ps;
+    if (use) newpos[s] = d;
 }
 
 sd_status launch_resort_u64(const int* mcount, int cap, const uint64_t* mnew, const uint64_t* mold,
                             uint64_t* msorted_new, uint64_t* msorted_old, const uint64_t* keys, int n,
                             int* cell_start, int n_cells, const float4* pos_state, float4* posB, uint64_t* keys_out,
-                            int* next_count, int* step_ctl, hipStream_t s) {
+                            int* next_count, StepCtl* ctl, int* newpos, int lists, float list_cell,
+                            hipStream_t s) {
     if (n <= 0) return SD_OK;
     hipLaunchKernelGGL(k_resort_movers, dim3(div_up(cap, RANK_MOVERS)), dim3(RANK_BLOCK), 0, s, mcount, cap, mnew,
-                       mold, msorted_new, msorted_old, n, (const int*)cell_start, pos_state, posB, keys_out, step_ctl);
+                       mold, msorted_new, msorted_old, n, (const int*)cell_start, pos_state, posB, keys_out, ctl,
+                       newpos, lists, list_cell);
     SD_LAUNCH_CHECK();
     const int nblocks = div_up(n, RESORT_MERGE_BLOCK);
     const int cells_per_block = div_up(div_up(n_cells, nblocks), RESORT_MERGE_BLOCK) * RESORT_MERGE_BLOCK;
     hipLaunchKernelGGL(k_resort_merge, dim3(nblocks), dim3(RESORT_MERGE_BLOCK), 0, s, mcount, cap,
                        (const uint64_t*)msorted_new, (const uint64_t*)msorted_old, keys, n, pos_state, posB, keys_out,
-                       cell_start, n_cells, cells_per_block, next_count, (const int*)step_ctl);
+                       cell_start, n_cells, cells_per_block, next_count, (const StepCtl*)ctl, newpos, lists);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }
