@@ -517,9 +517,10 @@ sd_status sd_clump_upload(sd_clump_ctx* ctx, int nb, const float* pos4, const fl
                           const float* angvel4, const float* inertia6, const int* first, const int* count, int ns,
                           const float* local4);
 sd_status sd_clump_step(sd_clump_ctx* ctx, int nsteps);
-/* Stage times (ms, summed over nsteps eager steps): [0] prep + pose + body AABBs,
- * [1] domain + Morton + sort, [2] LBVH build, [3] and [4] empty (kept for the
- * layout), [5] partner search in the tree + contacts + integration. */
+/* Stage times (ms, summed over nsteps eager steps): [0] poses + body AABBs,
+ * [1] domain + Morton + sort, [2] LBVH build (both empty in a step on partner
+ * lists), [3] and [4] empty (kept for the layout), [5] partners + contacts +
+ * integration. */
 sd_status sd_clump_profile(sd_clump_ctx* ctx, int nsteps, float* stage_ms, int nstages);
 sd_status sd_clump_download(sd_clump_ctx* ctx, float* pos4, float* vel4, float* quat4, float* angmom4);
 /* Unique candidate body pairs (a < b, AABBs overlap) of the last step's tree,

@@ -46,7 +46,8 @@ def contact_c3():
 
 
 class ClumpScene:
-    # stage times of sd_clump_profile; [3] and [4] are empty (the partner search
+    # stage times of sd_clump_profile (morton_sort and lbvh_build are empty in a step
+    # on partner lists); [3] and [4] are empty (the partner search
     # runs inside the contact kernel)
     STAGES = ("pose", "morton_sort", "lbvh_build", None, None, "partners_contacts")
 

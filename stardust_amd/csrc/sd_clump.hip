@@ -10,13 +10,15 @@
 // explicit 1/m = 0 instead of mass >= 10 (Q13), and each body gathers the forces
 // of its contacts instead of racing scatters (Q7).
 //
-// Per step: body prep (world angular velocity), sphere pose, body AABBs, global
-// domain, Morton keys, radix sort, LBVH build, then one kernel per body finds
-// its partners in the tree and sums its sphere-sphere contacts (partners
-// ascending, own spheres ascending, partner spheres ascending) and integrates
-// it. Every launch has a fixed size, so steps are captured into a hipGraph per
-// buffer parity and replayed; the candidate pair list (unique a < b) is built
-// from the last step's tree only when asked for (sd_clump_pairs).
+// Per step: poses (world angular velocity, sphere positions, body boxes), then
+// one kernel per body takes its partners, sums its sphere-sphere contacts
+// (partners ascending, own spheres ascending, partner spheres ascending) and
+// integrates it. Partners come from a list that a step every few tens builds
+// (ClumpCtl below), or, for bodies too fast or crowded for lists, from a tree
+// that every step builds: global domain, Morton keys, radix sort, LBVH build.
+// Every launch has a fixed size, so steps are captured into hipGraphs and
+// replayed; the candidate pair list (unique a < b) of the last step's boxes is
+// built only when asked for (sd_clump_pairs).
 //
 // Integration of a body with 1/m > 0 (FP32, fixed operation order):
 //   v += (F/m + g) dt;  x += v dt;  L += T dt
@@ -54,57 +56,144 @@ struct ClumpState {
     const float4* angm;  // (Lx, Ly, Lz, 0)
 };
 
-__global__ void k_body_prep(ClumpState st, const float4* __restrict__ i0, const float4* __restrict__ i1, int nb,
-                            float4* __restrict__ omega) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    const Rot R = quat_rot(st.quat[b]);
-    const float4 L = st.angm[b];
-    const V3 w = inv_inertia_apply(R, i0[b], i1[b], v3(L.x, L.y, L.z));
-    omega[b] = make_float4(w.x, w.y, w.z, 0.0f);
+// Partner lists of a clump context, as the near lists of the sphere contexts: a
+// step that builds them inflates the body boxes by a margin, and the steps
+// after it take a body's partners from the listed ones whose boxes overlap,
+// instead of building and walking a tree. displaced sums the largest movement
+// of a box face per step since the build; a pair outside the lists has boxes
+// apart while that is below limit (the margin, less what rounding can take). A
+// step whose lists have run out is given up and redone with a build.
+constexpr int CL_LIST = 16;  // partners listed per body
+struct ClumpCtl {
+    int given_up;        // != 0: every later kernel of the launch sequence returns at once
+    int ran;             // steps that ran
+    int error;           // malformed tree
+    int over;            // a body had more partners than its list holds
+    float displaced[2];  // by buffer parity of the step (written for the next one)
+    float limit;
+    float last;          // movement of the last step
+    float margin;
+    int pad[7];
+    uint32_t dmax[2][LIST_SLOTS * 16];  // by parity: face movements of the step (float bits)
+};
+constexpr int CLUMP_CTL_READ = 9;
+// The margin lasts 40 steps of the last movement, within these shares of the
+// mean body size.
+constexpr float CL_MARGIN_STEPS = 40.0f, CL_MARGIN_MIN = 0.005f, CL_MARGIN_MAX = 0.05f;
+inline float clump_margin(float last, float size) {
+    return fminf(fmaxf(CL_MARGIN_STEPS * last, CL_MARGIN_MIN * size), CL_MARGIN_MAX * size);
 }
 
-__global__ void k_clump_pose(ClumpState st, const float4* __restrict__ omega, const float4* __restrict__ slocal,
-                             const int* __restrict__ sbody, int ns, float4* __restrict__ sx,
-                             float4* __restrict__ sv) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= ns) return;
-    const int b = sbody[s];
-    const Rot R = quat_rot(st.quat[b]);
-    const float4 l = slocal[s];
-    const V3 r = rot_mul(R, v3(l.x, l.y, l.z));
-    const float4 X = st.pos[b], V = st.vel[b], w = omega[b];
-    sx[s] = make_float4(X.x + r.x, X.y + r.y, X.z + r.z, l.w);
-    sv[s] = make_float4(V.x + (w.y * r.z - w.z * r.y), V.y + (w.z * r.x - w.x * r.z), V.z + (w.x * r.y - w.y * r.x),
-                        0.0f);
+// Largest face movement of the step, by a whole wave.
+__device__ __forceinline__ float step_movement(const uint32_t* dmax) {
+    uint32_t u = dmax[lane_id() * 16];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        const uint32_t o = __shfl_xor(u, d);
+        u = o > u ? o : u;
+    }
+    return __uint_as_float(u) * 1.00001f;
 }
 
-__global__ void k_body_aabb(const float4* __restrict__ sx, const int* __restrict__ bfirst,
-                            const int* __restrict__ bcount, int nb, float4* __restrict__ lo4,
-                            float4* __restrict__ hi4) {
+// A build's margin and limit (domain: of the boxes), the lists' displacement 0.
+__global__ __launch_bounds__(64) void k_clump_margin(ClumpCtl* __restrict__ ctl, int par, float size,
+                                                     const float* __restrict__ domain) {
+    if (ctl->given_up) return;
+    const float m = step_movement(ctl->dmax[par]);
+    if (threadIdx.x != 0) return;
+    float far = 0.0f;
+    for (int k = 0; k < 6; ++k) far = fmaxf(far, fabsf(domain[k]));
+    const float margin = fminf(fmaxf(CL_MARGIN_STEPS * m, CL_MARGIN_MIN * size), CL_MARGIN_MAX * size);
+    ctl->margin = margin;
+    ctl->limit = 0.98f * margin - 5e-7f * (far + margin);
+    ctl->over = 0;
+}
+
+__global__ void k_clump_inflate(const float4* __restrict__ lo, const float4* __restrict__ hi, int nb,
+                                const ClumpCtl* __restrict__ ctl, float4* __restrict__ ilo,
+                                float4* __restrict__ ihi) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
+    if (b >= nb || ctl->given_up) return;
+    const float m = ctl->margin;
+    const float4 l = lo[b], h = hi[b];
+    ilo[b] = make_float4(l.x - m, l.y - m, l.z - m, 0.0f);
+    ihi[b] = make_float4(h.x + m, h.y + m, h.z + m, 0.0f);
+}
+
+// Angular velocity and box of every body, world positions of its spheres, how
+// far the box's faces moved since the step before. Bound by the rows it reads
+// and writes (36 bytes a sphere, 150 a body: 134 MB at 262,144 bodies of 10
+// spheres); POSE_LANES lanes share a body, so that its spheres are read and
+// written in runs. Three passes, with the velocity of every sphere written too,
+// took 41 us, this one 22.
+constexpr int POSE_LANES = 4;
+__global__ __launch_bounds__(256) void k_clump_pose(
+    ClumpState st, const float4* __restrict__ i0, const float4* __restrict__ i1, const float4* __restrict__ slocal,
+    const int* __restrict__ bfirst, const int* __restrict__ bcount, int nb, float4* __restrict__ omega,
+    float4* __restrict__ sx, float4* __restrict__ lo4, float4* __restrict__ hi4, ClumpCtl* __restrict__ ctl, int par,
+    int track) {
+    if (ctl->given_up) return;
+    const int at = blockIdx.x * (256 / POSE_LANES) + threadIdx.x / POSE_LANES, sub = threadIdx.x % POSE_LANES;
+    const bool mine = at < nb;
+    const int b = min(at, nb - 1);  // (past the end: the last body again, nothing written or counted)
+    const int k0 = bfirst[b], kn = bcount[b];
+    const float4 X = st.pos[b], L = st.angm[b];
+    const Rot R = quat_rot(st.quat[b]);
     float lx = 3.402823466e38f, ly = 3.402823466e38f, lz = 3.402823466e38f;
     float hx = -3.402823466e38f, hy = -3.402823466e38f, hz = -3.402823466e38f;
-    const int k0 = bfirst[b], kn = bcount[b];
-    // 8 spheres per step with their loads in flight; indices past the last
+    // 4 spheres a lane with their loads in flight; indices past the last
     // sphere repeat it (min and max do not change)
-    for (int k = 0; k < kn; k += 8) {
-        float4 p[8];
+    for (int k = sub; k < kn; k += 4 * POSE_LANES) {
+        float4 l[4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p[j] = sx[k0 + min(k + j, kn - 1)];
+        for (int j = 0; j < 4; ++j) l[j] = slocal[k0 + min(k + j * POSE_LANES, kn - 1)];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            lx = fminf(lx, p[j].x - p[j].w);
-            ly = fminf(ly, p[j].y - p[j].w);
-            lz = fminf(lz, p[j].z - p[j].w);
-            hx = fmaxf(hx, p[j].x + p[j].w);
-            hy = fmaxf(hy, p[j].y + p[j].w);
-            hz = fmaxf(hz, p[j].z + p[j].w);
+        for (int j = 0; j < 4; ++j) {
+            const V3 r = rot_mul(R, v3(l[j].x, l[j].y, l[j].z));
+            const float4 x = make_float4(X.x + r.x, X.y + r.y, X.z + r.z, l[j].w);
+            lx = fminf(lx, x.x - x.w);
+            ly = fminf(ly, x.y - x.w);
+            lz = fminf(lz, x.z - x.w);
+            hx = fmaxf(hx, x.x + x.w);
+            hy = fmaxf(hy, x.y + x.w);
+            hz = fmaxf(hz, x.z + x.w);
+            if (mine && k + j * POSE_LANES < kn) sx[k0 + k + j * POSE_LANES] = x;
         }
     }
+#pragma unroll
+    for (int d = 1; d < POSE_LANES; d <<= 1) {
+        lx = fminf(lx, __shfl_xor(lx, d));
+        ly = fminf(ly, __shfl_xor(ly, d));
+        lz = fminf(lz, __shfl_xor(lz, d));
+        hx = fmaxf(hx, __shfl_xor(hx, d));
+        hy = fmaxf(hy, __shfl_xor(hy, d));
+        hz = fmaxf(hz, __shfl_xor(hz, d));
+    }
+    if (track) {
+        const float4 l = lo4[b], h = hi4[b];
+        const float a0 = fabsf(lx - l.x), a1 = fabsf(ly - l.y), a2 = fabsf(lz - l.z);
+        const float a3 = fabsf(hx - h.x), a4 = fabsf(hy - h.y), a5 = fabsf(hz - h.z);
+        const float sum = ((a0 + a1) + (a2 + a3)) + (a4 + a5);
+        const float m = sum < 3.4e38f ? fmaxf(fmaxf(fmaxf(a0, a1), fmaxf(a2, a3)), fmaxf(a4, a5)) : __builtin_inff();
+        uint32_t u = mine ? __float_as_uint(m) : 0u;
+#pragma unroll
+        for (int d = POSE_LANES; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_xor(u, d);
+            u = o > u ? o : u;
+        }
+        if (lane_id() == 0) atomicMax(&ctl->dmax[par][((blockIdx.x * 4u + (threadIdx.x >> 6)) & 63u) * 16u], u);
+    }
+    if (!mine || sub != 0) return;
+    const V3 w = inv_inertia_apply(R, i0[b], i1[b], v3(L.x, L.y, L.z));
+    omega[b] = make_float4(w.x, w.y, w.z, 0.0f);
     lo4[b] = make_float4(lx, ly, lz, 0.0f);
     hi4[b] = make_float4(hx, hy, hz, 0.0f);
+}
+
+// Velocity of the point at l (body frame) of a body.
+__device__ __forceinline__ V3 sphere_velocity(float4 quat, float4 V, float4 w, float4 l) {
+    const V3 r = rot_mul(quat_rot(quat), v3(l.x, l.y, l.z));
+    return v3(V.x + (w.y * r.z - w.z * r.y), V.y + (w.z * r.x - w.x * r.z), V.z + (w.x * r.y - w.y * r.x));
 }
 
 constexpr int CL_BLOCK = 128;
@@ -116,22 +205,51 @@ __device__ __forceinline__ bool cl_overlap(float4 al, float4 ah, float4 bl, floa
     return al.x <= bh.x && bl.x <= ah.x && al.y <= bh.y && bl.y <= ah.y && al.z <= bh.z && bl.z <= ah.z;
 }
 
-// One body per thread: its partners from the LBVH (every body whose AABB
-// overlaps its own), visited in ascending body id, then integration. A pass
-// walks the tree (stackless, ropes) and keeps the CL_PCAP smallest partner ids
-// above the last pass's largest, sorted in LDS; a body with more partners takes
-// more passes. The walk's bound turns a malformed tree into an error flag.
-template <bool INTEGRATE>
+// One body per thread: its partners (every body whose AABB overlaps its own),
+// visited in ascending body id, then integration. LIST_USE takes them from the
+// body's list. Otherwise a pass walks the tree (stackless, ropes) and keeps the
+// CL_PCAP smallest partner ids above the last pass's largest, sorted in LDS; a
+// body with more partners takes more passes. The walk's bound turns a malformed
+// tree into an error flag. LIST_BUILD: the tree is one of inflated boxes, and
+// what the walk finds is listed.
+//
+// Bound by the latency of dependent loads: a node a step of the walk, then
+// batches of 4 spheres. 262,144 bodies of 10 spheres: 169 us where every sphere
+// of a body is tested against every one of a partner; 162 with the lists alone;
+// 46 with the lists and the spheres beyond the partner's box left out (119 for
+// the step that builds them). Batches of 8 (157 registers) took 51. The lists
+// also save the step the keys, sort and tree (116 us).
+template <int LISTS>
 __global__ __launch_bounds__(CL_BLOCK) void k_clump_contacts(
     ClumpState st, ClumpState out, const float4* __restrict__ omega, const float4* __restrict__ i0,
-    const float4* __restrict__ i1, const float4* __restrict__ sx, const float4* __restrict__ sv,
+    const float4* __restrict__ i1, const float4* __restrict__ sx, const float4* __restrict__ slocal,
     const int* __restrict__ bfirst, const int* __restrict__ bcount, int nb, const float4* __restrict__ blo,
-    const float4* __restrict__ bhi, const float4* __restrict__ pnode, ContactDev c, int* __restrict__ error,
-    float4* __restrict__ force, float4* __restrict__ torque) {
-    __shared__ int plist[CL_BLOCK][CL_PCAP + 1];  // (+1: rows start in different banks)
+    const float4* __restrict__ bhi, const float4* __restrict__ pnode, ContactDev c, ClumpCtl* __restrict__ ctl,
+    int par, uint8_t* __restrict__ lcount, int* __restrict__ list) {
+    if (ctl->given_up) return;
+    {
+        const float m = step_movement(ctl->dmax[par]);
+        const float D = LISTS == LIST_USE ? (ctl->displaced[par] + m) * 1.0000002f  // (rounded up)
+                                          : (LISTS == LIST_BUILD ? 0.0f : __builtin_inff());
+        const bool out_of_margin = LISTS == LIST_USE && (!(D <= ctl->limit) || ctl->over);
+        if (blockIdx.x == 0 && threadIdx.x < 64) {
+            if (out_of_margin) {
+                // (every block sees the same: nothing else is written)
+                if (threadIdx.x == 0) ctl->given_up = GIVEN_UP_LIST;
+            } else {
+                ctl->dmax[1 - par][threadIdx.x * 16] = 0u;
+                if (threadIdx.x == 0) {
+                    ctl->displaced[1 - par] = D;
+                    ctl->last = m;
+                    ctl->ran += 1;
+                }
+            }
+        }
+        if (out_of_margin) return;
+    }
+    __shared__ int plist[LISTS == LIST_USE ? 1 : CL_BLOCK][CL_PCAP + 1];  // (+1: rows start in different banks)
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nb) return;
-    int* pl = plist[threadIdx.x];  // this body's partner list
     const float4 X = st.pos[b];
     const float4 wb4 = omega[b];
     const int f0 = bfirst[b], fn = bcount[b];
@@ -140,78 +258,131 @@ __global__ __launch_bounds__(CL_BLOCK) void k_clump_contacts(
     auto partner = [&](int p) {
         const float inv_mp = st.pos[p].w;
         if (X.w + inv_mp == 0.0f) return;  // two static bodies
-        const float4 wp4 = omega[p];
+        const float4 wp4 = omega[p], pl4 = blo[p], ph4 = bhi[p];
         const int g0 = bfirst[p], gn = bcount[p];
-        for (int i = f0; i < f0 + fn; ++i) {
-            const float4 xi = sx[i], vi = sv[i];
-            for (int j = g0; j < g0 + gn; ++j) {
-                const float4 xj = sx[j];
-                const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                const float d2 = dx * dx + dy * dy + dz * dz;
-                const float rs = xi.w + xj.w;
-                if (!(d2 < rs * rs) || d2 == 0.0f) continue;
-                const float4 vj = sv[j];
-                const float d = sqrtf(d2);
-                const float inv_d = 1.0f / d;
-                float hx = 0.0f, hy = 0.0f, hz = 0.0f;  // no tangential history for clumps
-                const PairForce f = contact_law(c, dx * inv_d, dy * inv_d, dz * inv_d, rs - d, xi.w, xj.w, X.w, inv_mp,
-                                                vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, wb4.x, wb4.y, wb4.z, wp4.x,
-                                                wp4.y, wp4.z, hx, hy, hz);
-                Fx = Fx + f.fx;
-                Fy = Fy + f.fy;
-                Fz = Fz + f.fz;
-                const float ax = xi.x - X.x, ay = xi.y - X.y, az = xi.z - X.z;
-                Tx = Tx + ((ay * f.fz - az * f.fy) + f.tx);
-                Ty = Ty + ((az * f.fx - ax * f.fz) + f.ty);
-                Tz = Tz + ((ax * f.fy - ay * f.fx) + f.tz);
+        // A sphere beyond the partner's box touches none of its spheres; the
+        // slack covers what rounding can take from the sums on both sides.
+        const float ex = 1e-6f * (fabsf(pl4.x) + fabsf(ph4.x)), ey = 1e-6f * (fabsf(pl4.y) + fabsf(ph4.y)),
+                    ez = 1e-6f * (fabsf(pl4.z) + fabsf(ph4.z));
+        auto beyond = [&](float x, float w, float lo, float hi, float e) {
+            const float s = e + 1e-6f * (fabsf(x) + w);
+            return (x - w) - hi > s || lo - (x + w) > s;
+        };
+        for (int ib = f0; ib < f0 + fn; ib += 4) {
+            uint32_t near = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float4 x = sx[min(ib + u, f0 + fn - 1)];
+                const bool out = beyond(x.x, x.w, pl4.x, ph4.x, ex) || beyond(x.y, x.w, pl4.y, ph4.y, ey) ||
+                                 beyond(x.z, x.w, pl4.z, ph4.z, ez);
+                if (!out && ib + u < f0 + fn) near |= 1u << u;
+            }
+            while (near) {
+                const int i = ib + __builtin_ctz(near);
+                near &= near - 1u;
+                const float4 xi = sx[i];
+                for (int jb = g0; jb < g0 + gn; jb += 4) {
+                    uint32_t hit = 0;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const float4 xj = sx[min(jb + u, g0 + gn - 1)];
+                        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+                        const float d2 = dx * dx + dy * dy + dz * dz;
+                        const float rs = xi.w + xj.w;
+                        if (d2 < rs * rs && d2 != 0.0f && jb + u < g0 + gn) hit |= 1u << u;
+                    }
+                    while (hit) {
+                        const int j = jb + __builtin_ctz(hit);
+                        hit &= hit - 1u;
+                        const float4 xj = sx[j];
+                        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+                        const float d = sqrtf(dx * dx + dy * dy + dz * dz);
+                        const float inv_d = 1.0f / d;
+                        const V3 vi = sphere_velocity(st.quat[b], st.vel[b], wb4, slocal[i]);
+                        const V3 vj = sphere_velocity(st.quat[p], st.vel[p], wp4, slocal[j]);
+                        float hx = 0.0f, hy = 0.0f, hz = 0.0f;  // no tangential history for clumps
+                        const PairForce f = contact_law(c, dx * inv_d, dy * inv_d, dz * inv_d, xi.w + xj.w - d, xi.w,
+                                                        xj.w, X.w, inv_mp, vi.x - vj.x, vi.y - vj.y, vi.z - vj.z,
+                                                        wb4.x, wb4.y, wb4.z, wp4.x, wp4.y, wp4.z, hx, hy, hz);
+                        Fx = Fx + f.fx;
+                        Fy = Fy + f.fy;
+                        Fz = Fz + f.fz;
+                        const float ax = xi.x - X.x, ay = xi.y - X.y, az = xi.z - X.z;
+                        Tx = Tx + ((ay * f.fz - az * f.fy) + f.tx);
+                        Ty = Ty + ((az * f.fx - ax * f.fz) + f.ty);
+                        Tz = Tz + ((ax * f.fy - ay * f.fx) + f.tz);
+                    }
+                }
             }
         }
     };
-    for (int lower = -1;;) {
-        int np = 0;
-        bool more = false;
-        int node = nb == 1 ? CL_SENTINEL : 0;
-        for (int guard = 0; node != CL_SENTINEL; ++guard) {
-            if (guard > 2 * nb + 2 || node < 0 || node >= 2 * nb - 1) {
-                atomicOr(error, 4);
-                break;
-            }
-            // one load step per node: box, the next node if the boxes
-            // overlap (left child, or a leaf's body), and the rope
-            const float4 nl = pnode[2 * (size_t)node], nh = pnode[2 * (size_t)node + 1];
-            if (!cl_overlap(ql, qh, nl, nh)) {
-                node = __float_as_int(nh.w);
-                continue;
-            }
-            if (node >= nb - 1) {  // a leaf: one body
-                const int p = __float_as_int(nl.w);
-                if (p != b && p > lower && p < nb) {
-                    if (np == CL_PCAP) more = true;  // partners beyond this pass's list
-                    if (np < CL_PCAP || p < pl[CL_PCAP - 1]) {
-                        int k = np < CL_PCAP ? np++ : CL_PCAP - 1;  // the largest drops out of a full list
-                        while (k > 0 && pl[k - 1] > p) {
-                            pl[k] = pl[k - 1];
-                            --k;
-                        }
-                        pl[k] = p;
-                    }
-                }
-                node = __float_as_int(nh.w);
-            } else {
-                node = __float_as_int(nl.w);
-            }
+    if constexpr (LISTS == LIST_USE) {
+        const int n = lcount[b];
+        for (int k = 0; k < n; ++k) {
+            const int p = list[(size_t)k * nb + b];
+            if (cl_overlap(ql, qh, blo[p], bhi[p])) partner(p);
         }
-        for (int e = 0; e < np; ++e) partner(pl[e]);
-        if (!more) break;
-        lower = pl[CL_PCAP - 1];
+    } else {
+        int* const pl = plist[threadIdx.x];  // this body's partners
+        float4 wl = ql, wh = qh;             // the box that walks
+        if (LISTS == LIST_BUILD) {
+            const float m = ctl->margin;
+            wl = make_float4(ql.x - m, ql.y - m, ql.z - m, 0.0f);
+            wh = make_float4(qh.x + m, qh.y + m, qh.z + m, 0.0f);
+        }
+        int listed = 0;
+        for (int lower = -1;;) {
+            int np = 0;
+            bool more = false;
+            int node = nb == 1 ? CL_SENTINEL : 0;
+            for (int guard = 0; node != CL_SENTINEL; ++guard) {
+                if (guard > 2 * nb + 2 || node < 0 || node >= 2 * nb - 1) {
+                    atomicOr(&ctl->error, 4);
+                    break;
+                }
+                // one load step per node: box, the next node if the boxes
+                // overlap (left child, or a leaf's body), and the rope
+                const float4 nl = pnode[2 * (size_t)node], nh = pnode[2 * (size_t)node + 1];
+                if (!cl_overlap(wl, wh, nl, nh)) {
+                    node = __float_as_int(nh.w);
+                    continue;
+                }
+                if (node >= nb - 1) {  // a leaf: one body
+                    const int p = __float_as_int(nl.w);
+                    if (p != b && p > lower && p < nb) {
+                        if (np == CL_PCAP) more = true;  // partners beyond this pass's list
+                        if (np < CL_PCAP || p < pl[CL_PCAP - 1]) {
+                            int k = np < CL_PCAP ? np++ : CL_PCAP - 1;  // the largest drops out of a full list
+                            while (k > 0 && pl[k - 1] > p) {
+                                pl[k] = pl[k - 1];
+                                --k;
+                            }
+                            pl[k] = p;
+                        }
+                    }
+                    node = __float_as_int(nh.w);
+                } else {
+                    node = __float_as_int(nl.w);
+                }
+            }
+            for (int e = 0; e < np; ++e) {
+                const int p = pl[e];
+                if (LISTS == LIST_BUILD) {
+                    if (listed < CL_LIST) list[(size_t)listed * nb + b] = p;
+                    ++listed;
+                    if (!cl_overlap(ql, qh, blo[p], bhi[p])) continue;
+                }
+                partner(p);
+            }
+            if (!more) break;
+            lower = pl[CL_PCAP - 1];
+        }
+        if (LISTS == LIST_BUILD) {
+            lcount[b] = (uint8_t)min(listed, CL_LIST);
+            if (listed > CL_LIST) ctl->over = 1;
+        }
     }
-    if (!INTEGRATE) {
-        force[b] = make_float4(Fx, Fy, Fz, 0.0f);
-        torque[b] = make_float4(Tx, Ty, Tz, 0.0f);
-        return;
-    }
-    float4 V = st.vel[b], q = st.quat[b], L = st.angm[b];
-    float4 P = X;
+    float4 P = X, V = st.vel[b], q = st.quat[b], L = st.angm[b];
     integrate_body(P, V, q, L, i0[b], i1[b], Fx, Fy, Fz, Tx, Ty, Tz, c);
     ((float4*)out.pos)[b] = P;
     ((float4*)out.vel)[b] = V;
@@ -308,8 +479,8 @@ struct sd_clump_ctx {
     float4 *pos[2] = {}, *vel[2] = {}, *quat[2] = {}, *angm[2] = {};
     int cur = 0;
     float4 *i0 = nullptr, *i1 = nullptr, *omega = nullptr;
-    int *bfirst = nullptr, *bcount = nullptr, *sbody = nullptr;
-    float4 *slocal = nullptr, *sx = nullptr, *sv = nullptr;
+    int *bfirst = nullptr, *bcount = nullptr;
+    float4 *slocal = nullptr, *sx = nullptr;
     float4 *blo = nullptr, *bhi = nullptr;
     float* domain = nullptr;
     float* dom_scratch = nullptr;
@@ -319,17 +490,27 @@ struct sd_clump_ctx {
     int *left = nullptr, *right = nullptr, *parent = nullptr, *first = nullptr, *last = nullptr, *rope = nullptr;
     float4 *nlo = nullptr, *nhi = nullptr;
     float4* pnode = nullptr;  // 2 per node: the walk's packed tree
-    int *counters = nullptr, *error = nullptr;
+    int* counters = nullptr;
     void* q_scratch = nullptr;
     size_t q_scratch_bytes = 0;
     int* pairs = nullptr;
     int pair_cap = 0;
     int npairs = 0;
     const uint64_t* ksorted = nullptr;  // sorted Morton keys of the last step's tree
-    bool have_tree = false;
-    hipGraphExec_t graph[2] = {nullptr, nullptr};  // two steps from buffer parity 0 / 1
-    hipGraph_t graph_obj[2] = {nullptr, nullptr};
-    float4 *force = nullptr, *torque = nullptr;
+    bool have_tree = false;   // a step has run
+    bool tree_last = false;   // the tree is that of the last step's boxes
+    hipGraphExec_t graph[2][3] = {};  // two steps from buffer parity 0 / 1, by what they do with the lists
+    hipGraph_t graph_obj[2][3] = {};
+    float4 *ilo = nullptr, *ihi = nullptr;  // inflated boxes of a step that builds lists
+    ClumpCtl* ctl = nullptr;
+    uint8_t* lcount = nullptr;
+    int* list = nullptr;
+    float size = 0.0f;        // mean extent of the bodies
+    int list_steps = 0;       // steps the lists are expected to last (0: build them next)
+    int list_rest = 0;        // steps to run without lists before they are tried again
+    float last_move = -1.0f;  // as last read back (negative: not known)
+    bool crowded = false;     // the last lists did not hold some body's partners
+    bool boxes = false;       // blo / bhi are those of the step before
     long long steps_done = 0;
     uint64_t static_hash = 0;  // of the fixed rows (inverse inertia, sphere ranges and offsets)
 };
@@ -343,21 +524,23 @@ sd_status dalloc(T** p, size_t count) {
 }
 
 void drop_clump_graphs(sd_clump_ctx* c) {
-    for (int k = 0; k < 2; ++k) {
-        if (c->graph[k]) (void)hipGraphExecDestroy(c->graph[k]);
-        if (c->graph_obj[k]) (void)hipGraphDestroy(c->graph_obj[k]);
-        c->graph[k] = nullptr;
-        c->graph_obj[k] = nullptr;
-    }
+    for (int k = 0; k < 2; ++k)
+        for (int l = 0; l < 3; ++l) {
+            if (c->graph[k][l]) (void)hipGraphExecDestroy(c->graph[k][l]);
+            if (c->graph_obj[k][l]) (void)hipGraphDestroy(c->graph_obj[k][l]);
+            c->graph[k][l] = nullptr;
+            c->graph_obj[k][l] = nullptr;
+        }
 }
 
 void cfree(sd_clump_ctx* c) {
     void* bufs[] = {c->pos[0],  c->pos[1],    c->vel[0],     c->vel[1],   c->quat[0], c->quat[1],  c->angm[0],
-                    c->angm[1], c->i0,        c->i1,         c->omega,    c->bfirst,  c->bcount,   c->sbody,
-                    c->slocal,  c->sx,        c->sv,         c->blo,      c->bhi,     c->domain,   c->dom_scratch,
+                    c->angm[1], c->i0,        c->i1,         c->omega,    c->bfirst,  c->bcount,
+                    c->slocal,  c->sx,        c->blo,      c->bhi,     c->domain,   c->dom_scratch,
                     c->mkeys,   c->mkeys2,    c->sort_tmp,   c->left,     c->right,   c->parent,   c->first,
-                    c->last,    c->rope,      c->nlo,        c->nhi,      c->counters, c->error,   c->q_scratch,
-                    c->pairs,   c->force,     c->torque,     c->pnode};
+                    c->last,    c->rope,      c->nlo,        c->nhi,      c->counters, c->q_scratch,
+                    c->pairs,   c->ilo,       c->ihi,        c->pnode,
+                    c->ctl,     c->lcount,    c->list};
     drop_clump_graphs(c);
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -387,52 +570,89 @@ int bits_for(uint64_t v) {
 
 ClumpState state_of(sd_clump_ctx* c, int k) { return ClumpState{c->pos[k], c->vel[k], c->quat[k], c->angm[k]}; }
 
-// One step. ev (optional, 6 events): prep+pose+aabb | domain+morton+sort | lbvh build |
-// (empty) | (empty) | partner search + contacts + integrate.
-sd_status clump_step(sd_clump_ctx* c, hipEvent_t* ev) {
+// The tree of the boxes lo / hi over the domain of the exact ones.
+sd_status clump_tree(sd_clump_ctx* c, const float4* lo, const float4* hi, hipEvent_t* ev) {
     hipStream_t s = c->stream;
-    const int nb = c->nb, ns = c->ns;
-    const ClumpState cs = state_of(c, c->cur), nx = state_of(c, 1 - c->cur);
-    const ContactDev cd = to_dev(c->p.contact);
-#define MARK(i) \
-    if (ev) SD_HIP(hipEventRecord(ev[i], s))
-    MARK(0);
-    hipLaunchKernelGGL(k_body_prep, dim3(div_up(nb, 256)), dim3(256), 0, s, cs, c->i0, c->i1, nb, c->omega);
-    SD_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_clump_pose, dim3(div_up(ns, 256)), dim3(256), 0, s, cs, c->omega, c->slocal, c->sbody, ns,
-                       c->sx, c->sv);
-    SD_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_body_aabb, dim3(div_up(nb, 256)), dim3(256), 0, s, c->sx, c->bfirst, c->bcount, nb, c->blo,
-                       c->bhi);
-    SD_LAUNCH_CHECK();
-    MARK(1);
-    sd_status st = sd_global_domain((const float*)c->blo, (const float*)c->bhi, nb, c->domain, c->dom_scratch, s);
-    if (st != SD_OK) return st;
+    const int nb = c->nb;
     // Morton codes with their 6 lowest bits cleared (8 bits per axis), sorted
     // in 3 passes: partner sets are exact and contacts are gathered in
     // ascending partner id, so the results do not depend on the tree, and a
     // 256-cell axis is far finer than the bodies' spacing
-    st = launch_morton((const float*)c->blo, (const float*)c->bhi, nb, c->domain, c->mkeys, CL_MORTON_DROP, s);
+    sd_status st = launch_morton((const float*)lo, (const float*)hi, nb, c->domain, c->mkeys, CL_MORTON_DROP, s);
     if (st != SD_OK) return st;
     uint64_t *K = c->mkeys, *Ka = c->mkeys2;
     st = radix_sort_keys_u64(&K, &Ka, nb, 32 + CL_MORTON_DROP, 62, c->sort_tmp, c->sort_tmp_bytes, s, 0);
     if (st != SD_OK) return st;
-    MARK(2);
-    st = lbvh_build(K, nb, (const float*)c->blo, (const float*)c->bhi, c->left, c->right, c->parent, c->first,
-                    c->last, c->rope, (float*)c->nlo, (float*)c->nhi, c->counters, c->error, c->pnode, s);
-    if (st != SD_OK) return st;
+    if (ev) SD_HIP(hipEventRecord(ev[2], s));
+    st = lbvh_build(K, nb, (const float*)lo, (const float*)hi, c->left, c->right, c->parent, c->first, c->last,
+                    c->rope, (float*)c->nlo, (float*)c->nhi, c->counters, &c->ctl->error, c->pnode, s);
     c->ksorted = K;
+    return st;
+}
+
+// One step. ev (optional, 7 events): poses and boxes | domain+morton+sort | lbvh build |
+// (empty) | (empty) | partner search + contacts + integrate. lists: what the
+// step does with the partner lists (LIST_*).
+sd_status clump_step(sd_clump_ctx* c, hipEvent_t* ev, int lists) {
+    hipStream_t s = c->stream;
+    const int nb = c->nb, par = c->cur;
+    const ClumpState cs = state_of(c, c->cur), nx = state_of(c, 1 - c->cur);
+    const ContactDev cd = to_dev(c->p.contact);
+    sd_status st;
+#define MARK(i) \
+    if (ev) SD_HIP(hipEventRecord(ev[i], s))
+    MARK(0);
+    hipLaunchKernelGGL(k_clump_pose, dim3(div_up(nb, 256 / POSE_LANES)), dim3(256), 0, s, cs, c->i0, c->i1, c->slocal,
+                       c->bfirst, c->bcount, nb, c->omega, c->sx, c->blo, c->bhi, c->ctl, par, c->boxes ? 1 : 0);
+    SD_LAUNCH_CHECK();
+    c->boxes = true;
+    MARK(1);
+    if (lists != LIST_USE) {
+        st = sd_global_domain((const float*)c->blo, (const float*)c->bhi, nb, c->domain, c->dom_scratch, s);
+        if (st != SD_OK) return st;
+        const float4 *lo = c->blo, *hi = c->bhi;
+        if (lists == LIST_BUILD) {
+            hipLaunchKernelGGL(k_clump_margin, dim3(1), dim3(64), 0, s, c->ctl, par, c->size,
+                               (const float*)c->domain);
+            SD_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_clump_inflate, dim3(div_up(nb, 256)), dim3(256), 0, s, lo, hi, nb,
+                               (const ClumpCtl*)c->ctl, c->ilo, c->ihi);
+            SD_LAUNCH_CHECK();
+            lo = c->ilo;
+            hi = c->ihi;
+        }
+        st = clump_tree(c, lo, hi, ev);
+        if (st != SD_OK) return st;
+    } else {
+        MARK(2);
+    }
+    c->tree_last = lists == LIST_NONE;
     MARK(3);
     MARK(4);  // (partner search is part of the contact kernel)
     MARK(5);
-    hipLaunchKernelGGL(k_clump_contacts<true>, dim3(div_up(nb, CL_BLOCK)), dim3(CL_BLOCK), 0, s, cs, nx, c->omega,
-                       c->i0, c->i1, c->sx, c->sv, c->bfirst, c->bcount, nb, c->blo, c->bhi,
-                       (const float4*)c->pnode, cd, c->error, nullptr, nullptr);
+#define CONTACTS(L)                                                                                                   \
+    hipLaunchKernelGGL(k_clump_contacts<L>, dim3(div_up(nb, CL_BLOCK)), dim3(CL_BLOCK), 0, s, cs, nx, c->omega, c->i0, \
+                       c->i1, c->sx, c->slocal, c->bfirst, c->bcount, nb, c->blo, c->bhi, (const float4*)c->pnode, cd,     \
+                       c->ctl, par, c->lcount, c->list)
+    if (lists == LIST_USE) CONTACTS(LIST_USE);
+    else if (lists == LIST_BUILD) CONTACTS(LIST_BUILD);
+    else CONTACTS(LIST_NONE);
+#undef CONTACTS
     SD_LAUNCH_CHECK();
     MARK(6);
 #undef MARK
     c->cur = 1 - c->cur;
     return SD_OK;
+}
+
+// A changed state (upload, load): no lists, and the boxes say nothing about how far bodies move.
+sd_status clump_forget_lists(sd_clump_ctx* c) {
+    c->list_steps = 0;
+    c->list_rest = 0;
+    c->last_move = -1.0f;
+    c->crowded = false;
+    c->boxes = false;
+    return launch_fill_u32((uint32_t*)c->ctl, 0u, sizeof(ClumpCtl) / 4, c->stream);
 }
 
 }  // namespace
@@ -620,10 +840,8 @@ sd_status write_clump_rows(sd_clump_ctx* c, const ClumpRows& r) {
     ALLOC(c->omega, nb);
     ALLOC(c->bfirst, nb);
     ALLOC(c->bcount, nb);
-    ALLOC(c->sbody, ns);
     ALLOC(c->slocal, ns);
     ALLOC(c->sx, ns);
-    ALLOC(c->sv, ns);
     ALLOC(c->blo, nb);
     ALLOC(c->bhi, nb);
     ALLOC(c->domain, 8);
@@ -642,11 +860,13 @@ sd_status write_clump_rows(sd_clump_ctx* c, const ClumpRows& r) {
     ALLOC(c->nhi, 2 * (size_t)nb);
     ALLOC(c->pnode, 4 * (size_t)nb);
     ALLOC(c->counters, 3 * (size_t)nb + 8);
-    ALLOC(c->error, 1);
     sd_lbvh_query_scratch_bytes(nb, &c->q_scratch_bytes);
     ALLOC(*(char**)&c->q_scratch, c->q_scratch_bytes);
-    ALLOC(c->force, nb);
-    ALLOC(c->torque, nb);
+    ALLOC(c->ilo, nb);
+    ALLOC(c->ihi, nb);
+    ALLOC(c->ctl, 1);
+    ALLOC(c->lcount, nb);
+    ALLOC(c->list, (size_t)CL_LIST * nb);
 #undef ALLOC
     if (st == SD_OK) st = grow_pairs(c, 8 * nb);
     if (st != SD_OK) {
@@ -662,13 +882,26 @@ sd_status write_clump_rows(sd_clump_ctx* c, const ClumpRows& r) {
     SD_HIP(hipMemcpyAsync(c->i1, r.I1.data(), nb * sizeof(float4), hipMemcpyHostToDevice, s));
     SD_HIP(hipMemcpyAsync(c->bfirst, r.first.data(), nb * sizeof(int), hipMemcpyHostToDevice, s));
     SD_HIP(hipMemcpyAsync(c->bcount, r.count.data(), nb * sizeof(int), hipMemcpyHostToDevice, s));
-    SD_HIP(hipMemcpyAsync(c->sbody, sbody.data(), ns * sizeof(int), hipMemcpyHostToDevice, s));
     SD_HIP(hipMemcpyAsync(c->slocal, r.loc.data(), ns * sizeof(float4), hipMemcpyHostToDevice, s));
     SD_HIP(hipStreamSynchronize(s));
     c->cur = 0;
     c->have_tree = false;
     c->npairs = -1;
     c->static_hash = static_hash(r);
+    // mean extent of a body: twice the reach of its spheres from the centre
+    double size = 0.0;
+    for (int b = 0; b < nb; ++b) {
+        float reach = 0.0f;
+        for (int k = r.first[b]; k < r.first[b] + r.count[b]; ++k) {
+            const float4 l = r.loc[k];
+            reach = fmaxf(reach, sqrtf(l.x * l.x + l.y * l.y + l.z * l.z) + l.w);
+        }
+        size += 2.0 * (double)reach;
+    }
+    c->size = (float)(size / nb);
+    st = clump_forget_lists(c);
+    if (st != SD_OK) return st;
+    SD_HIP(hipStreamSynchronize(s));
     return SD_OK;
 }
 
@@ -719,13 +952,13 @@ extern "C" sd_status sd_clump_upload(sd_clump_ctx* c, int nb, const float* pos4,
     return SD_OK;
 }
 
-// Two steps from the current buffer parity, captured once per parity.
-static sd_status clump_graph_pair(sd_clump_ctx* c) {
+// Two steps from the current buffer parity, captured once per parity and kind.
+static sd_status clump_graph_pair(sd_clump_ctx* c, int lists) {
     const int k = c->cur;
-    if (!c->graph[k]) {
+    if (!c->graph[k][lists]) {
         SD_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        sd_status st = clump_step(c, nullptr);
-        if (st == SD_OK) st = clump_step(c, nullptr);
+        sd_status st = clump_step(c, nullptr, lists);
+        if (st == SD_OK) st = clump_step(c, nullptr, lists);
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         c->cur = k;  // capture advanced the parity twice: back where it was
@@ -740,10 +973,52 @@ static sd_status clump_graph_pair(sd_clump_ctx* c) {
             (void)hipGraphDestroy(g);
             SD_HIP(e);
         }
-        c->graph[k] = ge;
-        c->graph_obj[k] = g;
+        c->graph[k][lists] = ge;
+        c->graph_obj[k][lists] = g;
     }
-    SD_HIP(hipGraphLaunch(c->graph[k], c->stream));
+    SD_HIP(hipGraphLaunch(c->graph[k][lists], c->stream));
+    c->tree_last = lists == LIST_NONE;
+    return SD_OK;
+}
+
+// Steps between two looks at how long the lists last, or whether they would do.
+constexpr int CL_REST = 64;
+
+// Steps that lists are expected to last, a tenth short of what the last movement says.
+static int clump_list_life(float displaced, float limit, float last) {
+    const float steps = 0.9f * (limit - displaced) / fmaxf(last, 1e-30f);
+    return steps >= (float)CL_REST ? CL_REST : (steps > 0.0f ? (int)steps : 0);  // (not a number: 0)
+}
+
+// Whether lists pay at the bodies' speed: not where the largest margin would last fewer than 4 steps.
+static bool clump_lists_pay(const sd_clump_ctx* c) {
+    return c->size > 0.0f && 4.0f * c->last_move <= CL_MARGIN_MAX * c->size;
+}
+
+// What a launch sequence left: the steps that ran set the buffer parity, the
+// movement says how long lists will last.
+static sd_status clump_read_ctl(sd_clump_ctx* c, int cur0, int limit, bool use, int* ran) {
+    ClumpCtl ctl;
+    SD_HIP(hipMemcpyAsync(&ctl, c->ctl, CLUMP_CTL_READ * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    SD_HIP(hipStreamSynchronize(c->stream));
+    if (ctl.ran < 0 || ctl.ran > limit || (ctl.ran == 0 && ctl.given_up == 0))
+        return set_error(SD_ERR_STATE, "sd_clump_step: %d of %d steps ran", ctl.ran, limit);
+    *ran = ctl.ran;
+    c->cur = cur0 ^ (ctl.ran & 1);
+    c->last_move = isfinite(ctl.last) ? ctl.last : 3.4e38f;
+    // the movement of the step to come is not in yet: count it as the last one
+    c->list_steps = ctl.given_up ? 0 : clump_list_life(ctl.displaced[c->cur] + ctl.last, ctl.limit, ctl.last);
+    if (use) {
+        c->crowded = ctl.over != 0;
+        if (c->crowded) {
+            c->list_steps = 0;
+            c->list_rest = 4 * CL_REST;
+        }
+    } else {
+        c->list_steps = 0;
+        c->list_rest = std::max(0, c->list_rest - ctl.ran);
+    }
+    if (ctl.error) return set_error(SD_ERR_STATE, "sd_clump_step: malformed tree (error bits %d)", ctl.error);
     return SD_OK;
 }
 
@@ -751,24 +1026,47 @@ extern "C" sd_status sd_clump_step(sd_clump_ctx* c, int nsteps) {
     SD_REQUIRE(c && nsteps >= 0, "sd_clump_step: bad argument");
     if (c->nb == 0) return set_error(SD_ERR_STATE, "sd_clump_step: no bodies uploaded");
     if (nsteps == 0) return SD_OK;
-    sd_status st = launch_fill_u32((uint32_t*)c->error, 0u, 1, c->stream);
-    if (st != SD_OK) return st;
+    auto run = [&](int l, int lists) -> sd_status {
+        sd_status e = SD_OK;
+        for (; l >= 2 && e == SD_OK; l -= 2) e = clump_graph_pair(c, lists);
+        if (l > 0 && e == SD_OK) e = clump_step(c, nullptr, lists);
+        return e;
+    };
     int left = nsteps;
-    for (; left >= 2; left -= 2) {
-        st = clump_graph_pair(c);
+    while (left > 0) {
+        sd_status st = launch_fill_u32((uint32_t*)c->ctl, 0u, 3, c->stream);  // given_up, ran, error
+        if (st != SD_OK) return st;
+        const int cur0 = c->cur;
+        const bool use = clump_lists_pay(c) && c->list_rest == 0;
+        if (!use) {
+            // the first step's boxes are compared with none, so never one of a captured pair
+            int l = std::min(left, CL_REST);
+            if (!c->boxes) {
+                st = clump_step(c, nullptr, LIST_NONE);
+                --l;
+            }
+            if (st == SD_OK) st = run(l, LIST_NONE);
+        } else {
+            int l = left;
+            if (c->list_steps < std::min(left, 2)) {
+                st = clump_step(c, nullptr, LIST_BUILD);
+                // (of unknown speed, or too full for lists the last time: a look first)
+                c->list_steps = c->crowded || c->last_move < 0.0f
+                                    ? 2
+                                    : clump_list_life(0.0f, 0.98f * clump_margin(c->last_move, c->size), c->last_move);
+                --l;
+            }
+            if (st == SD_OK) st = run(std::min(l, c->list_steps), LIST_USE);
+        }
+        if (st != SD_OK) return st;
+        int ran = 0;
+        st = clump_read_ctl(c, cur0, left, use, &ran);
+        left -= ran;
+        c->steps_done += ran;
+        c->have_tree = true;
+        c->npairs = -1;  // the pair list of the new last step is built when asked for
         if (st != SD_OK) return st;
     }
-    if (left) {
-        st = clump_step(c, nullptr);
-        if (st != SD_OK) return st;
-    }
-    int err = 0;
-    SD_HIP(hipMemcpyAsync(&err, c->error, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SD_HIP(hipStreamSynchronize(c->stream));
-    c->steps_done += nsteps;
-    c->have_tree = true;
-    c->npairs = -1;  // the pair list of the new last step is built when asked for
-    if (err) return set_error(SD_ERR_STATE, "sd_clump_step: malformed tree (error bits %d)", err);
     return SD_OK;
 }
 
@@ -781,11 +1079,23 @@ extern "C" sd_status sd_clump_profile(sd_clump_ctx* c, int nsteps, float* stage_
     for (int k = 0; k < 7; ++k) SD_HIP(hipEventCreate(&ev[k]));
     sd_status st = SD_OK;
     for (int i = 0; i < nsteps && st == SD_OK; ++i) {
-        st = clump_step(c, ev);
+        // the lists as a run would use them, the step redone if they ran out
+        const int cur0 = c->cur;
+        const bool use = clump_lists_pay(c);
+        const int lists = !use ? LIST_NONE : (c->list_steps < 1 || c->crowded ? LIST_BUILD : LIST_USE);
+        st = launch_fill_u32((uint32_t*)c->ctl, 0u, 3, c->stream);
+        if (st == SD_OK) st = clump_step(c, ev, lists);
         if (st != SD_OK) break;
         if (hipEventSynchronize(ev[6]) != hipSuccess) {
             st = set_error(SD_ERR_HIP, "sd_clump_profile: event wait failed");
             break;
+        }
+        int ran = 0;
+        st = clump_read_ctl(c, cur0, 1, use, &ran);
+        if (st != SD_OK) break;
+        if (ran == 0) {
+            --i;
+            continue;
         }
         for (int k = 0; k < ns; ++k) {
             float ms = 0.0f;
@@ -824,14 +1134,22 @@ extern "C" sd_status sd_clump_pairs(sd_clump_ctx* c, int* pairs, int capacity, i
     if (!c->have_tree) return set_error(SD_ERR_STATE, "sd_clump_pairs: no step has run");
     if (c->npairs < 0) {  // query the last step's tree
         int np = 0;
-        sd_status st = sd_lbvh_query(c->ksorted, c->nb, c->left, c->last, c->rope, (const float*)c->nlo,
-                                     (const float*)c->nhi, c->pairs, c->pair_cap, &np, c->error, c->q_scratch,
+        sd_status st = SD_OK;
+        if (!c->tree_last) {  // a step on lists has none, one that builds them a tree of inflated boxes
+            st = sd_global_domain((const float*)c->blo, (const float*)c->bhi, c->nb, c->domain, c->dom_scratch,
+                                  c->stream);
+            if (st == SD_OK) st = clump_tree(c, c->blo, c->bhi, nullptr);
+            if (st != SD_OK) return st;
+            c->tree_last = true;
+        }
+        st = sd_lbvh_query(c->ksorted, c->nb, c->left, c->last, c->rope, (const float*)c->nlo,
+                                     (const float*)c->nhi, c->pairs, c->pair_cap, &np, &c->ctl->error, c->q_scratch,
                                      c->q_scratch_bytes, c->stream);
         if (st == SD_ERR_CAPACITY) {
             st = grow_pairs(c, np);
             if (st != SD_OK) return st;
             st = sd_lbvh_query(c->ksorted, c->nb, c->left, c->last, c->rope, (const float*)c->nlo,
-                               (const float*)c->nhi, c->pairs, c->pair_cap, &np, c->error, c->q_scratch,
+                               (const float*)c->nhi, c->pairs, c->pair_cap, &np, &c->ctl->error, c->q_scratch,
                                c->q_scratch_bytes, c->stream);
         }
         if (st != SD_OK) return st;
@@ -921,6 +1239,8 @@ extern "C" sd_status sd_clump_load(sd_clump_ctx* c, const void* buffer, size_t b
         SD_HIP(hipMemcpyAsync(dst[k], b, b4, hipMemcpyHostToDevice, c->stream));
         b += b4;
     }
+    const sd_status st = clump_forget_lists(c);
+    if (st != SD_OK) return st;
     SD_HIP(hipStreamSynchronize(c->stream));
     c->steps_done = h.steps_done;
     c->have_tree = false;
