@@ -131,7 +131,10 @@ sd_status sd_cell_ranges_u64(const uint64_t* sorted_keys, int n, int n_cells, in
  * (a, b) int pairs, grouped by a ascending and, within a, in stencil order.
  * If the pair count exceeds capacity, *n_pairs receives the required count and
  * SD_ERR_CAPACITY is returned. Replaces resolveCollisionsCUDA's pair loop
- * (collision_resolution.cu:56-97) and the SAP pair rows (sap_detection.cu:293-324). */
+ * (collision_resolution.cu:56-97) and the SAP pair rows (sap_detection.cu:293-324).
+ * Scratch of sd_neighbor_pairs_scratch_bytes holds every sphere's first 8
+ * partners between the count and the output; 32 bytes a sphere less will do,
+ * at the price of a second search. */
 sd_status sd_neighbor_pairs(const float* pos4, int n, const sd_grid* grid, const int* ranges, float skin,
                             int* pairs, int capacity, int* n_pairs, void* scratch, size_t scratch_bytes,
                             void* stream);

@@ -100,7 +100,6 @@ __device__ __forceinline__ void find_history(const ContactArgs& a, int os, int o
     }
 }
 
-constexpr int XCDS = 8;       // gfx950: 8 accelerator complex dies, one L2 each
 constexpr int CAND_UNROLL = 4; // candidate positions loaded per batch (loads in flight)
 static_assert(CAND_UNROLL - 1 <= CONTACT_POS_PAD, "sorted positions must be padded for a whole batch");
 constexpr int CONTACT_STAGE = 224;  // staged candidate positions per wave (3.5 KiB of LDS)
@@ -118,15 +117,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Workgroup i is dispatched to XCD i % 8. Remap so that every XCD works on a
-// contiguous range of logical blocks: blocks resident on one XCD then touch
-// neighbouring cells and share that XCD's L2. Returns -1 for padding blocks.
-__device__ __forceinline__ int xcd_logical_block(int nblocks) {
-    const int per = (nblocks + XCDS - 1) / XCDS;
-    const int lb = (int)(blockIdx.x % XCDS) * per + (int)(blockIdx.x / XCDS);
-    return lb < nblocks ? lb : -1;
 }
 
 // Largest of the wave's squared displacements into one of the step's maxima

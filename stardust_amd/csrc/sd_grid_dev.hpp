@@ -5,6 +5,17 @@
 
 namespace sd {
 
+constexpr int XCDS = 8; //  gfx950: 8 accelerator complex dies, one L2 each
+
+// Workgroup i is dispatched to XCD i % 8. Remap so that every XCD works on a
+// contiguous range of logical blocks: blocks resident on one XCD then touch
+// neighbouring cells and share that XCD's L2. Returns -1 for padding blocks.
+__device__ __forceinline__ int xcd_logical_block(int nblocks) {
+    const int per = (nblocks + XCDS - 1) / XCDS;
+    const int lb = (int)(blockIdx.x % XCDS) * per + (int)(blockIdx.x / XCDS);
+    return lb < nblocks ? lb : -1;
+}
+
 // clamp(floor((p - lo) / cell), 0, nc - 1); NaN maps to 0.
 __device__ __forceinline__ int axis_cell(float p, float lo, float cell, int nc) {
     float f = floorf((p - lo) / cell);
