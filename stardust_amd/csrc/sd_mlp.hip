@@ -10,6 +10,9 @@
 // normalised to a unit vector. Parameters (FP32 master copy, 9,987 floats):
 //   W1[22][64] b1[64] W2[64][64] b2[64] W3[64][64] b3[64] W4[64][3] b4[3]
 // (W[i][j]: input i -> output j). Loss per sample: 1 - u . t (u = y/|y|).
+#include <algorithm>
+#include <type_traits>
+
 #include "sd_gjk_dev.hpp"
 #include "sd_internal.hpp"
 
@@ -178,206 +181,279 @@ __global__ void k_mlp_init(float* __restrict__ w, uint64_t seed) {
 
 // ------------------------------------------------------------------ training
 
-constexpr int TB_S = 64;       // samples per block
-constexpr int TB_T = 256;      // threads per block
-constexpr int XS = NIN + 2;    // padded row of the input tile
+constexpr int TB_S = 32;       // samples per tile
+constexpr int TB_T = 256;      // threads per block: a wave per 16 columns
+constexpr int TB_GRID = 256;   // blocks: one a CU, which take several tiles of a larger batch
+constexpr int TB_MIN = 64;     // samples per partial gradient that the scratch must hold at least
+constexpr int XS = NH / 2 + 1; // row of the input tile (inputs 22 .. 31 are 0)
+constexpr int HS = NH + 4;     // row of a layer's tile (16-byte aligned, rows start in different banks)
+static_assert(NH == 64 && TB_T == 4 * NH && NIN <= 24 && TB_S == 32, "the tiling below");
 
-// Forward + backward of one block of samples; writes this block's gradient
-// (summed over its samples, already divided by the batch size) and loss sum.
-// Sample s of the block is dataset row idx[blk * 64 + s] (rows past `count`
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(4))) Floats4 {  // four floats anywhere
+    float x, y, z, w;
+};
+
+// Forward + backward of the block's tiles of 32 samples; writes the block's
+// gradient (summed over its samples, already divided by the batch size) and loss
+// sum. Sample s of a tile is dataset row idx[tile * 32 + s] (rows past `count`
 // contribute nothing).
-__global__ __launch_bounds__(TB_T) void k_mlp_fwd_bwd(const float* __restrict__ X, const float* __restrict__ T,
-                                                     const int* __restrict__ idx, int count, float inv_batch,
-                                                     const float* __restrict__ w, float* __restrict__ gpart,
-                                                     float* __restrict__ lpart) {
+//
+// The products run on the FP32 matrix instruction (16x16 tiles, 4 terms at a
+// time, each a fused multiply-add): operands in FP32, so its error against 64
+// bits is no larger than that of the multiply and add it replaces. Wave w owns
+// columns 16 w .. 16 w + 15 of every layer: a lane (group g = lane / 16, c =
+// lane % 16) holds results of rows 4 g .. 4 g + 3 and column c, so activations'
+// derivatives and the sums over samples stay in its registers, as do the weights.
+// Terms are handed out so that group g has a run of 16 of the 64 inputs (or of
+// 8 of the 32 samples): read 16 bytes at a time.
+//
+// Bound by the chain of nine barriers and the LDS reads between them (the
+// arithmetic of 8,192 samples is 3 us): 64 samples a block and multiplies fed
+// from LDS one by one took 74 us, this takes 20 (a gradient of 65,536 samples:
+// 526 us, now 95). Limited to 2 waves a SIMD's registers, it spills and takes 23.
+__global__ __launch_bounds__(TB_T, 1) void k_mlp_fwd_bwd(const float* __restrict__ X, const float* __restrict__ T,
+                                                        const int* __restrict__ idx, int count, float inv_batch,
+                                                        const float* __restrict__ w, float* __restrict__ gpart,
+                                                        float* __restrict__ lpart) {
     __shared__ float sx[TB_S][XS];
-    __shared__ float z1[TB_S][NH], h1[TB_S][NH], z2[TB_S][NH], h2[TB_S][NH], z3[TB_S][NH], h3[TB_S][NH];
-    __shared__ float g[TB_S][NH];
-    __shared__ float sy[TB_S][4], st[TB_S][4], sdy[TB_S][4], sl[TB_S];
-    __shared__ int valid[TB_S];
-    const int tid = threadIdx.x;
-    const int base = blockIdx.x * TB_S;
-    for (int e = tid; e < TB_S * NIN; e += TB_T) {
-        const int s = e / NIN, i = e % NIN;
-        const int r = base + s < count ? idx[base + s] : -1;
-        sx[s][i] = r >= 0 ? X[(size_t)r * NIN + i] : 0.0f;
-    }
-    for (int e = tid; e < TB_S * NOUT; e += TB_T) {
-        const int s = e / NOUT, k = e % NOUT;
-        const int r = base + s < count ? idx[base + s] : -1;
-        st[s][k] = r >= 0 ? T[(size_t)r * NOUT + k] : 0.0f;
-    }
-    if (tid < TB_S) valid[tid] = base + tid < count ? 1 : 0;
-    __syncthreads();
+    __shared__ __align__(16) float H1[TB_S][HS], H2[TB_S][HS], H3[TB_S][HS], G[TB_S][HS];
+    __shared__ __align__(16) float sy[TB_S][4], st[TB_S][4], sdy[TB_S][4];
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    const int wave = tid >> 6, j = wave * 16 + c;
 
-    // thread -> (output column j, 16 samples)
-    const int j = tid & (NH - 1);
-    const int s0 = (tid >> 6) * 16;
-    float acc[16];
-    // layer 1
+    // this lane's weights: column j (forward), row j (backward)
+    float w1[6], w2[16], w3[16], r2[16], r3[16], w4[3];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = w[OFF_B1 + j];
-    for (int i = 0; i < NIN; ++i) {
-        const float wij = w[OFF_W1 + i * NH + j];
+    for (int k = 0; k < 6; ++k) w1[k] = g * 6 + k < NIN ? w[OFF_W1 + (g * 6 + k) * NH + j] : 0.0f;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = acc[q] + sx[s0 + q][i] * wij;
+    for (int k = 0; k < 16; ++k) {
+        w2[k] = w[OFF_W2 + (g * 16 + k) * NH + j];
+        w3[k] = w[OFF_W3 + (g * 16 + k) * NH + j];
     }
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        z1[s0 + q][j] = acc[q];
-        h1[s0 + q][j] = acc[q] * sigm(acc[q]);
-    }
-    __syncthreads();
-    // layer 2
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = w[OFF_B2 + j];
-    for (int i = 0; i < NH; ++i) {
-        const float wij = w[OFF_W2 + i * NH + j];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = acc[q] + h1[s0 + q][i] * wij;
+    for (int k = 0; k < 16; k += 4) {
+        const Floats4 a = *reinterpret_cast<const Floats4*>(w + OFF_W2 + j * NH + g * 16 + k);
+        const Floats4 b = *reinterpret_cast<const Floats4*>(w + OFF_W3 + j * NH + g * 16 + k);
+        r2[k] = a.x, r2[k + 1] = a.y, r2[k + 2] = a.z, r2[k + 3] = a.w;
+        r3[k] = b.x, r3[k + 1] = b.y, r3[k + 2] = b.z, r3[k + 3] = b.w;
     }
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        z2[s0 + q][j] = acc[q];
-        h2[s0 + q][j] = acc[q] * sigm(acc[q]);
-    }
-    __syncthreads();
-    // layer 3
+    for (int k = 0; k < 3; ++k) w4[k] = w[OFF_W4 + j * NOUT + k];
+    const float b1 = w[OFF_B1 + j], b2 = w[OFF_B2 + j], b3 = w[OFF_B3 + j];
+
+    f32x4 dw1[2] = {}, dw2[4] = {}, dw3[4] = {};
+    float db1 = 0.0f, db2 = 0.0f, db3 = 0.0f, dw4[3] = {0.0f, 0.0f, 0.0f};
+    float db4[3] = {0.0f, 0.0f, 0.0f}, lsum = 0.0f;  // of sample tid (the first 32 threads)
+
+    // rows of A, 64 terms, times the lane's operands b, added to acc (both row tiles)
+    auto layer = [&](const float (*A)[HS], const float* b, f32x4* acc) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = w[OFF_B3 + j];
-    for (int i = 0; i < NH; ++i) {
-        const float wij = w[OFF_W3 + i * NH + j];
+        for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = acc[q] + h2[s0 + q][i] * wij;
-    }
+            for (int k = 0; k < 16; k += 4) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(&A[m * 16 + c][g * 16 + k]);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        z3[s0 + q][j] = acc[q];
-        h3[s0 + q][j] = acc[q] * sigm(acc[q]);
+                for (int u = 0; u < 4; ++u)
+                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[k + u], acc[m], 0, 0, 0);
+            }
+    };
+    // SiLU of acc to H, its derivative to d
+    auto activate = [&](const f32x4* acc, float (*H)[HS], f32x4* d) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float z = acc[m][r], sg = sigm(z);
+                H[m * 16 + 4 * g + r][j] = z * sg;
+                d[m][r] = sg * (1.0f + z * (1.0f - sg));
+            }
+    };
+    // D += A^T B over the tile's samples: MT tiles of 16 columns of A, column j of B
+    auto outer = [&](const float* A, int stride, const float (*B)[HS], f32x4* D, auto mt) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int s = g * 8 + k;
+            const float b = B[s][j];
+#pragma unroll
+            for (int m = 0; m < decltype(mt)::value; ++m)
+                D[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[s * stride + m * 16 + c], b, D[m], 0, 0, 0);
+        }
+    };
+
+    for (int base = (int)blockIdx.x * TB_S; base < count; base += (int)gridDim.x * TB_S) {
+        for (int e = tid; e < TB_S * 32; e += TB_T) {
+            const int s = e >> 5, i = e & 31;
+            const int r = base + s < count ? idx[base + s] : -1;
+            sx[s][i] = r >= 0 && i < NIN ? X[(size_t)r * NIN + i] : 0.0f;
+        }
+        if (tid < TB_S * 4) {
+            const int s = tid >> 2, k = tid & 3;
+            const int r = base + s < count ? idx[base + s] : -1;
+            st[s][k] = r >= 0 && k < NOUT ? T[(size_t)r * NOUT + k] : 0.0f;
+        }
+        __syncthreads();
+        f32x4 d1[2], d2[2], d3[2], acc[2];
+        acc[0] = acc[1] = f32x4{b1, b1, b1, b1};
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[m * 16 + c][g * 6 + k], w1[k], acc[m], 0, 0, 0);
+        activate(acc, H1, d1);
+        __syncthreads();
+        acc[0] = acc[1] = f32x4{b2, b2, b2, b2};
+        layer(H1, w2, acc);
+        activate(acc, H2, d2);
+        __syncthreads();
+        acc[0] = acc[1] = f32x4{b3, b3, b3, b3};
+        layer(H2, w3, acc);
+        activate(acc, H3, d3);
+        __syncthreads();
+        if (wave < 2) {  // the outputs of 16 samples (columns past the third: 0)
+            const float b = c < NOUT ? w[OFF_B4 + c] : 0.0f;
+            f32x4 y = {b, b, b, b};
+#pragma unroll
+            for (int k = 0; k < 16; k += 4) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(&H3[wave * 16 + c][g * 16 + k]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float b4 = c < NOUT ? w[OFF_W4 + (g * 16 + k + u) * NOUT + c] : 0.0f;
+                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b4, y, 0, 0, 0);
+                }
+            }
+            if (c < NOUT)
+                for (int r = 0; r < 4; ++r) sy[wave * 16 + 4 * g + r][c] = y[r];
+        }
+        __syncthreads();
+        if (tid < TB_S) {
+            const int s = tid;
+            const float y0 = sy[s][0], y1 = sy[s][1], y2 = sy[s][2];
+            const float ny = sqrtf(y0 * y0 + y1 * y1 + y2 * y2) + 1e-12f;
+            const float u0 = y0 / ny, u1 = y1 / ny, u2 = y2 / ny;
+            const float ut = u0 * st[s][0] + u1 * st[s][1] + u2 * st[s][2];
+            const bool valid = base + s < count;
+            const float sc = valid ? inv_batch : 0.0f;
+            lsum = lsum + (valid ? 1.0f - ut : 0.0f);
+            // d(1 - u.t)/dy = -(t - (u.t) u) / |y|
+            const float e0 = -(st[s][0] - ut * u0) / ny * sc;
+            const float e1 = -(st[s][1] - ut * u1) / ny * sc;
+            const float e2 = -(st[s][2] - ut * u2) / ny * sc;
+            sdy[s][0] = e0, sdy[s][1] = e1, sdy[s][2] = e2;
+            db4[0] = db4[0] + e0, db4[1] = db4[1] + e1, db4[2] = db4[2] + e2;
+        }
+        __syncthreads();
+        // dz3 = (dy W4^T) * silu'(z3) -> G, dW4, db3
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int s = m * 16 + 4 * g + r;
+                const f32x4 e = *reinterpret_cast<const f32x4*>(sdy[s]);
+                const float h = H3[s][j];
+                const float gv = (e[0] * w4[0] + e[1] * w4[1] + e[2] * w4[2]) * d3[m][r];
+                G[s][j] = gv;
+                db3 = db3 + gv;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) dw4[k] = dw4[k] + h * e[k];
+            }
+        __syncthreads();
+        // dW3 = h2^T dz3, dz2 = (dz3 W3^T) * silu'(z2) -> H3 (free now)
+        outer(&H2[0][0], HS, G, dw3, std::integral_constant<int, 4>{});
+        acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        layer(G, r3, acc);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float gv = acc[m][r] * d2[m][r];
+                H3[m * 16 + 4 * g + r][j] = gv;
+                db2 = db2 + gv;
+            }
+        __syncthreads();
+        // dW2 = h1^T dz2, dz1 = (dz2 W2^T) * silu'(z1) -> G
+        outer(&H1[0][0], HS, H3, dw2, std::integral_constant<int, 4>{});
+        acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        layer(H3, r2, acc);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float gv = acc[m][r] * d1[m][r];
+                G[m * 16 + 4 * g + r][j] = gv;
+                db1 = db1 + gv;
+            }
+        // dW1 = x^T dz1 (column j of G is this wave's own, but other lanes')
+        __syncthreads();
+        outer(&sx[0][0], XS, G, dw1, std::integral_constant<int, 2>{});
+        __syncthreads();  // every read precedes the next tile
     }
-    __syncthreads();
-    // output layer + loss + dL/dy
-    if (tid < TB_S * NOUT) {
-        const int s = tid / NOUT, k = tid % NOUT;
-        float y = w[OFF_B4 + k];
-        for (int i = 0; i < NH; ++i) y = y + h3[s][i] * w[OFF_W4 + i * NOUT + k];
-        sy[s][k] = y;
-    }
-    __syncthreads();
-    if (tid < TB_S) {
-        const int s = tid;
-        const float y0 = sy[s][0], y1 = sy[s][1], y2 = sy[s][2];
-        const float ny = sqrtf(y0 * y0 + y1 * y1 + y2 * y2) + 1e-12f;
-        const float u0 = y0 / ny, u1 = y1 / ny, u2 = y2 / ny;
-        const float ut = u0 * st[s][0] + u1 * st[s][1] + u2 * st[s][2];
-        const float sc = valid[s] ? inv_batch : 0.0f;
-        sl[s] = valid[s] ? 1.0f - ut : 0.0f;
-        // d(1 - u.t)/dy = -(t - (u.t) u) / |y|
-        sdy[s][0] = -(st[s][0] - ut * u0) / ny * sc;
-        sdy[s][1] = -(st[s][1] - ut * u1) / ny * sc;
-        sdy[s][2] = -(st[s][2] - ut * u2) / ny * sc;
-    }
-    __syncthreads();
+
     float* gp = gpart + (size_t)blockIdx.x * NPARAM;
-    // dW4, db4
-    if (tid < NH * NOUT) {
-        const int i = tid / NOUT, k = tid % NOUT;
-        float a = 0.0f;
-        for (int s = 0; s < TB_S; ++s) a = a + h3[s][i] * sdy[s][k];
-        gp[OFF_W4 + i * NOUT + k] = a;
-    }
-    if (tid < NOUT) {
-        float a = 0.0f;
-        for (int s = 0; s < TB_S; ++s) a = a + sdy[s][tid];
-        gp[OFF_B4 + tid] = a;
-    }
-    // dz3 = (dy W4^T) * silu'(z3) -> g
-    for (int e = tid; e < TB_S * NH; e += TB_T) {
-        const int s = e / NH, i = e % NH;
-        const float dh = sdy[s][0] * w[OFF_W4 + i * NOUT] + sdy[s][1] * w[OFF_W4 + i * NOUT + 1] +
-                         sdy[s][2] * w[OFF_W4 + i * NOUT + 2];
-        const float z = z3[s][i], sg = sigm(z);
-        g[s][i] = dh * (sg * (1.0f + z * (1.0f - sg)));
-    }
-    __syncthreads();
-    // dW3 = h2^T g, db3 ; then dz2 = (g W3^T) * silu'(z2) -> h3 (free now)
-    {
-        const int i0 = (tid >> 6) * 16;  // 16 input rows per thread, column j
-        for (int q = 0; q < 16; ++q) {
-            float a = 0.0f;
-            for (int s = 0; s < TB_S; ++s) a = a + h2[s][i0 + q] * g[s][j];
-            gp[OFF_W3 + (i0 + q) * NH + j] = a;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = m * 16 + 4 * g + r;
+            if (m < 2 && i < NIN) gp[OFF_W1 + i * NH + j] = dw1[m & 1][r];
+            gp[OFF_W2 + i * NH + j] = dw2[m][r];
+            gp[OFF_W3 + i * NH + j] = dw3[m][r];
         }
-        if (tid < NH) {
-            float a = 0.0f;
-            for (int s = 0; s < TB_S; ++s) a = a + g[s][tid];
-            gp[OFF_B3 + tid] = a;
+    auto groups = [&](float v) {  // over the 4 groups
+        v = v + __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
+    db1 = groups(db1);
+    db2 = groups(db2);
+    db3 = groups(db3);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) dw4[k] = groups(dw4[k]);
+    if (g == 0) {
+        gp[OFF_B1 + j] = db1;
+        gp[OFF_B2 + j] = db2;
+        gp[OFF_B3 + j] = db3;
+        for (int k = 0; k < 3; ++k) gp[OFF_W4 + j * NOUT + k] = dw4[k];
+    }
+    if (wave == 0) {
+#pragma unroll
+        for (int d = 1; d < TB_S; d <<= 1) {
+            lsum = lsum + __shfl_xor(lsum, d);
+            for (int k = 0; k < 3; ++k) db4[k] = db4[k] + __shfl_xor(db4[k], d);
         }
-    }
-    for (int e = tid; e < TB_S * NH; e += TB_T) {
-        const int s = e / NH, i = e % NH;
-        float dh = 0.0f;
-        for (int k = 0; k < NH; ++k) dh = dh + g[s][k] * w[OFF_W3 + i * NH + k];
-        const float z = z2[s][i], sg = sigm(z);
-        h3[s][i] = dh * (sg * (1.0f + z * (1.0f - sg)));
-    }
-    __syncthreads();
-    // dW2 = h1^T dz2, db2 ; dz1 = (dz2 W2^T) * silu'(z1) -> g
-    {
-        const int i0 = (tid >> 6) * 16;
-        for (int q = 0; q < 16; ++q) {
-            float a = 0.0f;
-            for (int s = 0; s < TB_S; ++s) a = a + h1[s][i0 + q] * h3[s][j];
-            gp[OFF_W2 + (i0 + q) * NH + j] = a;
+        if (lane == 0) {
+            for (int k = 0; k < 3; ++k) gp[OFF_B4 + k] = db4[k];
+            lpart[blockIdx.x] = lsum;
         }
-        if (tid < NH) {
-            float a = 0.0f;
-            for (int s = 0; s < TB_S; ++s) a = a + h3[s][tid];
-            gp[OFF_B2 + tid] = a;
-        }
-    }
-    __syncthreads();  // g is rewritten below; everyone finished reading it above
-    for (int e = tid; e < TB_S * NH; e += TB_T) {
-        const int s = e / NH, i = e % NH;
-        float dh = 0.0f;
-        for (int k = 0; k < NH; ++k) dh = dh + h3[s][k] * w[OFF_W2 + i * NH + k];
-        const float z = z1[s][i], sg = sigm(z);
-        g[s][i] = dh * (sg * (1.0f + z * (1.0f - sg)));
-    }
-    __syncthreads();
-    // dW1 = x^T dz1, db1
-    for (int e = tid; e < NIN * NH; e += TB_T) {
-        const int i = e / NH, jj = e % NH;
-        float a = 0.0f;
-        for (int s = 0; s < TB_S; ++s) a = a + sx[s][i] * g[s][jj];
-        gp[OFF_W1 + i * NH + jj] = a;
-    }
-    if (tid < NH) {
-        float a = 0.0f;
-        for (int s = 0; s < TB_S; ++s) a = a + g[s][tid];
-        gp[OFF_B1 + tid] = a;
-    }
-    if (tid == 0) {
-        float a = 0.0f;
-        for (int s = 0; s < TB_S; ++s) a = a + sl[s];
-        lpart[blockIdx.x] = a;
     }
 }
 
 // grad[p] = sum over blocks (fixed order); loss = sum of block losses * inv_batch.
-__global__ void k_mlp_reduce(const float* __restrict__ gpart, const float* __restrict__ lpart, int nblocks,
-                             float inv_batch, float* __restrict__ grad, float* __restrict__ loss) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < NPARAM) {
-        float a = 0.0f;
-        for (int b = 0; b < nblocks; ++b) a = a + gpart[(size_t)b * NPARAM + p];
-        grad[p] = a;
+// A block sums 64 parameters with 16 waves, each a sixteenth of the partial
+// gradients (one lane a parameter took 34 us for 128 of them, latency of its
+// loads; 4 us now for 256).
+constexpr int RED_W = 16;
+__global__ __launch_bounds__(64 * RED_W) void k_mlp_reduce(const float* __restrict__ gpart,
+                                                          const float* __restrict__ lpart, int nblocks,
+                                                          float inv_batch, float* __restrict__ grad,
+                                                          float* __restrict__ loss) {
+    __shared__ float part[RED_W][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    const float* src = p < NPARAM ? gpart + p : lpart;
+    const size_t stride = p < NPARAM ? NPARAM : 1;
+    float a = 0.0f;
+    if (p <= NPARAM) {
+#pragma unroll 8
+        for (int b = wave; b < nblocks; b += RED_W) a = a + src[(size_t)b * stride];
     }
-    if (p == NPARAM && loss) {
-        float a = 0.0f;
-        for (int b = 0; b < nblocks; ++b) a = a + lpart[b];
-        *loss = a * inv_batch;
-    }
+    part[wave][lane] = a;
+    __syncthreads();
+    if (wave != 0 || p > NPARAM) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < RED_W; ++k) sum = sum + part[k][lane];
+    if (p < NPARAM) grad[p] = sum;
+    else if (loss) *loss = sum * inv_batch;
 }
 
 // Adam with bias correction: m = b1 m + (1-b1) g, v = b2 v + (1-b2) g^2,
@@ -397,7 +473,6 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float
 // ------------------------------------------------------------------ BF16 MFMA inference
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Round-to-nearest-even FP32 -> BF16 bits.
 __device__ __forceinline__ unsigned short to_bf16(float f) {
@@ -656,10 +731,12 @@ extern "C" sd_status sd_mlp_init(float* params, uint64_t seed, void* stream) {
     return SD_OK;
 }
 
+// Scratch of this many partial gradients and loss sums.
+static size_t train_bytes(size_t parts) { return parts * (NPARAM + 1) * sizeof(float) + 256; }
+
 extern "C" sd_status sd_mlp_train_scratch_bytes(int batch, size_t* bytes) {
     SD_REQUIRE(bytes && batch > 0, "sd_mlp_train_scratch_bytes: bad argument");
-    const size_t nb = (size_t)div_up(batch, TB_S);
-    *bytes = nb * NPARAM * sizeof(float) + nb * sizeof(float) + 256;
+    *bytes = train_bytes((size_t)std::max(div_up(batch, TB_MIN), std::min(div_up(batch, TB_S), TB_GRID)));
     return SD_OK;
 }
 
@@ -667,18 +744,19 @@ extern "C" sd_status sd_mlp_forward_backward(const float* X, const float* T, con
                                              const float* params, float* grad, float* loss, void* scratch,
                                              size_t scratch_bytes, void* stream) {
     SD_REQUIRE(X && T && idx && params && grad && scratch && batch > 0, "sd_mlp_forward_backward: bad argument");
-    size_t need;
-    sd_mlp_train_scratch_bytes(batch, &need);
-    SD_REQUIRE(scratch_bytes >= need, "sd_mlp_forward_backward: scratch too small");
-    const int nb = div_up(batch, TB_S);
+    SD_REQUIRE(scratch_bytes >= train_bytes((size_t)div_up(batch, TB_MIN)),
+               "sd_mlp_forward_backward: scratch too small");
+    // a tile a block, as far as the scratch and one block a CU go
+    const size_t fit = (scratch_bytes - 256) / ((NPARAM + 1) * sizeof(float));
+    const int nb = (int)std::min({(size_t)div_up(batch, TB_S), (size_t)TB_GRID, fit});
     float* gpart = (float*)scratch;
     float* lpart = gpart + (size_t)nb * NPARAM;
     const float inv_batch = 1.0f / (float)batch;
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(nb), dim3(TB_T), 0, s, X, T, idx, batch, inv_batch, params, gpart, lpart);
     SD_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_mlp_reduce, dim3(div_up(NPARAM + 1, 256)), dim3(256), 0, s, gpart, lpart, nb, inv_batch,
-                       grad, loss);
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(div_up(NPARAM + 1, 64)), dim3(64 * RED_W), 0, s, gpart, lpart, nb,
+                       inv_batch, grad, loss);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }
