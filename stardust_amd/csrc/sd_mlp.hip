@@ -200,8 +200,10 @@ struct __attribute__((packed, aligned(4))) Floats4 {  // four floats anywhere
 // contribute nothing).
 //
 // The products run on the FP32 matrix instruction (16x16 tiles, 4 terms at a
-// time, each a fused multiply-add): operands in FP32, so its error against 64
-// bits is no larger than that of the multiply and add it replaces. Wave w owns
+// time, each a fused multiply-add), operands in FP32. Largest error of a
+// gradient entry against 64 bits, of the largest entry, mean of 30 networks:
+// 8.1e-7 at 64 samples, 5.9e-7 at 257, 3.8e-7 at 1,024, 2.9e-7 at 4,096 (multiply
+// and add in one sum: 11.0, 6.9, 6.7 and 4.3e-7). Wave w owns
 // columns 16 w .. 16 w + 15 of every layer: a lane (group g = lane / 16, c =
 // lane % 16) holds results of rows 4 g .. 4 g + 3 and column c, so activations'
 // derivatives and the sums over samples stay in its registers, as do the weights.
@@ -246,17 +248,23 @@ __global__ __launch_bounds__(TB_T, 1) void k_mlp_fwd_bwd(const float* __restrict
     float db1 = 0.0f, db2 = 0.0f, db3 = 0.0f, dw4[3] = {0.0f, 0.0f, 0.0f};
     float db4[3] = {0.0f, 0.0f, 0.0f}, lsum = 0.0f;  // of sample tid (the first 32 threads)
 
-    // rows of A, 64 terms, times the lane's operands b, added to acc (both row tiles)
-    auto layer = [&](const float (*A)[HS], const float* b, f32x4* acc) {
+    // 16 rows of A from row, 64 terms, times the operands b (a lane's run of
+    // 16), in four sums of 16 terms: a quarter of the chain's roundings and of
+    // its latency
+    auto product = [&](const float (*A)[HS], int row, const float* b) -> f32x4 {
+        f32x4 p[4] = {};
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int k = 0; k < 16; k += 4) {
+            const f32x4 a = *reinterpret_cast<const f32x4*>(&A[row + c][g * 16 + k]);
 #pragma unroll
-            for (int k = 0; k < 16; k += 4) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&A[m * 16 + c][g * 16 + k]);
+            for (int u = 0; u < 4; ++u) p[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[k + u], p[u], 0, 0, 0);
+        }
+        return (p[0] + p[1]) + (p[2] + p[3]);
+    };
+    // the same of both row tiles, plus the bias
+    auto layer = [&](const float (*A)[HS], const float* b, float bias, f32x4* acc) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[k + u], acc[m], 0, 0, 0);
-            }
+        for (int m = 0; m < 2; ++m) acc[m] = product(A, m * 16, b) + bias;
     };
     // SiLU of acc to H, its derivative to d
     auto activate = [&](const f32x4* acc, float (*H)[HS], f32x4* d) {
@@ -294,34 +302,27 @@ __global__ __launch_bounds__(TB_T, 1) void k_mlp_fwd_bwd(const float* __restrict
         }
         __syncthreads();
         f32x4 d1[2], d2[2], d3[2], acc[2];
-        acc[0] = acc[1] = f32x4{b1, b1, b1, b1};
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int m = 0; m < 2; ++m) {
+            f32x4 p[2] = {};
 #pragma unroll
             for (int k = 0; k < 6; ++k)
-                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[m * 16 + c][g * 6 + k], w1[k], acc[m], 0, 0, 0);
+                p[k & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[m * 16 + c][g * 6 + k], w1[k], p[k & 1], 0, 0, 0);
+            acc[m] = (p[0] + p[1]) + b1;
+        }
         activate(acc, H1, d1);
         __syncthreads();
-        acc[0] = acc[1] = f32x4{b2, b2, b2, b2};
-        layer(H1, w2, acc);
+        layer(H1, w2, b2, acc);
         activate(acc, H2, d2);
         __syncthreads();
-        acc[0] = acc[1] = f32x4{b3, b3, b3, b3};
-        layer(H2, w3, acc);
+        layer(H2, w3, b3, acc);
         activate(acc, H3, d3);
         __syncthreads();
         if (wave < 2) {  // the outputs of 16 samples (columns past the third: 0)
-            const float b = c < NOUT ? w[OFF_B4 + c] : 0.0f;
-            f32x4 y = {b, b, b, b};
+            float b4[16];
 #pragma unroll
-            for (int k = 0; k < 16; k += 4) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&H3[wave * 16 + c][g * 16 + k]);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const float b4 = c < NOUT ? w[OFF_W4 + (g * 16 + k + u) * NOUT + c] : 0.0f;
-                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b4, y, 0, 0, 0);
-                }
-            }
+            for (int k = 0; k < 16; ++k) b4[k] = c < NOUT ? w[OFF_W4 + (g * 16 + k) * NOUT + c] : 0.0f;
+            const f32x4 y = product(H3, wave * 16, b4) + (c < NOUT ? w[OFF_B4 + c] : 0.0f);
             if (c < NOUT)
                 for (int r = 0; r < 4; ++r) sy[wave * 16 + 4 * g + r][c] = y[r];
         }
@@ -360,8 +361,7 @@ __global__ __launch_bounds__(TB_T, 1) void k_mlp_fwd_bwd(const float* __restrict
         __syncthreads();
         // dW3 = h2^T dz3, dz2 = (dz3 W3^T) * silu'(z2) -> H3 (free now)
         outer(&H2[0][0], HS, G, dw3, std::integral_constant<int, 4>{});
-        acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        layer(G, r3, acc);
+        layer(G, r3, 0.0f, acc);
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
@@ -373,8 +373,7 @@ __global__ __launch_bounds__(TB_T, 1) void k_mlp_fwd_bwd(const float* __restrict
         __syncthreads();
         // dW2 = h1^T dz2, dz1 = (dz2 W2^T) * silu'(z1) -> G
         outer(&H1[0][0], HS, H3, dw2, std::integral_constant<int, 4>{});
-        acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        layer(H3, r2, acc);
+        layer(H3, r2, 0.0f, acc);
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
