@@ -392,7 +392,7 @@ def clump_section(args):
             "ms_per_step": round(ms, 4), "sphere_steps_per_s": sc.ns / (ms / 1000.0),
             "body_steps_per_s": sc.nb / (ms / 1000.0), "stage_ms": {k: round(v, 4) for k, v in per.items()},
             "broadphase_pairs": npairs,
-            "form": "graph-replayed step pairs; partners found in the LBVH inside the contact kernel"}
+            "form": "graph-replayed step pairs; partners from lists, found in the LBVH by the steps that build them"}
 
 
 def batch_section(args):

@@ -43,18 +43,6 @@ constexpr int HB_FEATURE_BATCH = 8;
 // nearer ones are redone cold.
 constexpr float HB_WARM_NEAR_MARGIN = 1e-6f;
 
-__global__ void k_hb_pose(const float4* __restrict__ P, const float4* __restrict__ Q, const float4* __restrict__ L,
-                          const float4* __restrict__ I0, const float4* __restrict__ I1,
-                          const float* __restrict__ radius, int n, float4* __restrict__ spos,
-                          float4* __restrict__ omega) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n) return;
-    const float4 p = P[b], l = L[b];
-    spos[b] = make_float4(p.x, p.y, p.z, radius[b]);
-    const V3 w = inv_inertia_apply(quat_rot(Q[b]), I0[b], I1[b], v3(l.x, l.y, l.z));
-    omega[b] = make_float4(w.x, w.y, w.z, 0.0f);
-}
-
 // Support-feature tolerance of every body: HB_FEATURE_REL times its radius
 // (largest vertex distance from its centre); 0 for a sphere. Fixed at upload.
 __global__ void k_hb_feature_tol(const float4* __restrict__ verts, const int* __restrict__ vstart,
@@ -163,18 +151,24 @@ __device__ __forceinline__ int hb_cell_axis(float x, float lo, float inv, int nd
     return (int)fminf(fmaxf(floorf((x - lo) * inv), 0.0f), (float)(nd - 1));
 }
 
-// key = (global cell of the body's centre) << 32 | body index; a large body
-// (bucketed in its scene's second grid at upload) takes cell ncells, past
-// every scene's cells of the first grids
-__global__ void k_hb_cell_keys(const float4* __restrict__ P, const int* __restrict__ scene_of,
-                               const HbGrid* __restrict__ grid, const int* __restrict__ large, int n, int ncells,
-                               uint64_t* __restrict__ keys) {
+// Also the body's sort key (global cell of its centre) << 32 | body index; a
+// large body (bucketed in its scene's second grid at upload) takes cell ncells,
+// past every scene's cells of the first grids.
+__global__ void k_hb_pose(const float4* __restrict__ P, const float4* __restrict__ Q, const float4* __restrict__ L,
+                          const float4* __restrict__ I0, const float4* __restrict__ I1,
+                          const float* __restrict__ radius, int n, float4* __restrict__ spos,
+                          float4* __restrict__ omega, const int* __restrict__ scene_of,
+                          const HbGrid* __restrict__ grid, const int* __restrict__ large, int ncells,
+                          uint64_t* __restrict__ keys) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= n) return;
+    const float4 p = P[b], l = L[b];
+    spos[b] = make_float4(p.x, p.y, p.z, radius[b]);
+    const V3 w = inv_inertia_apply(quat_rot(Q[b]), I0[b], I1[b], v3(l.x, l.y, l.z));
+    omega[b] = make_float4(w.x, w.y, w.z, 0.0f);
     uint32_t cell = (uint32_t)ncells;
     if (!large[b]) {
         const HbGrid g = grid[scene_of[b]];
-        const float4 p = P[b];
         const int cx = hb_cell_axis(p.x, g.lox, g.inv, g.nx);
         const int cy = hb_cell_axis(p.y, g.loy, g.inv, g.ny);
         const int cz = hb_cell_axis(p.z, g.loz, g.inv, g.nz);
@@ -210,6 +204,11 @@ struct HbGridArgs {
 // the same or neighbouring cells, so each such pair is found once, from the
 // body whose cell comes first. Pair k goes to emit(k, lo, hi); returns the
 // count.
+//
+// Bound by the chain of loads (a wave or so per SIMD at tens of thousands of
+// bodies): windows of all rows together, candidates HB_WALK at a time; 64,000
+// bodies 20 us, 35 one candidate after the other.
+constexpr int HB_WALK = 4;
 template <typename Emit>
 __device__ __forceinline__ int hb_grid_walk(const HbGridArgs& G, int a, Emit emit) {
     const HbGrid g = G.grid[G.scene_of[a]];
@@ -222,26 +221,40 @@ __device__ __forceinline__ int hb_grid_walk(const HbGridArgs& G, int a, Emit emi
     // the stencil's rows (dz, dy) in order; a row's cells are consecutive in
     // the sorted keys, so each row is one window of positions: from a's own
     // cell (the bodies after a) for the first row, x - 1 .. x + 1 (clamped)
-    // for the others
-    for (int dz = 0; dz <= 1; ++dz) {
-        const int z = cz + dz;
-        if (z >= g.nz) continue;
-        for (int dy = -1; dy <= 1; ++dy) {
-            const int y = cy + dy;
-            if (y < 0 || y >= g.ny || (dz == 0 && dy < 0)) continue;
-            const bool own_row = dz == 0 && dy == 0;
-            const int x0 = own_row ? cx : max(cx - 1, 0), x1 = min(cx + 1, g.nx - 1);
-            const int row = g.cbase + (z * g.ny + y) * g.nx;
-            const int t0 = G.cell_start[row + x0], t1 = G.cell_start[row + x1 + 1];
-            const int own_end = own_row ? G.cell_start[row + cx + 1] : t0;  // a's own cell: [t0, own_end)
-            for (int t = t0; t < t1; ++t) {
-                const int b = (int)(uint32_t)G.sorted[t];
-                if (t < own_end && b <= a) continue;
-                if (sa && G.P[b].w == 0.0f) continue;
-                const float4 lb = G.lo[b], hb = G.hi[b];
-                if (!(lb.x <= ha.x && la.x <= hb.x && lb.y <= ha.y && la.y <= hb.y && lb.z <= ha.z && la.z <= hb.z))
-                    continue;
-                emit(k++, min(a, b), max(a, b));
+    // for the others. The windows of all rows are loaded together (a row
+    // outside the grid: a's own, then emptied).
+    int t0[5], t1[5];
+    const int x1 = min(cx + 1, g.nx - 1);
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+        const int z = r < 2 ? cz : cz + 1, y = r < 2 ? cy + r : cy + r - 3;
+        const bool in = z < g.nz && y >= 0 && y < g.ny;
+        const int row = g.cbase + ((in ? z : cz) * g.ny + (in ? y : cy)) * g.nx;
+        t0[r] = G.cell_start[row + (r == 0 ? cx : max(cx - 1, 0))];
+        t1[r] = G.cell_start[row + x1 + 1];
+        if (!in) t1[r] = t0[r];
+    }
+    const int own_end = G.cell_start[g.cbase + (cz * g.ny + cy) * g.nx + cx + 1];  // a's own cell: [t0[0], own_end)
+    auto overlaps = [&](const float4& lb, const float4& hb) {
+        return lb.x <= ha.x && la.x <= hb.x && lb.y <= ha.y && la.y <= hb.y && lb.z <= ha.z && la.z <= hb.z;
+    };
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+        for (int t = t0[r]; t < t1[r]; t += HB_WALK) {
+            int b[HB_WALK];
+            float4 lb[HB_WALK], hb[HB_WALK];
+#pragma unroll
+            for (int u = 0; u < HB_WALK; ++u) b[u] = (int)(uint32_t)G.sorted[min(t + u, t1[r] - 1)];
+#pragma unroll
+            for (int u = 0; u < HB_WALK; ++u) {
+                lb[u] = G.lo[b[u]];
+                hb[u] = G.hi[b[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < HB_WALK; ++u) {
+                if (t + u >= t1[r] || (r == 0 && t + u < own_end && b[u] <= a)) continue;
+                if (!overlaps(lb[u], hb[u]) || (sa && G.P[b[u]].w == 0.0f)) continue;
+                emit(k++, min(a, b[u]), max(a, b[u]));
             }
         }
     }
@@ -250,21 +263,22 @@ __device__ __forceinline__ int hb_grid_walk(const HbGridArgs& G, int a, Emit emi
     const int qy = hb_cell_axis(pa.y, g.lloy, g.linv, g.lny);
     const int qz = hb_cell_axis(pa.z, g.lloz, g.linv, g.lnz);
     const int qx0 = max(qx - 1, 0), qx1 = min(qx + 1, g.lnx - 1);
-    for (int dz = -1; dz <= 1; ++dz) {
-        const int z = qz + dz;
-        if (z < 0 || z >= g.lnz) continue;
-        for (int dy = -1; dy <= 1; ++dy) {
-            const int y = qy + dy;
-            if (y < 0 || y >= g.lny) continue;
-            const int row = g.lcbase + (z * g.lny + y) * g.lnx;
-            const int t1 = G.lstart[row + qx1 + 1];
-            for (int t = G.lstart[row + qx0]; t < t1; ++t) {
-                const int b = G.llist[t];
-                const float4 lb = G.lo[b], hb = G.hi[b];
-                if (!(lb.x <= ha.x && la.x <= hb.x && lb.y <= ha.y && la.y <= hb.y && lb.z <= ha.z && la.z <= hb.z))
-                    continue;
-                emit(k++, min(a, b), max(a, b));
-            }
+    int u0[9], u1[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const int z = qz + r / 3 - 1, y = qy + r % 3 - 1;
+        const bool in = z >= 0 && z < g.lnz && y >= 0 && y < g.lny;
+        const int row = g.lcbase + ((in ? z : qz) * g.lny + (in ? y : qy)) * g.lnx;
+        u0[r] = G.lstart[row + qx0];
+        u1[r] = G.lstart[row + qx1 + 1];
+        if (!in) u1[r] = u0[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        for (int t = u0[r]; t < u1[r]; ++t) {
+            const int b = G.llist[t];
+            if (!overlaps(G.lo[b], G.hi[b])) continue;
+            emit(k++, min(a, b), max(a, b));
         }
     }
     return k;
@@ -272,9 +286,13 @@ __device__ __forceinline__ int hb_grid_walk(const HbGridArgs& G, int a, Emit emi
 
 // One thread per body: its pair count (0 for a large body, which pairs only
 // through the gridded bodies) and its first HB_GRID_SLOTS pairs in its slots.
-__global__ void k_hb_grid_pairs(HbGridArgs G, int n, int* __restrict__ cnt, int2* __restrict__ slots) {
+// Also clears the step's contact counters, body by body (two launches less).
+__global__ void k_hb_grid_pairs(HbGridArgs G, int n, int* __restrict__ cnt, int2* __restrict__ slots,
+                                int* __restrict__ contacts, int* __restrict__ filled) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= n) return;
+    contacts[a] = 0;
+    filled[a] = 0;
     if (G.large[a]) {
         cnt[a] = 0;
         return;
@@ -557,16 +575,13 @@ sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s) {
     const int mi = c->p.max_iter ? c->p.max_iter : 64;
     hipLaunchKernelGGL(k_hb_pose, dim3(div_up(n, 256)), dim3(256), 0, s, (const float4*)c->P, (const float4*)c->Q,
                        (const float4*)c->L, (const float4*)c->I0, (const float4*)c->I1, (const float*)c->radius, n,
-                       c->spos, c->omega);
+                       c->spos, c->omega, (const int*)c->scene_of, (const HbGrid*)c->grid, (const int*)c->large,
+                       (int)c->ncells, c->gkeys);
     SD_LAUNCH_CHECK();
     sd_status st = launch_hull_aabbs(c->spos, c->Q, c->vstart, c->nv, c->verts, n, c->lo, c->hi, s);
     if (st != SD_OK) return st;
     // candidate pairs: bodies sorted by grid cell (index order within a
     // cell), cell starts, then per body its count, the offsets and the pairs
-    hipLaunchKernelGGL(k_hb_cell_keys, dim3(div_up(n, 256)), dim3(256), 0, s, (const float4*)c->P,
-                       (const int*)c->scene_of, (const HbGrid*)c->grid, (const int*)c->large, n, (int)c->ncells,
-                       c->gkeys);
-    SD_LAUNCH_CHECK();
     uint64_t *K = c->gkeys, *Ka = c->gkeys2;
     int cbits = 1;  // cell ids run to ncells (the bodies kept out of the grids)
     while (cbits < 32 && (1ll << cbits) <= c->ncells) ++cbits;
@@ -579,7 +594,8 @@ sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s) {
                        (const int*)c->scene_of, (const HbGrid*)c->grid,   (const int*)c->large,
                        (const int*)c->llist,    (const int*)c->lstart,    (const uint64_t*)K,
                        (const int*)c->cell_start};
-    hipLaunchKernelGGL(k_hb_grid_pairs, dim3(div_up(n, 256)), dim3(256), 0, s, G, n, c->gcnt, c->gslots);
+    hipLaunchKernelGGL(k_hb_grid_pairs, dim3(div_up(n, 256)), dim3(256), 0, s, G, n, c->gcnt, c->gslots,
+                       c->cnt, c->fillc);
     SD_LAUNCH_CHECK();
     st = exclusive_scan_i32(c->gcnt, c->goff, n, c->goff + n, c->scan_tmp, s);
     if (st != SD_OK) return st;
@@ -596,9 +612,6 @@ sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s) {
         st = enqueue_gjk_cold(c->pairs, cap, c->total, c->spos, c->Q, c->vstart, c->nv, c->verts, n, c->n_verts, mi,
                               0.0f, c->sep, c->normal, c->flags, c->iters, c->gjk_scratch, s);
     }
-    if (st != SD_OK) return st;
-    st = launch_fill_u32((uint32_t*)c->cnt, 0u, n, s);
-    if (st == SD_OK) st = launch_fill_u32((uint32_t*)c->fillc, 0u, n, s);
     if (st != SD_OK) return st;
     const HbBodies B{c->P, c->V, c->Q, c->omega, c->radius, c->ftol, c->vstart, c->nv, c->verts};
     hipLaunchKernelGGL(k_hb_pairs, dim3(div_up(cap, 256)), dim3(256), 0, s, (const int*)c->pairs, cap,
