@@ -84,6 +84,9 @@ constexpr int DENSE_CHUNK = 16;
 // Steps run between two looks at how long the near lists last, or whether they
 // would do.
 constexpr int LIST_REST = 64;
+// The same with rigid bodies attached: what a given-up sequence has computed for
+// the bodies is lost, and a body step (0.5 ms and more) is long against the look.
+constexpr int BODY_CHUNK = 16;
 
 }  // namespace sd
 
@@ -169,7 +172,7 @@ struct sd_ctx {
     bool persistent = false;
     int* pcounters = nullptr;
     hipStream_t hside = nullptr;
-    hipEvent_t hev_fork = nullptr, hev_join = nullptr;
+    hipEvent_t hev_fork = nullptr, hev_sorted = nullptr, hev_join = nullptr;
     HostStage stage;  // pinned staging of the read-backs
 };
 
@@ -261,13 +264,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev, bool full, int lists) {
     a.ids_o = c->ids[sn];
     sd_status st;
     MARK(0);
-    if (c->hulls) {  // the rigid-body scenes' step runs beside the sphere step
-        SD_HIP(hipEventRecord(c->hev_fork, s));
-        SD_HIP(hipStreamWaitEvent(c->hside, c->hev_fork, 0));
-        st = hull_enqueue_step(c->hulls, c->hside);
-        if (st != SD_OK) return st;
-        SD_HIP(hipEventRecord(c->hev_join, c->hside));
-    }
+    if (c->hulls) SD_HIP(hipEventRecord(c->hev_fork, s));
     // sorted keys: the radix sort (full), or the re-sort from the previous
     // order and the spheres that changed cell, with the positions permuted
     // in the same pass. Either leaves them in the other key buffer.
@@ -290,6 +287,16 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev, bool full, int lists) {
     }
     if (st != SD_OK) return st;
     MARK(1);
+    // The rigid-body scenes' step runs beside the sphere step; the bodies are
+    // moved when it is known that the sphere step is not given up, so that
+    // both have made the same steps.
+    if (c->hulls) {
+        SD_HIP(hipEventRecord(c->hev_sorted, s));
+        SD_HIP(hipStreamWaitEvent(c->hside, c->hev_fork, 0));
+        st = hull_enqueue_step(c->hulls, c->hside, c->hev_sorted, &c->ctl->given_up);
+        if (st != SD_OK) return st;
+        SD_HIP(hipEventRecord(c->hev_join, c->hside));
+    }
     // after the full sort: cell starts, the permutation, mc_write = 0
     if (full) st = launch_step_starts_u64(K, n, c->n_cells, c->cell_start, &c->ctl->given_up, true, c->pos[so],
                                           c->posB, mc_write, nullptr, c->ctl, lists, c->list_cell, s);
@@ -385,8 +392,8 @@ int list_life(float displaced, float sigma, float last) {
 
 // Whether near lists pay at the scene's speed: not where even the largest
 // margin would last fewer than 4 steps, nor in dense runs (whose spheres cross
-// cells). Steps with rigid bodies attached keep none: a given-up sphere step
-// would not take the bodies' step back.
+// cells). Steps with rigid bodies attached keep none: the bodies' part of a
+// given-up step would be computed twice.
 bool lists_pay(const sd_ctx* c) {
     return !c->dense && !c->hulls && c->list_cell > 0.0f && 8.0f * c->last_move <= LIST_MAX * c->list_cell;
 }
@@ -421,7 +428,8 @@ sd_status run_steps(sd_ctx* c, int nsteps) {
             // full-sort steps: one after a given-up step or an upload, DENSE_CHUNK
             // of them while the scene is dense, before the changed-cell count is
             // read again
-            rest = full ? (c->dense ? std::min(left, DENSE_CHUNK) : 1) : std::min(left, LIST_REST);
+            rest = full ? (c->dense ? std::min(left, DENSE_CHUNK) : 1)
+                        : std::min(left, c->hulls ? BODY_CHUNK : LIST_REST);
             st = run(rest, full, LIST_NONE);
             c->list_steps = 0;
         } else {
@@ -537,6 +545,7 @@ extern "C" sd_status sd_batch_attach_hulls(sd_ctx* c, sd_hull_ctx* h) {
         if (!c->hside) {
             SD_HIP(hipStreamCreateWithFlags(&c->hside, hipStreamNonBlocking));
             SD_HIP(hipEventCreateWithFlags(&c->hev_fork, hipEventDisableTiming));
+            SD_HIP(hipEventCreateWithFlags(&c->hev_sorted, hipEventDisableTiming));
             SD_HIP(hipEventCreateWithFlags(&c->hev_join, hipEventDisableTiming));
         }
     }
@@ -552,6 +561,7 @@ extern "C" sd_status sd_ctx_destroy(sd_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->hside) (void)hipStreamSynchronize(c->hside);
     if (c->hev_fork) (void)hipEventDestroy(c->hev_fork);
+    if (c->hev_sorted) (void)hipEventDestroy(c->hev_sorted);
     if (c->hev_join) (void)hipEventDestroy(c->hev_join);
     if (c->hside) (void)hipStreamDestroy(c->hside);
     if (c->pcounters) (void)hipFree(c->pcounters);

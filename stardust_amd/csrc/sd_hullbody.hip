@@ -408,13 +408,16 @@ __global__ void k_hb_fill(const int* __restrict__ pairs, int capacity, const int
 // ascending entry order (f = +pf on b, -pf on a), then the integration step.
 // A static body has no listed contacts (F = T = 0) and is left as it is: a
 // wall triangle under a whole layer of hulls would otherwise order thousands
-// of entries on one thread.
-__global__ void k_hb_gather_integrate(int n, const int* __restrict__ offs, const int* __restrict__ cnt,
+// of entries on one thread. The only kernel of a step that changes the bodies'
+// state: with *given_up (nullable) it changes nothing, and the step can be
+// made again.
+__global__ void k_hb_gather_integrate(const int* __restrict__ given_up, int n, const int* __restrict__ offs, const int* __restrict__ cnt,
                                       const int* __restrict__ list, const float4* __restrict__ pf,
                                       const float4* __restrict__ pp, float4* __restrict__ P, float4* __restrict__ V,
                                       float4* __restrict__ Q, float4* __restrict__ L, const float4* __restrict__ I0,
                                       const float4* __restrict__ I1, ContactDev c, float4* __restrict__ fout,
                                       float4* __restrict__ tout) {
+    if (given_up && *given_up) return;
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= n) return;
     float4 X = P[b];
@@ -570,7 +573,7 @@ sd_status hb_check_params(const sd_hull_params* p) {
 namespace sd {
 
 // One step of the context, enqueued on s (no host synchronisation).
-sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s) {
+sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s, hipEvent_t ready, const int* given_up) {
     const int n = c->n, cap = c->capacity;
     const int mi = c->p.max_iter ? c->p.max_iter : 64;
     hipLaunchKernelGGL(k_hb_pose, dim3(div_up(n, 256)), dim3(256), 0, s, (const float4*)c->P, (const float4*)c->Q,
@@ -624,9 +627,11 @@ sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s) {
                        (const int*)c->total, (const float4*)c->P, (const float4*)c->pf, (const int*)c->offs, c->fillc,
                        c->list);
     SD_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_hb_gather_integrate, dim3(div_up(n, 256)), dim3(256), 0, s, n, (const int*)c->offs,
-                       (const int*)c->cnt, (const int*)c->list, (const float4*)c->pf, (const float4*)c->pp, c->P,
-                       c->V, c->Q, c->L, (const float4*)c->I0, (const float4*)c->I1, c->c, c->F, c->T);
+    if (ready) SD_HIP(hipStreamWaitEvent(s, ready, 0));
+    hipLaunchKernelGGL(k_hb_gather_integrate, dim3(div_up(n, 256)), dim3(256), 0, s, given_up, n,
+                       (const int*)c->offs, (const int*)c->cnt, (const int*)c->list, (const float4*)c->pf,
+                       (const float4*)c->pp, c->P, c->V, c->Q, c->L, (const float4*)c->I0, (const float4*)c->I1, c->c,
+                       c->F, c->T);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }

@@ -315,6 +315,67 @@ def test_batch_checkpoint_resume_and_scene_table_check():
     d.close()
 
 
+def fast_scenes(scale, speed, seed=43):
+    """Scenes of spheres that change cell often: (scenes, arrays)."""
+    from stardust_amd import _lib as L
+    rng = np.random.default_rng(seed)
+    scenes, cols = [], {k: [] for k in ("x", "y", "z", "r", "m", "vx", "vy", "vz")}
+    for n, box, r, org in ((1500, 0.2, 0.004, (0.0, 0.0, 0.0)), (2000, 0.25, 0.005, (-3.0, 0.0, 0.0))):
+        n, box = int(n * scale), box * scale ** (1.0 / 3.0)
+        lo = np.array(org, np.float32)
+        pos = (lo + rng.uniform(r, box - r, (n, 3))).astype(np.float32)
+        rad = rng.uniform(0.5 * r, r, n).astype(np.float32)
+        vel = rng.normal(0, speed, (n, 3)).astype(np.float32)
+        nc = int(math.ceil(box / (2 * r)))
+        walls = (tuple(float(v) for v in lo), tuple(float(v) + box for v in lo))
+        scenes.append((n, L.Grid.make(walls[0], 2 * r, (nc, nc, nc)),
+                       L.ContactParams.make(1e5, 0.3, 0.5, 2e-6, gravity=(0.0, 0.0, -9.81), walls=walls,
+                                            max_contacts=32)))
+        for k, a in (("x", pos[:, 0]), ("y", pos[:, 1]), ("z", pos[:, 2]), ("r", rad), ("m", W.sphere_mass(rad)),
+                     ("vx", vel[:, 0]), ("vy", vel[:, 1]), ("vz", vel[:, 2])):
+            cols[k].append(np.ascontiguousarray(a))
+    return scenes, {k: np.concatenate(v) for k, v in cols.items()}
+
+
+# about 1,024 changed cells a step, the most a re-sort takes (some steps of a
+# call are given up and made again), and many more (the first is)
+@pytest.mark.parametrize("scale,graph", [(4.0, True), (4.0, False), (3.8, True), (8.0, True)])
+def test_attached_bodies_and_given_up_steps(scale, graph):
+    """Bodies attached to scenes whose re-sorts are given up make as many steps
+    as the spheres: both equal their own contexts stepped alone, bit for bit."""
+    say("attached bodies, given-up re-sorts", scale, graph)
+    from stardust_amd import _lib as L
+    from stardust_amd import hullbody as HB
+    from stardust_amd import hulls as H
+    scenes, s = fast_scenes(scale, 150.0)
+    v = [s["vx"], s["vy"], s["vz"]]
+    h = H.generate_hulls(0x4C40, 200, lo=(0.0, 0.0, 0.0), hi=(0.1, 0.1, 0.1), v_sigma=2.0)
+    bodies, first = HB.concat([HB.make_bodies(h, 0x4C41)])
+    c = L.ContactParams.make(2e4, 0.3, 0.5, 2e-6, gravity=(0.0, 0.0, -9.81), walls=None, max_contacts=16)
+    a, b = batch_of(None, scenes, s, v, use_graph=graph), batch_of(None, scenes, s, v)
+    ha, hb = HB.HullBodyScene(c), HB.HullBodyScene(c)
+    ha.upload(bodies, first)
+    hb.upload(bodies, first)
+    a.attach_hulls(ha)
+    changes = []
+    for k in (5, 20, 37):
+        a.step(k)
+        for _ in range(k):
+            b.step(1)
+            changes.append(b.cell_changes()[0])
+        hb.step(k)
+        assert_same(a.download(), b.download(), "spheres with bodies attached")
+        ga, gb = ha.download(), hb.download()
+        for key in ("pos4", "vel4", "quat4", "angm4"):
+            assert np.array_equal(ga[key], gb[key]), (key, k)
+        assert np.array_equal(ha.contacts()[0], hb.contacts()[0])
+    say("changed cells per step", min(changes), max(changes))
+    assert max(changes) > 1024 and (scale > 5.0 or min(changes) <= 1024)
+    a.attach_hulls(None)
+    for x in (a, b, ha, hb):
+        x.close()
+
+
 def test_batch_steps_attached_hull_scenes(warm_model):
     """sd_batch_attach_hulls: the rigid-body scenes step inside the batched
     step (graph-captured, forked stream); afterwards the spheres equal the
