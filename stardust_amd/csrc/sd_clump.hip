@@ -32,6 +32,7 @@
 #include "sd_contact_law.hpp"
 #include "sd_gjk_dev.hpp"
 #include "sd_internal.hpp"
+#include "sd_list_plan.hpp"
 #include "sd_rigid_dev.hpp"
 
 extern "C" sd_status sd_global_domain(const float* lo4, const float* hi4, int n, float* domain6, void* scratch,
@@ -77,12 +78,6 @@ struct ClumpCtl {
     uint32_t dmax[2][LIST_SLOTS * 16];  // by parity: face movements of the step (float bits)
 };
 constexpr int CLUMP_CTL_READ = 9;
-// The margin lasts 40 steps of the last movement, within these shares of the
-// mean body size.
-constexpr float CL_MARGIN_STEPS = 40.0f, CL_MARGIN_MIN = 0.005f, CL_MARGIN_MAX = 0.05f;
-inline float clump_margin(float last, float size) {
-    return fminf(fmaxf(CL_MARGIN_STEPS * last, CL_MARGIN_MIN * size), CL_MARGIN_MAX * size);
-}
 
 // Largest face movement of the step, by a whole wave.
 __device__ __forceinline__ float step_movement(const uint32_t* dmax) {
@@ -103,9 +98,9 @@ __global__ __launch_bounds__(64) void k_clump_margin(ClumpCtl* __restrict__ ctl,
     if (threadIdx.x != 0) return;
     float far = 0.0f;
     for (int k = 0; k < 6; ++k) far = fmaxf(far, fabsf(domain[k]));
-    const float margin = fminf(fmaxf(CL_MARGIN_STEPS * m, CL_MARGIN_MIN * size), CL_MARGIN_MAX * size);
+    const float margin = clump_build_margin(m, size, far);
     ctl->margin = margin;
-    ctl->limit = 0.98f * margin - 5e-7f * (far + margin);
+    ctl->limit = clump_limit(margin, far);
     ctl->over = 0;
 }
 
@@ -506,10 +501,7 @@ struct sd_clump_ctx {
     uint8_t* lcount = nullptr;
     int* list = nullptr;
     float size = 0.0f;        // mean extent of the bodies
-    int list_steps = 0;       // steps the lists are expected to last (0: build them next)
-    int list_rest = 0;        // steps to run without lists before they are tried again
-    float last_move = -1.0f;  // as last read back (negative: not known)
-    bool crowded = false;     // the last lists did not hold some body's partners
+    ListPlan plan;
     bool boxes = false;       // blo / bhi are those of the step before
     long long steps_done = 0;
     uint64_t static_hash = 0;  // of the fixed rows (inverse inertia, sphere ranges and offsets)
@@ -647,10 +639,7 @@ sd_status clump_step(sd_clump_ctx* c, hipEvent_t* ev, int lists) {
 
 // A changed state (upload, load): no lists, and the boxes say nothing about how far bodies move.
 sd_status clump_forget_lists(sd_clump_ctx* c) {
-    c->list_steps = 0;
-    c->list_rest = 0;
-    c->last_move = -1.0f;
-    c->crowded = false;
+    c->plan = ListPlan();
     c->boxes = false;
     return launch_fill_u32((uint32_t*)c->ctl, 0u, sizeof(ClumpCtl) / 4, c->stream);
 }
@@ -981,18 +970,11 @@ static sd_status clump_graph_pair(sd_clump_ctx* c, int lists) {
     return SD_OK;
 }
 
-// Steps between two looks at how long the lists last, or whether they would do.
-constexpr int CL_REST = 64;
-
-// Steps that lists are expected to last, a tenth short of what the last movement says.
-static int clump_list_life(float displaced, float limit, float last) {
-    const float steps = 0.9f * (limit - displaced) / fmaxf(last, 1e-30f);
-    return steps >= (float)CL_REST ? CL_REST : (steps > 0.0f ? (int)steps : 0);  // (not a number: 0)
-}
-
-// Whether lists pay at the bodies' speed: not where the largest margin would last fewer than 4 steps.
-static bool clump_lists_pay(const sd_clump_ctx* c) {
-    return c->size > 0.0f && 4.0f * c->last_move <= CL_MARGIN_MAX * c->size;
+// The next launch sequence of at most `left` steps.
+static ListRun clump_next(sd_clump_ctx* c, int left) {
+    const float largest = clump_largest(c->size);
+    return c->plan.next(left, c->size > 0.0f && c->plan.pays(largest), false, largest,
+                        CL_MARGIN_KEPT * clump_margin(c->plan.last, c->size));
 }
 
 // What a launch sequence left: the steps that ran set the buffer parity, the
@@ -1005,19 +987,15 @@ static sd_status clump_read_ctl(sd_clump_ctx* c, int cur0, int limit, bool use, 
         return set_error(SD_ERR_STATE, "sd_clump_step: %d of %d steps ran", ctl.ran, limit);
     *ran = ctl.ran;
     c->cur = cur0 ^ (ctl.ran & 1);
-    c->last_move = isfinite(ctl.last) ? ctl.last : 3.4e38f;
-    // the movement of the step to come is not in yet: count it as the last one
-    c->list_steps = ctl.given_up ? 0 : clump_list_life(ctl.displaced[c->cur] + ctl.last, ctl.limit, ctl.last);
-    if (use) {
-        c->crowded = ctl.over != 0;
-        if (c->crowded) {
-            c->list_steps = 0;
-            c->list_rest = 4 * CL_REST;
-        }
-    } else {
-        c->list_steps = 0;
-        c->list_rest = std::max(0, c->list_rest - ctl.ran);
-    }
+    ListReport r;
+    r.ran = ctl.ran;
+    r.given_up = ctl.given_up != 0;
+    r.crowded = ctl.over != 0;
+    r.last = ctl.last;
+    r.budget = ctl.limit;
+    r.used = ctl.displaced[c->cur];
+    r.lost = CL_MARGIN_KEPT * ctl.margin - ctl.limit;
+    c->plan.read(r, use, clump_largest(c->size));
     if (ctl.error) return set_error(SD_ERR_STATE, "sd_clump_step: malformed tree (error bits %d)", ctl.error);
     return SD_OK;
 }
@@ -1037,26 +1015,19 @@ extern "C" sd_status sd_clump_step(sd_clump_ctx* c, int nsteps) {
         sd_status st = launch_fill_u32((uint32_t*)c->ctl, 0u, 3, c->stream);  // given_up, ran, error
         if (st != SD_OK) return st;
         const int cur0 = c->cur;
-        const bool use = clump_lists_pay(c) && c->list_rest == 0;
+        const ListRun next = clump_next(c, left);
+        const bool use = next.none == 0;
         if (!use) {
             // the first step's boxes are compared with none, so never one of a captured pair
-            int l = std::min(left, CL_REST);
+            int l = next.none;
             if (!c->boxes) {
                 st = clump_step(c, nullptr, LIST_NONE);
                 --l;
             }
             if (st == SD_OK) st = run(l, LIST_NONE);
         } else {
-            int l = left;
-            if (c->list_steps < std::min(left, 2)) {
-                st = clump_step(c, nullptr, LIST_BUILD);
-                // (of unknown speed, or too full for lists the last time: a look first)
-                c->list_steps = c->crowded || c->last_move < 0.0f
-                                    ? 2
-                                    : clump_list_life(0.0f, 0.98f * clump_margin(c->last_move, c->size), c->last_move);
-                --l;
-            }
-            if (st == SD_OK) st = run(std::min(l, c->list_steps), LIST_USE);
+            if (next.build) st = clump_step(c, nullptr, LIST_BUILD);
+            if (st == SD_OK) st = run(next.use, LIST_USE);
         }
         if (st != SD_OK) return st;
         int ran = 0;
@@ -1081,8 +1052,9 @@ extern "C" sd_status sd_clump_profile(sd_clump_ctx* c, int nsteps, float* stage_
     for (int i = 0; i < nsteps && st == SD_OK; ++i) {
         // the lists as a run would use them, the step redone if they ran out
         const int cur0 = c->cur;
-        const bool use = clump_lists_pay(c);
-        const int lists = !use ? LIST_NONE : (c->list_steps < 1 || c->crowded ? LIST_BUILD : LIST_USE);
+        const ListRun next = clump_next(c, 1);
+        const bool use = next.none == 0;
+        const int lists = !use ? LIST_NONE : (next.build ? LIST_BUILD : LIST_USE);
         st = launch_fill_u32((uint32_t*)c->ctl, 0u, 3, c->stream);
         if (st == SD_OK) st = clump_step(c, ev, lists);
         if (st != SD_OK) break;

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "sd_internal.hpp"
+#include "sd_list_plan.hpp"
 #include "sd_readback.hpp"
 
 namespace sd {
@@ -81,10 +82,7 @@ struct GraphKey {
 // Full-sort steps run between two reads of the changed-cell count while a
 // scene is dense (more changed cells per step than the re-sort takes).
 constexpr int DENSE_CHUNK = 16;
-// Steps run between two looks at how long the near lists last, or whether they
-// would do.
-constexpr int LIST_REST = 64;
-// The same with rigid bodies attached: what a given-up sequence has computed for
+// Steps between two looks with rigid bodies attached: what a given-up sequence has computed for
 // the bodies is lost, and a body step (0.5 ms and more) is long against the look.
 constexpr int BODY_CHUNK = 16;
 
@@ -136,10 +134,7 @@ struct sd_ctx {
     float list_cell = 0.0f;  // smallest cell edge; 0: no lists (spheres larger than their cell)
     float rmax = 0.0f;
     float* scene_rmax = nullptr;
-    int list_steps = 0;     // steps that the lists are expected to last (0: build them next)
-    int list_rest = 0;      // steps to run without lists before they are tried again
-    float last_move = -1.0f; // largest displacement of a step, as last read back (negative: not known)
-    bool crowded = false;    // the last lists did not hold some sphere's neighbours
+    ListPlan plan;
     int last_ovf = 0;        // StepCtl::overflow as last read back
     bool need_full = true;  // the next step's keys are not from a step of this order
     bool dense = false;     // the last full-sort step had more changed cells than the re-sort takes
@@ -382,20 +377,31 @@ sd_status run_graph_pair(sd_ctx* c, bool full, int lists) {
     return SD_OK;
 }
 
-// Steps that lists of margin sigma are expected to last from `displaced` on, a
-// tenth short of what the last displacement says (a shortfall costs a given-up
-// launch sequence, a surplus a build a few steps early).
-int list_life(float displaced, float sigma, float last) {
-    const float steps = 0.9f * (0.49f * sigma - displaced) / fmaxf(last, 1e-30f);
-    return steps >= (float)LIST_REST ? LIST_REST : (steps > 0.0f ? (int)steps : 0);  // (not a number: 0)
-}
+// Displacement that the widest near lists allow.
+float list_largest(const sd_ctx* c) { return LIST_KEPT * LIST_MAX * c->list_cell; }
 
-// Whether near lists pay at the scene's speed: not where even the largest
-// margin would last fewer than 4 steps, nor in dense runs (whose spheres cross
-// cells). Steps with rigid bodies attached keep none: the bodies' part of a
+// Whether near lists pay: at the scene's speed, and not in dense runs (whose
+// spheres cross cells). Steps with rigid bodies attached keep none: the bodies' part of a
 // given-up step would be computed twice.
 bool lists_pay(const sd_ctx* c) {
-    return !c->dense && !c->hulls && c->list_cell > 0.0f && 8.0f * c->last_move <= LIST_MAX * c->list_cell;
+    return !c->dense && !c->hulls && c->list_cell > 0.0f && c->plan.pays(list_largest(c));
+}
+
+// The next launch sequence of at most `left` steps, the first with the full sort or not.
+ListRun list_next(sd_ctx* c, int left, bool full) {
+    return c->plan.next(left, lists_pay(c), full, list_largest(c),
+                        LIST_KEPT * list_sigma(c->plan.last, c->list_cell));
+}
+
+void list_read(sd_ctx* c, const StepCtl& ctl, bool used) {
+    ListReport r;
+    r.ran = ctl.ran;
+    r.given_up = ctl.given_up != 0;
+    r.crowded = ctl.over != 0;
+    r.last = ctl.last;
+    r.budget = LIST_KEPT * ctl.sigma;
+    r.used = ctl.displaced;
+    c->plan.read(r, used, list_largest(c));
 }
 
 // Runs nsteps steps: re-sort steps (graph-replayed in pairs when
@@ -421,28 +427,17 @@ sd_status run_steps(sd_ctx* c, int nsteps) {
         if (st != SD_OK) return st;
         const int h0 = c->cur_hist, s0 = c->cur_state;
         const bool full = c->need_full || c->dense;
-        // lists, unless they were found not to hold some sphere's neighbours
-        const bool use = lists_pay(c) && c->list_rest == 0;
-        int rest = 0;
+        const ListRun next = list_next(c, left, full);
+        const bool use = next.none == 0;
         if (!use) {
             // full-sort steps: one after a given-up step or an upload, DENSE_CHUNK
             // of them while the scene is dense, before the changed-cell count is
             // read again
-            rest = full ? (c->dense ? std::min(left, DENSE_CHUNK) : 1)
-                        : std::min(left, c->hulls ? BODY_CHUNK : LIST_REST);
-            st = run(rest, full, LIST_NONE);
-            c->list_steps = 0;
+            const int most = full ? (c->dense ? DENSE_CHUNK : 1) : (c->hulls ? BODY_CHUNK : next.none);
+            st = run(std::min(next.none, most), full, LIST_NONE);
         } else {
-            int l = left;
-            if (full || c->list_steps < std::min(left, 2)) {
-                st = enqueue_step(c, nullptr, full, LIST_BUILD);
-                // (one that was too full for lists, or of unknown speed: a look first)
-                c->list_steps = c->crowded || c->last_move < 0.0f
-                                    ? 2
-                                    : list_life(0.0f, list_sigma(c->last_move, c->list_cell), c->last_move);
-                --l;
-            }
-            if (st == SD_OK) st = run(std::min(l, c->list_steps), false, LIST_USE);
+            if (next.build) st = enqueue_step(c, nullptr, full, LIST_BUILD);
+            if (st == SD_OK) st = run(next.use, false, LIST_USE);
         }
         if (st != SD_OK) return st;
         c->need_full = false;
@@ -456,19 +451,8 @@ sd_status run_steps(sd_ctx* c, int nsteps) {
         c->cur_state = s0 ^ (ran & 1);
         left -= ran;
         c->last_ovf = ctl.overflow;
-        c->last_move = isfinite(ctl.last) ? ctl.last : 3.4e38f;
-        // the displacement of the last step is not in yet: count it as the one before
-        c->list_steps = ctl.given_up ? 0 : list_life(ctl.displaced + ctl.last, ctl.sigma, ctl.last);
+        list_read(c, ctl, use);
         if (ctl.given_up == GIVEN_UP_SORT) c->need_full = true;  // redo the given-up step with the full sort
-        if (use) {
-            c->crowded = ctl.over != 0;
-            if (c->crowded) {
-                c->list_steps = 0;
-                c->list_rest = 4 * LIST_REST;
-            }
-        } else {
-            c->list_rest = std::max(0, c->list_rest - ran);
-        }
         if (full) {  // still dense: the last full-sort step's changed cells exceed the re-sort's cap
             int m = 0;
             SD_HIP(hipMemcpyAsync(&m, c->mcount + c->cur_hist, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -601,9 +585,7 @@ sd_status check_spheres(const char* who, int n, const float* x, const float* y, 
 sd_status force_full_sort(sd_ctx* c) {
     c->need_full = true;
     c->dense = false;
-    c->list_steps = 0;
-    c->list_rest = 0;
-    c->last_move = -1.0f;
+    c->plan = ListPlan();
     // nothing run, no lists (displaced infinite), no displacements
     sd_status st = launch_fill_u32((uint32_t*)c->ctl, 0u, sizeof(StepCtl) / 4, c->stream);
     if (st == SD_OK) st = launch_fill_u32((uint32_t*)&c->ctl->displaced, 0x7f800000u, 1, c->stream);
@@ -889,8 +871,9 @@ extern "C" sd_status sd_ctx_profile(sd_ctx* c, int nsteps, float* stage_ms, int 
         }
         c->need_full = false;
         // near lists as a run would use them, the step redone if they ran out
-        const bool use = lists_pay(c);
-        const int lists = !use ? LIST_NONE : (full || c->list_steps < 1 || c->crowded ? LIST_BUILD : LIST_USE);
+        const ListRun next = list_next(c, 1, full);
+        const bool use = next.none == 0;
+        const int lists = !use ? LIST_NONE : (next.build ? LIST_BUILD : LIST_USE);
         const int keys0 = c->cur_keys, hist0 = c->cur_hist, state0 = c->cur_state;
         StepCtl ctl;
         st = launch_fill_u32((uint32_t*)c->ctl, 0u, 2, c->stream);
@@ -901,9 +884,7 @@ extern "C" sd_status sd_ctx_profile(sd_ctx* c, int nsteps, float* stage_ms, int 
             st = set_error(SD_ERR_HIP, "sd_ctx_profile: control read failed");
             break;
         }
-        c->last_move = isfinite(ctl.last) ? ctl.last : 3.4e38f;
-        c->crowded = use && ctl.over != 0;
-        c->list_steps = ctl.given_up ? 0 : list_life(ctl.displaced + ctl.last, ctl.sigma, ctl.last);
+        list_read(c, ctl, use);
         if (ctl.given_up == GIVEN_UP_LIST) {
             c->cur_keys = keys0;
             c->cur_hist = hist0;

@@ -90,7 +90,7 @@ __device__ __forceinline__ void list_begin_step(StepCtl* L, int lists, float cel
     }
     const float m = sqrtf(__uint_as_float(u)) * 1.00001f;
     const float D = (L->displaced + m) * 1.0000002f;  // (rounded up; not a number: the lists have run out)
-    if (lists == LIST_USE && (!(2.0f * D <= 0.98f * L->sigma) || L->over)) {
+    if (lists == LIST_USE && (!(D <= LIST_KEPT * L->sigma) || L->over)) {
         if ((threadIdx.x & 63) == 0) L->given_up = GIVEN_UP_LIST;
         return;
     }

@@ -123,6 +123,9 @@ constexpr int STEP_CTL_READ = 8;
 // displacement, within [LIST_MIN, LIST_MAX] cells. 40 steps spread the cost of a
 // build (about twice a step without lists at most) and keep the lists short.
 constexpr float LIST_LIFE = 80.0f, LIST_MIN = 0.01f, LIST_MAX = 0.08f;
+// The displacement that a margin allows, of the margin: half of it, each sphere
+// of a pair moving, less what rounding can take.
+constexpr float LIST_KEPT = 0.49f;
 inline float list_sigma(float last, float cell) { return fminf(fmaxf(LIST_LIFE * last, LIST_MIN * cell), LIST_MAX * cell); }
 
 // Fused step kernel modes. CONTACT_FUSED_BATCH: packed u64 keys, every sphere

@@ -116,3 +116,32 @@ def test_lists_stay_off_without_numbers(oracle):
             w = 4 if key == "quat4" else 3
             assert np.array_equal(got[key][rest, :w], want[rest, :w]), key
     sc.close()
+
+
+# slow bodies away from the origin (by so much that rounding takes a part of the
+# lists' margin, and all of it), and near it with one far away (a static one)
+@pytest.mark.parametrize("off,stray", [(300.0, 0.0), (2500.0, 0.0), (30000.0, 0.0), (0.0, 5000.0), (0.0, 1e6)])
+def test_lists_far_from_the_origin(oracle, off, stray):
+    print("[gpu-case] clump lists, far", off, stray, flush=True)
+    s = bodies(300, 0.09, 0.02, 11)
+    s["pos4"][:, 0] += off
+    if stray:
+        s["pos4"][-1, 1] = stray
+        s["pos4"][-1, 3] = 0.0
+        s["vel4"][-1] = 0.0
+        s["angvel4"][-1] = 0.0
+    c = CL.contact_c3()
+    o = oracle.ClumpState(s)
+    sc = CL.ClumpScene(c)
+    sc.upload(s)
+    for k in (1, 3, 90, 200):
+        sc.step(k)
+        o.step(c, k - 1)
+        _, _, lo, hi = o.pose()
+        o.step(c, 1)
+        compare(sc, o)
+        assert pair_set(sc.pairs()) == pair_set(oracle.brute_aabb_pairs(lo, hi))
+    sc.profile(5)
+    o.step(c, 5)
+    compare(sc, o)
+    sc.close()
