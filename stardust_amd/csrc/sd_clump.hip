@@ -496,10 +496,13 @@ struct sd_clump_ctx {
     bool tree_last = false;   // the tree is that of the last step's boxes
     hipGraphExec_t graph[2][3] = {};  // two steps from buffer parity 0 / 1, by what they do with the lists
     hipGraph_t graph_obj[2][3] = {};
-    float4 *ilo = nullptr, *ihi = nullptr;  // inflated boxes of a step that builds lists
-    ClumpCtl* ctl = nullptr;
-    uint8_t* lcount = nullptr;
+    // partner lists, and the inflated boxes of a step that builds them, all in
+    // list_mem; NULL: none, every step walks a tree
+    char* list_mem = nullptr;
+    float4 *ilo = nullptr, *ihi = nullptr;
     int* list = nullptr;
+    uint8_t* lcount = nullptr;
+    ClumpCtl* ctl = nullptr;
     float size = 0.0f;        // mean extent of the bodies
     ListPlan plan;
     bool boxes = false;       // blo / bhi are those of the step before
@@ -531,8 +534,7 @@ void cfree(sd_clump_ctx* c) {
                     c->slocal,  c->sx,        c->blo,      c->bhi,     c->domain,   c->dom_scratch,
                     c->mkeys,   c->mkeys2,    c->sort_tmp,   c->left,     c->right,   c->parent,   c->first,
                     c->last,    c->rope,      c->nlo,        c->nhi,      c->counters, c->q_scratch,
-                    c->pairs,   c->ilo,       c->ihi,        c->pnode,
-                    c->ctl,     c->lcount,    c->list};
+                    c->pairs,   c->pnode,     c->ctl,        c->list_mem};
     drop_clump_graphs(c);
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -851,16 +853,23 @@ sd_status write_clump_rows(sd_clump_ctx* c, const ClumpRows& r) {
     ALLOC(c->counters, 3 * (size_t)nb + 8);
     sd_lbvh_query_scratch_bytes(nb, &c->q_scratch_bytes);
     ALLOC(*(char**)&c->q_scratch, c->q_scratch_bytes);
-    ALLOC(c->ilo, nb);
-    ALLOC(c->ihi, nb);
     ALLOC(c->ctl, 1);
-    ALLOC(c->lcount, nb);
-    ALLOC(c->list, (size_t)CL_LIST * nb);
 #undef ALLOC
     if (st == SD_OK) st = grow_pairs(c, 8 * nb);
     if (st != SD_OK) {
         cfree(c);
         return st;
+    }
+    // (97 bytes a body; bodies that fit without lists step without)
+    const size_t row = (size_t)nb * sizeof(float4), list = (size_t)nb * CL_LIST * sizeof(int);
+    if (hipMalloc((void**)&c->list_mem, 2 * row + list + (size_t)nb) == hipSuccess) {
+        c->ilo = (float4*)c->list_mem;
+        c->ihi = (float4*)(c->list_mem + row);
+        c->list = (int*)(c->list_mem + 2 * row);
+        c->lcount = (uint8_t*)c->list_mem + 2 * row + list;
+    } else {
+        (void)hipGetLastError();
+        c->list_mem = nullptr;
     }
     hipStream_t s = c->stream;
     SD_HIP(hipMemcpyAsync(c->pos[0], r.P.data(), nb * sizeof(float4), hipMemcpyHostToDevice, s));
@@ -973,7 +982,7 @@ static sd_status clump_graph_pair(sd_clump_ctx* c, int lists) {
 // The next launch sequence of at most `left` steps.
 static ListRun clump_next(sd_clump_ctx* c, int left) {
     const float largest = clump_largest(c->size);
-    return c->plan.next(left, c->size > 0.0f && c->plan.pays(largest), false, largest,
+    return c->plan.next(left, c->list_mem && c->size > 0.0f && c->plan.pays(largest), false, largest,
                         CL_MARGIN_KEPT * clump_margin(c->plan.last, c->size));
 }
 

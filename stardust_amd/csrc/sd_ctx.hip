@@ -127,7 +127,9 @@ struct sd_ctx {
     uint64_t* mold = nullptr;
     uint64_t* msn = nullptr;
     uint64_t* mso = nullptr;
-    // near lists, alternating with the history buffers (sd_internal.hpp)
+    // near lists, alternating with the history buffers (sd_internal.hpp), all in
+    // list_mem; NULL: none, every step searches
+    char* list_mem = nullptr;
     uint8_t* lcount[2] = {nullptr, nullptr};
     int* list[2] = {nullptr, nullptr};
     int* newpos = nullptr;
@@ -187,8 +189,7 @@ void release(sd_ctx* c) {
                     c->posB, c->k64[0], c->k64[1], c->sort_tmp,
                     c->cell_start, c->hcount[0], c->hcount[1], c->hist[0], c->hist[1], c->ctl, c->diag,
                     c->scenes_d, c->scene_of, c->straddle, c->mcount, c->mnew, c->mold, c->msn, c->mso,
-                    c->lcount[0], c->lcount[1], c->list[0], c->list[1], c->newpos,
-                    c->scene_rmax};
+                    c->list_mem, c->scene_rmax};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (int k = 0; k < 2; ++k) {
@@ -204,9 +205,7 @@ void release(sd_ctx* c) {
     c->ctl = nullptr;
     c->mcount = nullptr;
     c->mnew = c->mold = c->msn = c->mso = nullptr;
-    c->lcount[0] = c->lcount[1] = nullptr;
-    c->list[0] = c->list[1] = nullptr;
-    c->newpos = nullptr;
+    c->list_mem = nullptr;
     c->scene_rmax = nullptr;
     c->diag = nullptr;
     c->scenes_d = nullptr;
@@ -377,14 +376,35 @@ sd_status run_graph_pair(sd_ctx* c, bool full, int lists) {
     return SD_OK;
 }
 
+// The memory of the near lists (198 bytes a sphere), or none: with rigid bodies
+// attached (the bodies' part of a given-up step would be computed twice), or
+// where it cannot be had. A scene that fits without lists then steps without.
+void alloc_lists(sd_ctx* c) {
+    if (c->hulls) {
+        if (c->list_mem) (void)hipFree(c->list_mem);
+        c->list_mem = nullptr;
+    }
+    if (c->hulls || c->list_mem) return;
+    const size_t n = (size_t)c->n, list = LIST_CAP * n * sizeof(int);
+    if (hipMalloc((void**)&c->list_mem, 2 * list + n * sizeof(int) + 2 * n) != hipSuccess) {
+        (void)hipGetLastError();
+        c->list_mem = nullptr;
+        return;
+    }
+    for (int k = 0; k < 2; ++k) {
+        c->list[k] = (int*)(c->list_mem + k * list);
+        c->lcount[k] = (uint8_t*)c->list_mem + 2 * list + n * sizeof(int) + k * n;
+    }
+    c->newpos = (int*)(c->list_mem + 2 * list);
+}
+
 // Displacement that the widest near lists allow.
 float list_largest(const sd_ctx* c) { return LIST_KEPT * LIST_MAX * c->list_cell; }
 
 // Whether near lists pay: at the scene's speed, and not in dense runs (whose
-// spheres cross cells). Steps with rigid bodies attached keep none: the bodies' part of a
-// given-up step would be computed twice.
+// spheres cross cells).
 bool lists_pay(const sd_ctx* c) {
-    return !c->dense && !c->hulls && c->list_cell > 0.0f && c->plan.pays(list_largest(c));
+    return !c->dense && c->list_mem && c->list_cell > 0.0f && c->plan.pays(list_largest(c));
 }
 
 // The next launch sequence of at most `left` steps, the first with the full sort or not.
@@ -536,6 +556,8 @@ extern "C" sd_status sd_batch_attach_hulls(sd_ctx* c, sd_hull_ctx* h) {
     (void)hipStreamSynchronize(c->stream);
     drop_graphs(c);  // the step graphs are captured again with (or without) the bodies
     c->hulls = h;
+    if (c->n) alloc_lists(c);
+    c->plan = ListPlan();
     if (h) c->hull_gen = hull_generation(h);
     return SD_OK;
 }
@@ -616,6 +638,7 @@ sd_status set_list_bounds(sd_ctx* c, const float* r, int stride) {
         SD_HIP(hipMemcpyAsync(c->scene_rmax, rm.data(), scenes * sizeof(float), hipMemcpyHostToDevice, c->stream));
         SD_HIP(hipStreamSynchronize(c->stream));
     }
+    alloc_lists(c);
     return SD_OK;
 }
 
@@ -654,11 +677,6 @@ sd_status upload_state(sd_ctx* c, int n, const float* x, const float* y, const f
     ALLOC(c->mold, resort_cap(n));
     ALLOC(c->msn, resort_cap(n));
     ALLOC(c->mso, resort_cap(n));
-    for (int k = 0; k < 2; ++k) {
-        ALLOC(c->lcount[k], n);
-        ALLOC(c->list[k], (size_t)LIST_CAP * n);
-    }
-    ALLOC(c->newpos, n);
     c->diag_blocks = div_up(n, DIAG_BLOCK) < 1024 ? div_up(n, DIAG_BLOCK) : 1024;
     ALLOC(c->diag, (size_t)c->diag_blocks * DIAG_VALUES);
 #undef ALLOC
