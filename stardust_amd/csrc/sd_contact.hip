@@ -102,15 +102,21 @@ __device__ __forceinline__ void find_history(const ContactArgs& a, int os, int o
 
 constexpr int CAND_UNROLL = 4; // candidate positions loaded per batch (loads in flight)
 static_assert(CAND_UNROLL - 1 <= CONTACT_POS_PAD, "sorted positions must be padded for a whole batch");
-constexpr int CONTACT_STAGE = 224;  // staged candidate positions per wave (3.5 KiB of LDS)
 constexpr int CONTACT_ITEMS = 128;  // contacts of a wave handed out at a time (their places in the same LDS)
 constexpr int CONTACT_PASS = 12;    // contacts of one sphere spread over the wave
-// float4s of LDS per wave: the stage of a search, or only what shares it, and
-// the contacts found by each lane
+// float4s of LDS per wave: the stage of a search (candidate positions), or only
+// what shares it, and the contacts found by each lane. A search of dilute scenes
+// needs every wave that its registers allow: with 224 positions staged the LDS
+// held fewer. Forces of 1,000,003 dilute spheres 72 us with 224, 69 with 192, 68
+// with 160 (in contact 120, 117, 116); a step of 4,194,304 that searches 303, 291,
+// 291, but of 250,007, whose runs of candidates are longer, 33, 33, 36.
 constexpr int CONTACT_SHARED = CONTACT_ITEMS / 2 + 6 * WAVE / 4;
-constexpr int contact_lds(bool listed) { return (listed ? CONTACT_SHARED : CONTACT_STAGE) + CONTACT_PASS * WAVE / 4; }
+constexpr int contact_stage(int mode, int lists) {
+    return lists == LIST_USE ? CONTACT_SHARED : (mode == CONTACT_FORCES ? 160 : 192);
+}
+constexpr int contact_lds(int mode, int lists) { return contact_stage(mode, lists) + CONTACT_PASS * WAVE / 4; }
 static_assert(LIST_CAP % CAND_UNROLL == 0, "whole batches of a list are read");
-static_assert(CONTACT_SHARED <= CONTACT_STAGE, "items and results fit the stage");
+static_assert(CONTACT_SHARED <= contact_stage(CONTACT_FORCES, LIST_NONE), "items and results fit the stage");
 
 // Orders one wave's LDS writes and reads (the lanes of a wave only).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -177,10 +183,14 @@ __device__ __forceinline__ T uniform_copy(const T& src) {
 // went through its own contacts), 1,000 spheres 18 us (51). A step that makes
 // lists takes 416, 222 and 43 us, every 40th step or so.
 //
-// Two kernels: with the search as a branch of one, the steps on lists ran at 4
-// waves a SIMD or with spills (4,194,304 spheres 265 and 395 us).
-template <int MODE, bool INDIRECT, bool STRADDLE, bool LISTED>
+// A kernel for each use of the lists (LISTS): with the search as a branch of one,
+// the steps on lists ran at 4 waves a SIMD or with spills (4,194,304 spheres 265
+// and 395 us); with the making of lists as a branch of the search, a step that
+// only searches lost a wave a SIMD (4,194,304 spheres 318 us, 303 without).
+template <int MODE, bool INDIRECT, bool STRADDLE, int LISTS>
 __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
+    constexpr bool LISTED = LISTS == LIST_USE, BUILD = LISTS == LIST_BUILD;
+    constexpr int STAGE = contact_stage(MODE, LISTS);
     constexpr bool BATCH = MODE == CONTACT_FUSED_BATCH;
     constexpr bool FUSED = MODE != CONTACT_FORCES;
     constexpr bool PADDED = FUSED;  // fused modes read a context's padded buffer
@@ -226,14 +236,16 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
     // the velocity and spin are read where they are needed, after the
     // contacts: held from here they cost a wave a SIMD
     float4 p = rowpos[self];
-    const float inv_m = a.vel[self].w, inv_i = a.omg[self].w;
+    const float inv_m = a.vel[self].w;
+    float inv_i = 0.0f;
+    if constexpr (FUSED) inv_i = a.omg[self].w;  // (brings the row into the cache)
     const int myid = FUSED ? a.ids[self] : 0;
     int oc = a.hcount_old[os];
     oc = oc < c.maxc ? oc : c.maxc;
     int lcount = 0;      // LISTED: the sphere's list
     float sigma = 0.0f;  // a search that makes lists: their margin
     if constexpr (LISTED) lcount = live ? a.lcount_old[os] : 0;
-    else if (FUSED && a.lists == LIST_BUILD) sigma = a.ctl->sigma;
+    else if constexpr (BUILD) sigma = a.ctl->sigma;
 
     int cx, cy, cz;
     cell_coords(g, p.x, p.y, p.z, cx, cy, cz);
@@ -245,10 +257,10 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
     // wave (row, owning lane and number) and 64 results; the rows of each
     // lane's contacts (entry k of a lane at k * 64 + lane)
     extern __shared__ float4 cstage[];
-    float4* const stg = cstage + (threadIdx.x >> 6) * contact_lds(LISTED);
+    float4* const stg = cstage + (threadIdx.x >> 6) * contact_lds(MODE, LISTS);
     int2* const items = reinterpret_cast<int2*>(stg);
     float* const res = reinterpret_cast<float*>(stg + CONTACT_ITEMS / 2);
-    int* const pend = reinterpret_cast<int*>(stg + (LISTED ? CONTACT_SHARED : CONTACT_STAGE)) + lane;
+    int* const pend = reinterpret_cast<int*>(stg + STAGE) + lane;
 
     // Whether the sphere at row `row`, closer than the radii, (dx, dy, dz) away
     // and not coincident (the sphere itself, too), is a contact: not both
@@ -257,7 +269,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
     // cell is wide two cells apart, which is no contact (nearer pairs cannot
     // be, by far, on grids of up to 65,536 cells a side): a search of the 27
     // cells does not meet it.
-    const float near = FUSED && a.lists != LIST_NONE
+    const float near = LISTS != LIST_NONE
                            ? (max(g.nx, max(g.ny, g.nz)) > 65536 ? 0.0f : 0.9f * g.cell)
                            : 3.4e38f;
     auto is_contact = [&](int row, float dx, float dyy, float dzz) -> bool {
@@ -358,8 +370,8 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
                     const int t = t0 + __builtin_ctz(hit);
                     hit &= hit - 1u;
                     if (t >= hi || t == s) continue;
-                    if constexpr (FUSED) {
-                        if (ln < LIST_CAP && a.lists == LIST_BUILD) a.list_new[(size_t)ln * a.n + s] = t;
+                    if constexpr (BUILD) {
+                        if (ln < LIST_CAP) a.list_new[(size_t)ln * a.n + s] = t;
                         ++ln;
                     }
                     const float4 qt = sl[t];  // (the staged copy)
@@ -386,7 +398,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
         // positions a batch may read past a window, form one staged
         // sequence: sorted position t of a lane is entry t + off of it.
         // The wave copies the sequence into its LDS region with coalesced
-        // loads (in chunks of CONTACT_STAGE entries; one chunk unless the
+        // loads (in chunks of STAGE entries; one chunk unless the
         // wave spans several sparse rows) and every lane tests its
         // candidates in the chunk from LDS.
         const uint64_t amask = __ballot(1);  // the searching lanes
@@ -396,7 +408,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
         const bool segB = rowid != (uint32_t)__builtin_amdgcn_readfirstlane((int)rowid);
         const uint64_t bmask = __ballot(segB);
         constexpr int PAD = CAND_UNROLL - 1;        // a batch reads up to 3 positions past its window
-        constexpr int CHUNK = CONTACT_STAGE - PAD;  // sequence entries tested per chunk
+        constexpr int CHUNK = STAGE - PAD;  // sequence entries tested per chunk
         const char* const pos_bytes = reinterpret_cast<const char*>(a.pos);
 
         // Rows of the search, in ascending order: the 27 cells around the
@@ -408,17 +420,15 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
         // (windows ascend with the lane).
         int y0 = max(cy - 1, 0), y1 = min(cy + 1, g.ny - 1), z0 = max(cz - 1, 0), z1 = min(cz + 1, g.nz - 1);
         int e = 1;
-        if constexpr (FUSED) {
-            if (a.lists == LIST_BUILD) {
-                const float R = (reach + rmax) * 1.0001f;
-                y0 = axis_cell(p.y - R, g.loy, g.cell, g.ny);
-                y1 = axis_cell(p.y + R, g.loy, g.cell, g.ny);
-                z0 = axis_cell(p.z - R, g.loz, g.cell, g.nz);
-                z1 = axis_cell(p.z + R, g.loz, g.cell, g.nz);
-                const int x0 = axis_cell(p.x - R, g.lox, g.cell, g.nx);
-                const int x1 = axis_cell(p.x + R, g.lox, g.cell, g.nx);
-                e = __ballot(cx - x0 > 1 || x1 - cx > 1) ? 2 : 1;
-            }
+        if constexpr (BUILD) {
+            const float R = (reach + rmax) * 1.0001f;
+            y0 = axis_cell(p.y - R, g.loy, g.cell, g.ny);
+            y1 = axis_cell(p.y + R, g.loy, g.cell, g.ny);
+            z0 = axis_cell(p.z - R, g.loz, g.cell, g.nz);
+            z1 = axis_cell(p.z + R, g.loz, g.cell, g.nz);
+            const int x0 = axis_cell(p.x - R, g.lox, g.cell, g.nx);
+            const int x1 = axis_cell(p.x + R, g.lox, g.cell, g.nx);
+            e = __ballot(cx - x0 > 1 || x1 - cx > 1) ? 2 : 1;
         }
         // row offsets (dz, dy) that some lane of the wave has
         const int dz0 = __ballot(z0 < cz - 1) ? -2 : (__ballot(z0 < cz) ? -1 : 0);
@@ -463,7 +473,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
             const int off = segB ? offb - lb : -la;    // sequence entry of sorted position t: t + off
             const int lb_b = lb - offb;                // source of entry e >= offb: lb_b + e
             for (int e0 = 0; e0 < seq - PAD; e0 += CHUNK) {
-                const int m = min(CONTACT_STAGE, seq - e0);
+                const int m = min(STAGE, seq - e0);
                 for (int i = arank; i < m; i += 2 * nact) {
                     const int e1 = e0 + i, e2 = e1 + nact;
                     // sources reach at most n + 2 (3 padding entries past a
@@ -494,7 +504,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
         }
     }
 
-    asm volatile("" ::"v"(inv_i));  // (the row is in the cache by now; not held further)
+    if constexpr (FUSED) asm volatile("" ::"v"(inv_i));  // (the row is in the cache by now; not held further)
 
     // the wave's contacts: lane l's are [off, off + pc)
     if (!LISTED) pc = min(hc, CONTACT_PASS);
@@ -689,7 +699,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
     } else {
         if constexpr (LISTED) {
             if (live) a.lcount_new[s] = (uint8_t)lcount;
-        } else if (a.lists == LIST_BUILD) {
+        } else if constexpr (BUILD) {
             if (live) a.lcount_new[s] = (uint8_t)min(ln, LIST_CAP);
             if (__ballot(live && ln > LIST_CAP) != 0u && lane == 0) a.ctl->over = 1;
         }
@@ -729,10 +739,10 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
 }
 
 
-template <int MODE, bool INDIRECT, bool STRADDLE, bool LISTED>
+template <int MODE, bool INDIRECT, bool STRADDLE, int LISTS>
 __global__ __launch_bounds__(256) void k_contacts(ContactArgs a) {
     static_assert(!STRADDLE || MODE == CONTACT_FUSED_BATCH, "k_contacts: straddling waves exist in batch mode only");
-    static_assert(!LISTED || INDIRECT, "k_contacts: only a context's steps have lists");
+    static_assert(LISTS == LIST_NONE || INDIRECT, "k_contacts: only a context's steps have lists");
     if (MODE != CONTACT_FORCES) {
         if (a.ctl->given_up) return;
         if (!STRADDLE && blockIdx.x == 0 && threadIdx.x == 0) a.ctl->ran += 1;
@@ -745,7 +755,7 @@ __global__ __launch_bounds__(256) void k_contacts(ContactArgs a) {
         if (lb < 0) return;
         s = lb * (int)blockDim.x + (int)threadIdx.x;
     }
-    contact_wave<MODE, INDIRECT, STRADDLE, LISTED>(a, s);
+    contact_wave<MODE, INDIRECT, STRADDLE, LISTS>(a, s);
 }
 
 constexpr int PERSIST_CLAIM = 8;    // tiles a wave claims at a time
@@ -756,7 +766,7 @@ constexpr int PERSIST_STRIDE = 64;  // ints between the XCDs' counters
 // x-th eighth of the slots, so an XCD's L2 still holds neighbouring cells)
 // until its range is exhausted; the results are those of k_contacts (every
 // tile computes the same slots the same way). counters[0..7] start at 0.
-template <int MODE, bool LISTED>
+template <int MODE, int LISTS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_contacts_persistent(
     ContactArgs a, int* __restrict__ counters) {
     if (a.ctl->given_up) return;
@@ -772,7 +782,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         t = t0 + __shfl(t, 0);
         if (t >= t1) break;
         const int te = min(t + PERSIST_CLAIM, t1);
-        for (; t < te; ++t) contact_wave<MODE, true, false, LISTED>(a, t * WAVE + lane_id());
+        for (; t < te; ++t) contact_wave<MODE, true, false, LISTS>(a, t * WAVE + lane_id());
     }
 }
 
@@ -788,24 +798,28 @@ __global__ void k_integrate(float4* __restrict__ pos, float4* __restrict__ vel, 
     omg[i] = w;
 }
 
+template <typename F>
+static F by_lists(int lists, F use, F build, F none) {
+    return lists == LIST_USE ? use : (lists == LIST_BUILD ? build : none);
+}
+
 sd_status launch_contacts(int mode, const ContactArgs& a, hipStream_t s, int block) {
     if (a.n <= 0) return SD_OK;
     if (block <= 0) block = 128;
     SD_REQUIRE(block % WAVE == 0 && block <= 256, "contact kernel: block must be a multiple of 64, <= 256");
     const int nblocks = div_up(a.n, block);
     const dim3 grid(div_up(nblocks, XCDS) * XCDS);  // padded for the XCD remap
-    const bool listed = mode != CONTACT_FORCES && a.lists == LIST_USE;
-    const size_t lds = (size_t)(block / WAVE) * contact_lds(listed) * sizeof(float4);
-    if (mode == CONTACT_FORCES)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FORCES, false, false, false>), grid, dim3(block), lds, s, a);
-    else if (mode == CONTACT_FUSED_U64 && listed)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U64, true, false, true>), grid, dim3(block), lds, s, a);
-    else if (mode == CONTACT_FUSED_U64)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_U64, true, false, false>), grid, dim3(block), lds, s, a);
-    else if (listed)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, false, true>), grid, dim3(block), lds, s, a);
-    else
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, false, false>), grid, dim3(block), lds, s, a);
+    const int lists = mode == CONTACT_FORCES ? LIST_NONE : a.lists;
+    const size_t lds = (size_t)(block / WAVE) * contact_lds(mode, lists) * sizeof(float4);
+    void (*const kernel)(ContactArgs) =
+        mode == CONTACT_FORCES      ? &k_contacts<CONTACT_FORCES, false, false, LIST_NONE>
+        : mode == CONTACT_FUSED_U64 ? by_lists(lists, &k_contacts<CONTACT_FUSED_U64, true, false, LIST_USE>,
+                                               &k_contacts<CONTACT_FUSED_U64, true, false, LIST_BUILD>,
+                                               &k_contacts<CONTACT_FUSED_U64, true, false, LIST_NONE>)
+                                    : by_lists(lists, &k_contacts<CONTACT_FUSED_BATCH, true, false, LIST_USE>,
+                                               &k_contacts<CONTACT_FUSED_BATCH, true, false, LIST_BUILD>,
+                                               &k_contacts<CONTACT_FUSED_BATCH, true, false, LIST_NONE>);
+    hipLaunchKernelGGL(kernel, grid, dim3(block), lds, s, a);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }
@@ -816,13 +830,14 @@ sd_status launch_contacts_persistent(int mode, const ContactArgs& a, hipStream_t
     SD_REQUIRE(block % WAVE == 0 && block <= 256, "contact kernel: block must be a multiple of 64, <= 256");
     SD_REQUIRE(mode == CONTACT_FUSED_U64 || mode == CONTACT_FUSED_BATCH,
                "contact kernel: the persistent form is for packed 64-bit keys");
-    const bool listed = a.lists == LIST_USE;
     void (*const kernel)(ContactArgs, int*) =
-        mode == CONTACT_FUSED_U64 ? (listed ? &k_contacts_persistent<CONTACT_FUSED_U64, true>
-                                            : &k_contacts_persistent<CONTACT_FUSED_U64, false>)
-                                  : (listed ? &k_contacts_persistent<CONTACT_FUSED_BATCH, true>
-                                            : &k_contacts_persistent<CONTACT_FUSED_BATCH, false>);
-    const size_t lds = (size_t)(block / WAVE) * contact_lds(listed) * sizeof(float4);
+        mode == CONTACT_FUSED_U64 ? by_lists(a.lists, &k_contacts_persistent<CONTACT_FUSED_U64, LIST_USE>,
+                                             &k_contacts_persistent<CONTACT_FUSED_U64, LIST_BUILD>,
+                                             &k_contacts_persistent<CONTACT_FUSED_U64, LIST_NONE>)
+                                  : by_lists(a.lists, &k_contacts_persistent<CONTACT_FUSED_BATCH, LIST_USE>,
+                                             &k_contacts_persistent<CONTACT_FUSED_BATCH, LIST_BUILD>,
+                                             &k_contacts_persistent<CONTACT_FUSED_BATCH, LIST_NONE>);
+    const size_t lds = (size_t)(block / WAVE) * contact_lds(mode, a.lists) * sizeof(float4);
     int dev = 0, cus = 0, per_cu = 0;
     SD_HIP(hipGetDevice(&dev));
     SD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -842,14 +857,11 @@ sd_status launch_contacts_persistent(int mode, const ContactArgs& a, hipStream_t
 sd_status launch_contacts_straddle(const ContactArgs& a, hipStream_t s) {
     if (a.n <= 0 || a.n_straddle <= 0) return SD_OK;
     SD_REQUIRE(a.straddle && a.scenes && a.scene_of, "contact kernel: straddle launch without its lists");
-    const bool listed = a.lists == LIST_USE;
-    const size_t lds = (size_t)contact_lds(listed) * sizeof(float4);
-    if (listed)
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, true, true>), dim3(a.n_straddle), dim3(WAVE), lds, s,
-                           a);
-    else
-        hipLaunchKernelGGL((k_contacts<CONTACT_FUSED_BATCH, true, true, false>), dim3(a.n_straddle), dim3(WAVE), lds,
-                           s, a);
+    const size_t lds = (size_t)contact_lds(CONTACT_FUSED_BATCH, a.lists) * sizeof(float4);
+    hipLaunchKernelGGL(by_lists(a.lists, &k_contacts<CONTACT_FUSED_BATCH, true, true, LIST_USE>,
+                                &k_contacts<CONTACT_FUSED_BATCH, true, true, LIST_BUILD>,
+                                &k_contacts<CONTACT_FUSED_BATCH, true, true, LIST_NONE>),
+                       dim3(a.n_straddle), dim3(WAVE), lds, s, a);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }

@@ -483,3 +483,35 @@ def test_contact_forces_sparse_plane(oracle):
                           valid_hist(eh, exp["hcount"]).view(np.uint32))
     assert np.array_equal(got["force"], exp["force"])
     assert np.array_equal(got["torque"], exp["torque"])
+
+
+# candidates of a row of cells around the ends of a staged chunk (157 tested a
+# chunk in the force entry point, 189 in a step), and of two
+@pytest.mark.parametrize("m", [63, 65, 154, 157, 158, 160, 186, 189, 190, 192, 314, 315, 378, 379])
+def test_candidates_at_chunk_ends(oracle, m):
+    say("candidates at chunk ends", m)
+    rng = np.random.default_rng(m)
+    pos = rng.uniform(0.1, 0.9, (m, 3)).astype(np.float32)
+    rad = rng.uniform(0.02, 0.06, m).astype(np.float32)
+    vel = rng.normal(0, 0.5, (m, 3)).astype(np.float32)
+    mass = W.sphere_mass(rad)
+    g = L.Grid.make((0.0, 0.0, 0.0), 1.0, (1, 1, 1))
+    c = L.ContactParams.make(1e4, 0.3, 0.5, 1e-5, walls=((0.0, 0.0, 0.0), (1.0, 1.0, 1.0)), max_contacts=64)
+    init = {"x": pos[:, 0].copy(), "y": pos[:, 1].copy(), "z": pos[:, 2].copy(), "r": rad, "m": mass,
+            "vx": vel[:, 0].copy(), "vy": vel[:, 1].copy(), "vz": vel[:, 2].copy()}
+    st = oracle.SphereState(*[init[k] for k in ("x", "y", "z")], rad, mass, vx=init["vx"], vy=init["vy"],
+                            vz=init["vz"], max_contacts=64)
+    sc = make_scene(init, g, c, key64=True, graph=False)
+    for k in (1, 3):
+        sc.step(k)
+        st.step(g, c, nsteps=k, nthreads=8)
+        compare_scene(sc, st)
+    sc.close()
+    s = sorted_state(oracle, st, g)
+    exp = oracle.contact_forces(s["pos4"], s["vel4"], s["omg4"], s["ids"], g, s["ranges"], c, s["old_slot"],
+                                st.hcount, st.hist, nthreads=8)
+    got = gpu_contact_forces(s, st, g, c)
+    assert m < 150 or exp["hcount"].sum() > 0
+    assert np.array_equal(got["hcount"], exp["hcount"])
+    assert np.array_equal(got["force"], exp["force"])
+    assert np.array_equal(got["torque"], exp["torque"])
