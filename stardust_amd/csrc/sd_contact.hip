@@ -190,7 +190,7 @@ __device__ __forceinline__ T uniform_copy(const T& src) {
 template <int MODE, bool INDIRECT, bool STRADDLE, int LISTS>
 __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
     constexpr bool LISTED = LISTS == LIST_USE, BUILD = LISTS == LIST_BUILD;
-    constexpr int STAGE = contact_stage(MODE, LISTS);
+    constexpr int STAGE = contact_stage(MODE, LISTS), STAGE_MOST = 3 * STAGE;
     constexpr bool BATCH = MODE == CONTACT_FUSED_BATCH;
     constexpr bool FUSED = MODE != CONTACT_FORCES;
     constexpr bool PADDED = FUSED;  // fused modes read a context's padded buffer
@@ -349,6 +349,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
         // built, the distance is the contact's plus the margin, and every
         // sphere within it is listed.
         const float reach = p.w + sigma;
+        // sl: where the candidates are held (position t at sl[t]).
         auto test_batch = [&](const float4 (&q)[CAND_UNROLL], int t0, int hi, const float4* sl) {
             bool h[CAND_UNROLL];
             uint64_t any = 0u;  // lanes with a possible contact (scalar masks)
@@ -374,7 +375,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
                         if (ln < LIST_CAP) a.list_new[(size_t)ln * a.n + s] = t;
                         ++ln;
                     }
-                    const float4 qt = sl[t];  // (the staged copy)
+                    const float4 qt = sl[t];
                     const float dx = p.x - qt.x;
                     const float dyy = p.y - qt.y;
                     const float dzz = p.z - qt.z;
@@ -383,7 +384,9 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
                     if (!(d2 < rs * rs) || d2 == 0.0f) continue;
                     const int row = INDIRECT ? old_slot_of(a, t) : t;
                     if (!is_contact(row, dx, dyy, dzz)) continue;
+                    // (the rows past those kept wait where their history will be)
                     if (hc < CONTACT_PASS) pend[hc * WAVE] = row;
+                    else if (hc < c.maxc) a.hist_new[(size_t)hc * a.n + s].x = __int_as_float(row);
                     ++hc;
                 }
             }
@@ -472,6 +475,21 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
             const int seq = offb + nb + PAD;           // sequence length
             const int off = segB ? offb - lb : -la;    // sequence entry of sorted position t: t + off
             const int lb_b = lb - offb;                // source of entry e >= offb: lb_b + e
+            // A wave of a sparse region beside a dense one (its lanes in many
+            // rows of a half-filled layer, the layer below it full): the union of
+            // its windows is thousands of positions, of which each lane needs a
+            // few, and read chunk by chunk one such wave is all a step waits for
+            // (250,007 spheres in contact 227 us, now 51). From three chunks on
+            // each lane reads its own window.
+            if (seq > STAGE_MOST) {
+                for (int t0 = lo; t0 < hi; t0 += CAND_UNROLL) {
+                    float4 q[CAND_UNROLL];
+#pragma unroll
+                    for (int k = 0; k < CAND_UNROLL; ++k) q[k] = a.pos[min(t0 + k, hi - 1)];
+                    test_batch(q, t0, hi, a.pos);
+                }
+                continue;
+            }
             for (int e0 = 0; e0 < seq - PAD; e0 += CHUNK) {
                 const int m = min(STAGE, seq - e0);
                 for (int i = arank; i < m; i += 2 * nact) {
@@ -577,7 +595,9 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
 
     // A sphere with more contacts than that (one large sphere among many small
     // ones): the others one after the other. A second pass of the code above
-    // instead, in a loop around it, took 25 registers more.
+    // instead, in a loop around it, took 25 registers more. A search has left
+    // their rows where their history will be written: searching again made a
+    // step with 45 of them 135 us, now 88.
     if (__ballot(hc > CONTACT_PASS) != 0u && hc > CONTACT_PASS) {
         auto add = [&](int row) {
             const float4 q = rowpos[row], vi = a.vel[self], vj = a.vel[row], wi = a.omg[self], wj = a.omg[row];
@@ -624,7 +644,15 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
                 add(row);
             }
         } else {
-            int skip = CONTACT_PASS;
+            const int kept = min(hc, c.maxc);
+            int row = nc < kept ? __float_as_int(a.hist_new[(size_t)nc * a.n + s].x) : 0;
+            while (nc < kept) {
+                const int next = nc + 1 < kept ? __float_as_int(a.hist_new[(size_t)(nc + 1) * a.n + s].x) : 0;
+                add(row);
+                row = next;
+            }
+            // more than the history holds (an error, but their forces count): searched again
+            int skip = nc;
             for (int r = 0; r < 9 && nc < hc; ++r) {
                 const int z = cz + r / 3 - 1, y = cy + r % 3 - 1;
                 if (z < 0 || z >= g.nz || y < 0 || y >= g.ny) continue;
@@ -633,10 +661,10 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
                 else row_window(g, ranges, cx, 1, y, z, lo, hi);
                 for (int t = lo; t < hi && nc < hc; ++t) {
                     if (t == s) continue;
-                    const int row = INDIRECT ? old_slot_of(a, t) : t;
-                    if (!touches(row)) continue;
+                    const int at = INDIRECT ? old_slot_of(a, t) : t;
+                    if (!touches(at)) continue;
                     if (skip > 0) --skip;
-                    else add(row);
+                    else add(at);
                 }
             }
         }

@@ -425,8 +425,8 @@ def test_step_many_cell_changes(oracle, n, speed):
 def sparse_plane_scene():
     """One sphere per grid row in the bottom plane (64 rows) and 1,024 spheres in
     the plane above: the first wave's 64 lanes lie in 64 different rows, so the
-    candidates of their upper-plane rows (about 1,000 positions) are staged and
-    tested in several chunks."""
+    candidates of their upper-plane rows (about 1,000 positions) are more than
+    are staged, and every lane reads its own."""
     rng = np.random.default_rng(53)
     cell, nx, ny = 0.01, 4, 64
     n0, n1 = ny, 1024
@@ -452,7 +452,7 @@ def oracle_state(oracle, init):
 
 @pytest.mark.parametrize("key64", [False, True])
 def test_step_sparse_plane_under_dense_plane(oracle, key64):
-    """Stepping with the multi-chunk candidate staging: bit-identical to the oracle."""
+    """Stepping with candidates read by each lane: bit-identical to the oracle."""
     say("sparse plane under a dense plane", key64)
     init, g, c = sparse_plane_scene()
     st = oracle_state(oracle, init)
@@ -466,8 +466,7 @@ def test_step_sparse_plane_under_dense_plane(oracle, key64):
 
 def test_contact_forces_sparse_plane(oracle):
     """sd_contact_forces (unpadded positions, caller's (start, end) ranges) with
-    the multi-chunk candidate staging: forces, torques and history equal the
-    oracle's."""
+    candidates read by each lane: forces, torques and history equal the oracle's."""
     say("contact_forces sparse plane")
     init, g, c = sparse_plane_scene()
     st = oracle_state(oracle, init)
@@ -486,8 +485,10 @@ def test_contact_forces_sparse_plane(oracle):
 
 
 # candidates of a row of cells around the ends of a staged chunk (157 tested a
-# chunk in the force entry point, 189 in a step), and of two
-@pytest.mark.parametrize("m", [63, 65, 154, 157, 158, 160, 186, 189, 190, 192, 314, 315, 378, 379])
+# chunk in the force entry point, 189 in a step), of two, and around the most that
+# is staged (474 and 570)
+@pytest.mark.parametrize("m", [63, 65, 154, 157, 158, 160, 186, 189, 190, 192, 314, 315, 378, 379, 473, 474, 475,
+                               570, 571, 700])
 def test_candidates_at_chunk_ends(oracle, m):
     say("candidates at chunk ends", m)
     rng = np.random.default_rng(m)
@@ -515,3 +516,40 @@ def test_candidates_at_chunk_ends(oracle, m):
     assert np.array_equal(got["hcount"], exp["hcount"])
     assert np.array_equal(got["force"], exp["force"])
     assert np.array_equal(got["torque"], exp["torque"])
+
+
+@pytest.mark.parametrize("around", [11, 12, 13, 15, 16, 17, 40])
+def test_contacts_beyond_the_history(oracle, around):
+    """One sphere with up to and more contacts than are spread over the wave (12)
+    and than its history holds (16): all their forces count, the overflow is reported."""
+    say("contacts beyond the history", around)
+    rng = np.random.default_rng(around)
+    d = rng.normal(size=(around, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    pos = np.concatenate([[[0.05, 0.05, 0.05]], 0.05 + 0.0176 * d, rng.uniform(0.08, 0.1, (60, 3))]).astype(np.float32)
+    rad = np.concatenate([[0.015], np.full(around + 60, 0.003)]).astype(np.float32)
+    vel = rng.normal(0, 0.3, pos.shape).astype(np.float32)
+    g = L.Grid.make((0.0, 0.0, 0.0), 0.03, (4, 4, 4))
+    c = L.ContactParams.make(1e3, 0.3, 0.5, 1e-5, walls=None, max_contacts=16)
+    init = {"x": pos[:, 0].copy(), "y": pos[:, 1].copy(), "z": pos[:, 2].copy(), "r": rad, "m": W.sphere_mass(rad),
+            "vx": vel[:, 0].copy(), "vy": vel[:, 1].copy(), "vz": vel[:, 2].copy()}
+    st = oracle.SphereState(init["x"], init["y"], init["z"], rad, init["m"], vx=init["vx"], vy=init["vy"],
+                            vz=init["vz"], max_contacts=16)
+    s = sorted_state(oracle, st, g)
+    exp = oracle.contact_forces(s["pos4"], s["vel4"], s["omg4"], s["ids"], g, s["ranges"], c, s["old_slot"],
+                                st.hcount, st.hist, nthreads=1)
+    got = gpu_contact_forces(s, st, g, c)
+    assert exp["max_contacts"] >= around
+    assert (got["overflow"] > 16) == (exp["max_contacts"] > 16)
+    assert np.array_equal(got["hcount"], exp["hcount"])
+    eh = exp["hist"].reshape(c.max_contacts, -1, 4)
+    assert np.array_equal(valid_hist(got["hist"], got["hcount"]).view(np.uint32),
+                          valid_hist(eh, exp["hcount"]).view(np.uint32))
+    assert np.array_equal(got["force"], exp["force"])
+    assert np.array_equal(got["torque"], exp["torque"])
+    if exp["max_contacts"] <= 16:
+        sc = make_scene(init, g, c, key64=True, graph=False)
+        sc.step(1)
+        st.step(g, c, nsteps=1, nthreads=8)
+        compare_scene(sc, st)
+        sc.close()
