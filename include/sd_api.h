@@ -245,7 +245,7 @@ sd_status sd_ctx_step(sd_ctx* ctx, int nsteps);
  * previous step, else the radix sort (all passes),
  * and the positions are then permuted within [1]; [2] is empty. */
 sd_status sd_ctx_profile(sd_ctx* ctx, int nsteps, float* stage_ms, int nstages);
-/* Spheres that changed cell in the last step (u64 keys; 0 with u32 keys):
+/* Spheres that changed cell in the last step (0 after an upload or load):
  * *full_next = 1 if the next step uses the full radix sort (more than 1024
  * changes, or one in 256 up to 16384 of more than 262,144 spheres, or after
  * upload / load), else 0. Diagnostic with no counterpart in
@@ -283,8 +283,8 @@ sd_status sd_ctx_load(sd_ctx* ctx, const void* buffer, size_t bytes);
 sd_status sd_ctx_remove_spheres(sd_ctx* ctx, const int* ids, int count);
 sd_status sd_ctx_add_spheres(sd_ctx* ctx, int count, const float* x, const float* y, const float* z, const float* vx,
                              const float* vy, const float* vz, const float* radius, const float* mass);
-/* Persistent form of the fused step kernel (contexts with packed 64-bit keys,
- * single-scene or batch): instead of one 64-slot wave per launched wave, a
+/* Persistent form of the fused step kernel (batch contexts, and single scenes
+ * created with key64 = 1; others are refused): instead of one 64-slot wave per launched wave, a
  * grid of resident workgroups (the occupancy limit times the CUs) whose waves
  * claim runs of eight 64-slot tiles from one counter per XCD (the XCD's eighth
  * of the slots) until they run out. Results are bit-identical to the default form; the

@@ -120,7 +120,7 @@ struct sd_ctx {
     float4* hist[2] = {nullptr, nullptr};
     int cur_hist = 0;
     StepCtl* ctl = nullptr;
-    // spheres that changed cell in the last step (u64 keys): count (set above
+    // spheres that changed cell in the last step: count (set above
     // the cap to force the full sort), new and old keys, and the same sorted
     int* mcount = nullptr;
     uint64_t* mnew = nullptr;
@@ -1124,9 +1124,6 @@ extern "C" sd_status sd_ctx_contact_count(sd_ctx* c, long long* count) {
 extern "C" sd_status sd_ctx_cell_changes(sd_ctx* c, int* count, int* full_next) {
     SD_REQUIRE(c && count && full_next, "sd_ctx_cell_changes: NULL");
     if (c->n == 0) return set_error(SD_ERR_STATE, "sd_ctx_cell_changes: no spheres uploaded");
-    *count = 0;
-    *full_next = c->p.key64 ? 0 : 1;
-    if (!c->p.key64) return SD_OK;
     int m = 0;  // written by the last step, read by the next one
     SD_HIP(hipMemcpyAsync(&m, c->mcount + c->cur_hist, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     SD_HIP(hipStreamSynchronize(c->stream));

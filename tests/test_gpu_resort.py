@@ -53,3 +53,33 @@ def test_large_resort(oracle, n, speed, shear):
     assert all(full == (c > limit) for c, full in counts)
     assert max(c for c, _ in counts) > 500  # (the band of the shear case has crossed after a few steps)
     sc.close()
+
+
+@pytest.mark.parametrize("speed", [3.0, 150.0])
+def test_cell_changes_of_either_key_width(speed):
+    """Contexts of 32-bit and of 64-bit keys step alike and report the same changes."""
+    print("[gpu-case] cell changes by key width", speed, flush=True)
+    rng = np.random.default_rng(17)
+    n, cell, m = 20000, 0.02, 28
+    p = (rng.uniform(0.02, m - 0.02, (n, 3)) * cell).astype(np.float32)
+    r = rng.uniform(0.0005, 0.0015, n).astype(np.float32)
+    v = rng.normal(0, speed, (n, 3)).astype(np.float32)
+    hi = (m * cell,) * 3
+    cols = [np.ascontiguousarray(a) for a in (*p.T, *v.T)]
+    law = L.ContactParams.make(1e3, 0.3, 0.5, 1e-5, walls=((0, 0, 0), hi), max_contacts=16)
+    got = []
+    for key64 in (False, True):
+        sc = SphereScene(W.grid_for((0, 0, 0), hi, cell), law, key64=key64)
+        sc.upload(*cols[:3], r, W.sphere_mass(r), vx=cols[3], vy=cols[4], vz=cols[5])
+        seen = [sc.cell_changes()]
+        for k in (1, 2, 7):
+            sc.step(k)
+            seen.append(sc.cell_changes())
+        sc.load(sc.save())
+        seen.append(sc.cell_changes())
+        got.append(seen)
+        sc.close()
+    assert got[0] == got[1]
+    assert got[0][0] == got[0][-1] == (0, True)
+    assert all(c > 0 and full == (c > 1024) for c, full in got[0][1:-1])
+    assert got[0][-2][1] == (speed > 100.0)
