@@ -269,8 +269,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev, bool full, int lists) {
     int* mc_read = c->mcount + ho;
     int* mc_write = c->mcount + hn;
     if (full) {
-        st = radix_sort_keys_u64_gated(&K, &Ka, n, 32, 32 + c->key_bits, c->sort_tmp, c->sort_tmp_bytes, s,
-                                       c->items, nullptr, 0);
+        st = radix_sort_keys_u64_odd(&K, &Ka, n, 32, 32 + c->key_bits, c->sort_tmp, c->sort_tmp_bytes, s, c->items);
     } else {
         // also updates the cell starts and sets mc_write = 0
         st = launch_resort_u64(mc_read, resort_cap(n), c->mnew, c->mold, c->msn, c->mso, K, n, c->cell_start, c->n_cells,
@@ -293,7 +292,7 @@ sd_status enqueue_step(sd_ctx* c, hipEvent_t* ev, bool full, int lists) {
     }
     // after the full sort: cell starts, the permutation, mc_write = 0
     if (full) st = launch_step_starts_u64(K, n, c->n_cells, c->cell_start, &c->ctl->given_up, true, c->pos[so],
-                                          c->posB, mc_write, nullptr, c->ctl, lists, c->list_cell, s);
+                                          c->posB, mc_write, c->ctl, lists, c->list_cell, s);
     if (st != SD_OK) return st;
     MARK(2);
     MARK(3);

@@ -169,7 +169,7 @@ __device__ __forceinline__ void fill_cell_starts(int* __restrict__ start, int lo
 template <typename K, int SHIFT>
 __global__ void k_cell_starts(const K* __restrict__ keys, int n, int n_cells, int* __restrict__ start,
                               const int* __restrict__ skip, int permute, const float4* __restrict__ pos,
-                              float4* __restrict__ pos_o, int* __restrict__ next_count, int* __restrict__ newpos,
+                              float4* __restrict__ pos_o, int* __restrict__ next_count,
                               StepCtl* __restrict__ ctl, int lists, float list_cell) {
     if (skip && *skip) return;
     if (ctl && blockIdx.x == 0 && threadIdx.x < 64) list_begin_step(ctl, lists, list_cell);
@@ -180,10 +180,7 @@ __global__ void k_cell_starts(const K* __restrict__ keys, int n, int n_cells, in
         const K k = keys[i];
         if (permute) {
             const uint32_t src = (uint32_t)k;
-            if (src < (uint32_t)n) {
-                pos_o[i] = pos[src];
-                if (newpos) newpos[src] = i;
-            }
+            if (src < (uint32_t)n) pos_o[i] = pos[src];
         }
         const uint32_t c = min((uint32_t)(k >> SHIFT), (uint32_t)n_cells);
         const uint32_t prev = i == 0 ? 0u : min((uint32_t)(keys[i - 1] >> SHIFT), (uint32_t)n_cells) + 1u;
@@ -199,11 +196,11 @@ __global__ void k_cell_starts(const K* __restrict__ keys, int n, int n_cells, in
 }
 
 sd_status launch_step_starts_u64(const uint64_t* keys, int n, int n_cells, int* start, const int* skip, bool permute,
-                                 const float4* pos, float4* pos_o, int* next_count, int* newpos, StepCtl* ctl,
-                                 int lists, float list_cell, hipStream_t s) {
+                                 const float4* pos, float4* pos_o, int* next_count, StepCtl* ctl, int lists,
+                                 float list_cell, hipStream_t s) {
     if (n <= 0) return launch_fill_u32((uint32_t*)start, 0u, (size_t)n_cells + 1, s);
     hipLaunchKernelGGL((k_cell_starts<uint64_t, 32>), dim3(div_up(n, 256)), dim3(256), 0, s, keys, n, n_cells, start,
-                       skip, permute ? 1 : 0, pos, pos_o, next_count, newpos, ctl, lists, list_cell);
+                       skip, permute ? 1 : 0, pos, pos_o, next_count, ctl, lists, list_cell);
     SD_LAUNCH_CHECK();
     return SD_OK;
 }

@@ -591,7 +591,7 @@ sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s, hipEvent_t ready, con
     st = radix_sort_keys_u64(&K, &Ka, n, 32, 32 + cbits, c->sort_tmp, radix_temp_bytes(n), s, 0);
     if (st == SD_OK)
         st = launch_step_starts_u64(K, n, (int)c->ncells, c->cell_start, nullptr, false, nullptr, nullptr, nullptr,
-                                    nullptr, nullptr, 0, 0.0f, s);
+                                    nullptr, 0, 0.0f, s);
     if (st != SD_OK) return st;
     const HbGridArgs G{(const float4*)c->P,     (const float4*)c->lo,     (const float4*)c->hi,
                        (const int*)c->scene_of, (const HbGrid*)c->grid,   (const int*)c->large,

@@ -22,12 +22,10 @@ sd_status radix_sort_pairs_u32(uint32_t** keys, uint32_t** vals, uint32_t** keys
                                hipStream_t s, int items);
 sd_status radix_sort_keys_u64(uint64_t** keys, uint64_t** keys_alt, int n, int begin_bit, int end_bit,
                               void* temp, size_t temp_bytes, hipStream_t s, int items);
-// As radix_sort_keys_u64, with an odd number of passes (the result always ends
-// in *keys_alt's original buffer) and every kernel skipped on the device while
-// *gate <= gate_cap.
-sd_status radix_sort_keys_u64_gated(uint64_t** keys, uint64_t** keys_alt, int n, int begin_bit, int end_bit,
-                                    void* temp, size_t temp_bytes, hipStream_t s, int items, const int* gate,
-                                    int gate_cap);
+// As radix_sort_keys_u64, with an odd number of passes (the result of two keys
+// or more always ends in *keys_alt's original buffer).
+sd_status radix_sort_keys_u64_odd(uint64_t** keys, uint64_t** keys_alt, int n, int begin_bit, int end_bit, void* temp,
+                                  size_t temp_bytes, hipStream_t s, int items);
 // Number of LSD passes the sort makes over a bit range.
 int radix_passes(int begin_bit, int end_bit);
 
@@ -61,12 +59,11 @@ sd_status launch_cell_ranges_u32(const uint32_t* keys, int n, int n_cells, int* 
 sd_status launch_cell_ranges_u64(const uint64_t* keys, int n, int n_cells, int* ranges, hipStream_t s);
 // Cell starts of sorted keys: start[c] = number of keys whose cell is below c,
 // c = 0 .. n_cells (n_cells + 1 entries), every entry written. Also gathers pos
-// into sorted order (pos_o) with permute, sets *next_count = 0 and
-// newpos[slot] = sorted position, and begins the step's near lists; does
-// nothing while *skip.
+// into sorted order (pos_o) with permute, sets *next_count = 0, and begins the
+// step's near lists; does nothing while *skip.
 sd_status launch_step_starts_u64(const uint64_t* keys, int n, int n_cells, int* start, const int* skip, bool permute,
-                                 const float4* pos, float4* pos_o, int* next_count, int* newpos, StepCtl* ctl,
-                                 int lists, float list_cell, hipStream_t s);
+                                 const float4* pos, float4* pos_o, int* next_count, StepCtl* ctl, int lists,
+                                 float list_cell, hipStream_t s);
 // perm is either u32 values (perm32) or the low halves of u64 keys (perm64).
 sd_status launch_permute(const uint32_t* perm32, const uint64_t* perm64, int n, const float4* pos, const float4* vel,
                          const float4* omg, const int* ids, float4* pos_o, float4* vel_o, float4* omg_o, int* ids_o,
