@@ -244,6 +244,16 @@ __global__ __launch_bounds__(RESORT_MERGE_BLOCK) void k_resort_merge(
     if (use) newpos[s] = d;
 }
 
+// Cells whose starts one of nblocks merge blocks updates: whole rounds of its
+// threads, or all cells (a round more than 2^31 - 1 of them is no int).
+constexpr int merge_cells(int n_cells, int nblocks) {
+    const long long per = ((long long)n_cells + nblocks - 1) / nblocks;
+    const long long rounds = (per + RESORT_MERGE_BLOCK - 1) / RESORT_MERGE_BLOCK * RESORT_MERGE_BLOCK;
+    return (int)(rounds < n_cells ? rounds : n_cells);
+}
+static_assert(merge_cells(0x7fffffff, 1) == 0x7fffffff && merge_cells(0x7ffffe01, 1) == 0x7ffffe01, "no overflow");
+static_assert(merge_cells(1025, 2) == 1024 && merge_cells(1024, 2) == 512 && merge_cells(3, 1) == 3, "whole rounds");
+
 sd_status launch_resort_u64(const int* mcount, int cap, const uint64_t* mnew, const uint64_t* mold,
                             uint64_t* msorted_new, uint64_t* msorted_old, const uint64_t* keys, int n,
                             int* cell_start, int n_cells, const float4* pos_state, float4* posB, uint64_t* keys_out,
@@ -255,7 +265,7 @@ sd_status launch_resort_u64(const int* mcount, int cap, const uint64_t* mnew, co
                        newpos, lists, list_cell);
     SD_LAUNCH_CHECK();
     const int nblocks = div_up(n, RESORT_MERGE_BLOCK);
-    const int cells_per_block = div_up(div_up(n_cells, nblocks), RESORT_MERGE_BLOCK) * RESORT_MERGE_BLOCK;
+    const int cells_per_block = merge_cells(n_cells, nblocks);
     hipLaunchKernelGGL(k_resort_merge, dim3(nblocks), dim3(RESORT_MERGE_BLOCK), 0, s, mcount, cap,
                        (const uint64_t*)msorted_new, (const uint64_t*)msorted_old, keys, n, pos_state, posB, keys_out,
                        cell_start, n_cells, cells_per_block, next_count, (const StepCtl*)ctl, newpos, lists);
