@@ -572,8 +572,12 @@ sd_status hb_check_params(const sd_hull_params* p) {
 
 namespace sd {
 
-// One step of the context, enqueued on s (no host synchronisation).
-sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s, hipEvent_t ready, const int* given_up) {
+sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s) {
+    const sd_status st = hull_enqueue_forces(c, s);
+    return st == SD_OK ? hull_enqueue_move(c, s, nullptr) : st;
+}
+
+sd_status hull_enqueue_forces(sd_hull_ctx* c, hipStream_t s) {
     const int n = c->n, cap = c->capacity;
     const int mi = c->p.max_iter ? c->p.max_iter : 64;
     hipLaunchKernelGGL(k_hb_pose, dim3(div_up(n, 256)), dim3(256), 0, s, (const float4*)c->P, (const float4*)c->Q,
@@ -627,7 +631,11 @@ sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s, hipEvent_t ready, con
                        (const int*)c->total, (const float4*)c->P, (const float4*)c->pf, (const int*)c->offs, c->fillc,
                        c->list);
     SD_LAUNCH_CHECK();
-    if (ready) SD_HIP(hipStreamWaitEvent(s, ready, 0));
+    return SD_OK;
+}
+
+sd_status hull_enqueue_move(sd_hull_ctx* c, hipStream_t s, const int* given_up) {
+    const int n = c->n;
     hipLaunchKernelGGL(k_hb_gather_integrate, dim3(div_up(n, 256)), dim3(256), 0, s, given_up, n,
                        (const int*)c->offs, (const int*)c->cnt, (const int*)c->list, (const float4*)c->pf,
                        (const float4*)c->pp, c->P, c->V, c->Q, c->L, (const float4*)c->I0, (const float4*)c->I1, c->c,

@@ -245,10 +245,12 @@ sd_status prepare_rigid(const char* who, int nb, const float* pos4, const float*
 // Rigid-body context (sd_hull_ctx, sd_hullbody.hip): one step enqueued on s
 // with no host synchronisation; device errors of the steps since the last
 // check; accessors used by a batch context that steps the bodies with its
-// scenes. given_up (nullable): the bodies are moved only if *given_up is 0 after
-// the event `ready` (nullable); nothing that outlives the step is written before.
-sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s, hipEvent_t ready = nullptr,
-                            const int* given_up = nullptr);
+// scenes. A step is two parts: the forces, which write nothing that outlives the
+// step, and the move, which with *given_up (nullable) leaves the bodies as they
+// are.
+sd_status hull_enqueue_step(sd_hull_ctx* c, hipStream_t s);
+sd_status hull_enqueue_forces(sd_hull_ctx* c, hipStream_t s);
+sd_status hull_enqueue_move(sd_hull_ctx* c, hipStream_t s, const int* given_up);
 sd_status hull_check_errors(sd_hull_ctx* c);
 int hull_body_count(const sd_hull_ctx* c);
 // Changes whenever the context's step changes (upload, parameters, warm start).
