@@ -2,7 +2,10 @@
 every step: lists that run out and are built again, scenes whose spheres are as
 wide as their cell (pairs two cells apart can come into contact while a list
 lasts), spheres with more contacts than are spread over the wave and more neighbours
-than a list holds, static spheres, waves with a few lanes, batches. Exact."""
+than a list holds, static spheres, waves with a few lanes, batches, coordinates far
+from the origin, edits and loaded states. Exact."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -121,7 +124,8 @@ def test_batch_of_speeds(oracle):
 
 
 def test_edits_and_states_drop_the_lists(oracle):
-    """A loaded state, removed and added spheres and another law start from new lists."""
+    """A loaded state, removed and added spheres start from new lists; another law
+    keeps them (what bounds them is how far the spheres moved)."""
     p, v, r, g, walls = gas(2000, 0.004, 0.01, 0.02, 0.5, 0.12, 3)
     c = law(walls)
     cols = [np.ascontiguousarray(a) for a in (*p.T, *v.T)]
@@ -143,4 +147,63 @@ def test_edits_and_states_drop_the_lists(oracle):
     sc.step(25)
     st.step(g, c, nsteps=25, nthreads=8)
     compare(sc.download(), st.by_id())
+    more = [np.ascontiguousarray(a[3:400:7]) for a in cols]
+    sc.add(*more[:3], r[3:400:7], W.sphere_mass(r[3:400:7]), vx=more[3], vy=more[4], vz=more[5])
+    st.add(*more[:3], r[3:400:7], W.sphere_mass(r[3:400:7]), vx=more[3], vy=more[4], vz=more[5])
+    for kn, dt in ((1e3, 1e-5), (4e3, 2e-5), (5e2, 5e-6)):
+        c = L.ContactParams.make(kn, 0.2, 0.4, dt, walls=walls, max_contacts=MAXC)
+        L.call("sd_ctx_set_contact", sc.h, C.byref(c))
+        sc.step(25)
+        st.step(g, c, nsteps=25, nthreads=8)
+        compare(sc.download(), st.by_id())
     sc.close()
+
+
+def test_radii_beyond_the_cell(oracle):
+    """A loaded state with a sphere wider than its cell keeps no lists (the search
+    of 27 cells is the oracle's); the state without it has them again."""
+    print("[gpu-case] near lists, radii beyond the cell", flush=True)
+    p, v, r, g, walls = gas(2000, 0.004, 0.01, 0.02, 0.5, 0.12, 5)
+    c = law(walls)
+    cols = [np.ascontiguousarray(a) for a in (*p.T, *v.T)]
+    sc = SphereScene(g, c, key64=True)
+    sc.upload(*cols[:3], r, W.sphere_mass(r), vx=cols[3], vy=cols[4], vz=cols[5])
+    sc.step(20)
+    small = sc.save()
+    n, head = sc.n, small.nbytes - sc.n * (52 + 8 + 4 + 16 * MAXC)  # header; rows, ids, keys, counts, history
+    ids = small[head + 48 * n:head + 52 * n].view(np.int32)
+
+    def oracle_of(buf):
+        st = oracle.SphereState(*cols[:3], r, W.sphere_mass(r), max_contacts=MAXC)
+        rows = buf[head:head + 48 * n].view(np.float32).reshape(3, n, 4).copy()
+        st.pos4, st.vel4, st.omg4, st.ids = rows[0], rows[1], rows[2], ids.copy()
+        st.hcount = buf[head + 60 * n:head + 64 * n].view(np.int32).copy()
+        st.hist = buf[head + 64 * n:].view(np.float32).reshape(-1, 4).copy()
+        return st
+
+    wide = small.copy()
+    wide[head:head + 48 * n].view(np.float32).reshape(3, n, 4)[0, ::97, 3] = 0.0137
+    for buf in (wide, small, wide):
+        sc.load(buf)
+        st = oracle_of(buf)
+        for k in (1, 30):
+            sc.step(k)
+            st.step(g, c, nsteps=k, nthreads=8)
+            compare(sc.download(), st.by_id())
+    sc.close()
+
+
+# coordinates whose rounding is a thousandth of a radius and more; a grid of more
+# than 65,536 cells a side, where every pair's cells are looked at
+@pytest.mark.parametrize("off,nx", [(4000.0, 0), (65000.0, 0), (1300.0, 70000)])
+def test_lists_far_from_the_origin(oracle, off, nx):
+    print("[gpu-case] near lists, far from the origin", off, nx, flush=True)
+    cell = 0.02 if nx else 0.5
+    lo = (off, -0.5 * off if not nx else 0.0, 0.0)
+    p, v, r, g, walls = gas(2000, 0.4 * cell, 0.5 * cell, cell, 20.0, 0.12, 9, lo)
+    if nx:
+        hi = (nx * cell, *walls[1][1:])
+        walls = ((0.0, 0.0, 0.0), hi)
+        g = L.Grid.make((0.0, 0.0, 0.0), cell, (nx, *[max(1, int(np.ceil(a / cell))) for a in hi[1:]]))
+    r = np.minimum(r, np.float32(0.5 * cell))
+    run(oracle, p, v, r, W.sphere_mass(r), g, law(walls), (1, 2, 40, 90))
