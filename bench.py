@@ -59,13 +59,14 @@ sys.path.insert(0, ROOT)
 
 METRIC = "particle-steps/s and GJK pairs/s, batched+learned vs plain, 1×MI355X"
 HBM_PEAK_GBS = 8000.0
+LONG_STEPS = 400
 
-# HBM bytes per launch of the dominant kernel, from rocprofv3 FETCH_SIZE / WRITE_SIZE
+# HBM bytes per launch of the dominant kernel in a step on near lists, from rocprofv3 FETCH_SIZE / WRITE_SIZE
 # runs on MI355X (FETCH x 2.0 + WRITE x 1.0 KiB, factors from the plain copy kernel);
 # the runs and the counters are in profiles/contact_kernel_c2_counters.md.
 MEASURED_TRAFFIC = {
-    ("dem_c2_column_4194304", "contact"): (136485.2 * 2.0 + 262144.0) * 1024.0,
-    ("dem_c2_dense_4194304", "contact"): (1475726.9 * 2.0 + 717303.8) * 1024.0,
+    ("dem_c2_column_4194304", "contact"): (183317.0 * 2.0 + 278451.2) * 1024.0,
+    ("dem_c2_dense_4194304", "contact"): (1060276.6 * 2.0 + 692045.9) * 1024.0,
 }
 
 
@@ -73,33 +74,18 @@ def log(*a):
     print("[bench]", *a, file=sys.stderr, flush=True)
 
 
-def stage_bytes(w, n, contacts_per_sphere, n_cells):
-    """Algorithmic (compulsory) HBM bytes per launch of each stage."""
-    import math
-    key_b = 8 if w.key64 else 4
-    val_b = 0 if w.key64 else 4
-    bits = max(1, int(math.ceil(math.log2(n_cells))))
-    passes = (bits + 7) // 8
-    c = contacts_per_sphere
-    if w.key64:
-        # re-sort from the previous order: read keys and pos4, write sorted keys
-        # and pos4; the permutation and the cell-start update ride on it (the
-        # changed-cell lists are tiny and only cells between a changed sphere's
-        # old and new cell are rewritten)
-        sort_b, ranges_b, permute_b = n * 2 * (key_b + 16), 0, 0
-    else:
-        # one histogram read of the keys, then per pass read + write of keys and
-        # values; cell starts: read every sorted key once, write the start of
-        # every cell; permute: read the permutation, gather pos4, write sorted pos4
-        sort_b = n * (key_b + passes * 2 * (key_b + val_b))
-        ranges_b, permute_b = n * key_b + 4 * (n_cells + 1), n * ((key_b + val_b) + 2 * 16)
+def stage_bytes(n, contacts_per_sphere):
+    """Algorithmic (compulsory) HBM bytes per launch of each stage of a step on near lists."""
     return {
-        "sort": sort_b,
-        "ranges": ranges_b,
-        "permute": permute_b,
+        # re-sort from the previous order: keys read and written sorted, every
+        # sphere's new place written (the changed-cell lists are tiny, and only
+        # cells between a changed sphere's old and new cell are rewritten)
+        "sort": n * (2 * 8 + 4),
+        "ranges": 0,
+        "permute": 0,
         # own state 52 B + old slot + history count in/out 8 B + state out 52 B + next key;
         # per contact: old history row 16 B read + new row 16 B written
-        "contact": n * (52 + (key_b + val_b) + 8 + 52 + (key_b + val_b)) + n * c * 32,
+        "contact": n * (52 + 8 + 8 + 52 + 8) + n * contacts_per_sphere * 32,
     }
 
 
@@ -576,8 +562,9 @@ def calibrate_copy(nbytes=256 << 20, reps=5):
 
 def sphere_run(w, steps, warmup, autotune, profile_steps, s=None):
     """Times `steps` graph-replayed steps of sphere workload w (after the
-    autotuner and `warmup` steps), then profiles the stages eagerly. Returns
-    the measurements and the generated arrays."""
+    autotuner and `warmup` steps), then profiles the stages eagerly and times
+    LONG_STEPS more, which hold several builds of the near lists however few
+    `steps` are. Returns the measurements and the generated arrays."""
     import ctypes
 
     from stardust_amd import _lib as L
@@ -621,29 +608,37 @@ def sphere_run(w, steps, warmup, autotune, profile_steps, s=None):
     prof = sc.profile(profile_steps)
     per_launch = {k: v / profile_steps for k, v in prof.items()}
     log("per-step stage ms:", {k: round(v, 4) for k, v in per_launch.items()})
-    sbytes = stage_bytes(w, w.n, contacts / w.n, g.n_cells)
+    sbytes = stage_bytes(w.n, contacts / w.n)
     dominant = max(per_launch, key=per_launch.get)
     achieved = sbytes[dominant] / (per_launch[dominant] / 1000.0) / 1e9
     stages = {k: {"ms": round(per_launch[k], 5), "bytes": int(sbytes[k]),
                   "GBs": round(sbytes[k] / (per_launch[k] / 1000.0) / 1e9, 1) if per_launch[k] > 0 else None}
               for k in per_launch}
+    L.synchronize(stream)
+    t0 = time.perf_counter()
+    sc.step(LONG_STEPS)
+    L.synchronize(stream)
+    long_t = time.perf_counter() - t0
+    log("%d steps more: %.3f s -> %.3e particle-steps/s" % (LONG_STEPS, long_t, w.n * LONG_STEPS / long_t))
     sc.close()
-    r = {"value": value, "t": t, "tune": tune, "grid": g, "contacts": contacts, "changes": changes,
+    long_run = {"steps": LONG_STEPS, "ms_per_step": round(1000.0 * long_t / LONG_STEPS, 5),
+                "particle_steps_per_s": w.n * LONG_STEPS / long_t}
+    r = {"long_run": long_run, "value": value, "t": t, "tune": tune, "grid": g, "contacts": contacts, "changes": changes,
          "full_next": full_next, "diag": diag, "stages": stages, "dominant": dominant, "achieved": achieved,
          "sbytes": sbytes}
     return r, s
 
 
 def c1_section(args):
-    """dem_c1 (65,536 spheres, u32 cell keys, the full radix sort every step):
-    particle-steps/s of the graph-replayed step and its stages."""
+    """dem_c1 (65,536 spheres, a context of 32-bit keys): particle-steps/s of the
+    graph-replayed step and its stages."""
     from stardust_amd import workloads as W
     w = W.dem_c1()
     steps = args.steps if args.steps is not None else 1000
     r, _ = sphere_run(w, steps, args.warmup, not args.no_autotune, args.profile_steps)
     return {"workload": w.name, "spheres": w.n, "steps": steps, "ms_per_step": round(1000.0 * r["t"] / steps, 4),
             "particle_steps_per_s": r["value"], "contacts_per_sphere": r["contacts"] / w.n,
-            "launch_shapes": r["tune"], "stages": r["stages"]}
+            "long_run": r["long_run"], "launch_shapes": r["tune"], "stages": r["stages"]}
 
 
 def c2_dense_section(args):
@@ -657,7 +652,7 @@ def c2_dense_section(args):
     dom = r["dominant"]
     return {"workload": w.name, "spheres": w.n, "steps": steps, "ms_per_step": round(1000.0 * r["t"] / steps, 4),
             "particle_steps_per_s": r["value"], "contacts_per_sphere": r["contacts"] / w.n,
-            "cells": r["grid"].n_cells, "launch_shapes": r["tune"], "stages": r["stages"],
+            "long_run": r["long_run"], "cells": r["grid"].n_cells, "launch_shapes": r["tune"], "stages": r["stages"],
             "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(r["achieved"], 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(r["achieved"] / HBM_PEAK_GBS, 4),
                          "traffic": MEASURED_TRAFFIC.get((w.name, dom)), "algorithmic_bytes": r["sbytes"][dom]},
@@ -928,6 +923,7 @@ def main():
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(r["achieved"] / HBM_PEAK_GBS, 4),
                      "traffic": MEASURED_TRAFFIC.get((w.name, r["dominant"])),
                      "algorithmic_bytes": r["sbytes"][r["dominant"]]},
+        "long_run": r["long_run"],
         "stages": r["stages"],
         "contacts_per_sphere": r["contacts"] / w.n,
         "cell_changes_last_timed_step": {"spheres": r["changes"], "full_sort_next": r["full_next"]},

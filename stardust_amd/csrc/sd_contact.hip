@@ -175,9 +175,9 @@ __device__ __forceinline__ T uniform_copy(const T& src) {
 // sphere, and the loads of 64 contacts are in flight together. (3) Every lane
 // adds up its sphere's forces in order.
 //
-// A step on lists moves about 200 bytes a sphere (state in and out, keys,
-// history count, a list row or two) and is bound by that in a dilute scene:
-// 4,194,304 spheres 181 us, where the search of every step took 312 (VALU
+// A step on lists moves 157 bytes a sphere at rest (state in and out, keys,
+// history count, a list row or two; 661 MB by the counters) and is bound by that
+// in a dilute scene, at 4.6 TB/s: 4,194,304 spheres 143 us, 181 at 0.5 m/s, where the search of every step took 312 (VALU
 // issue, 97 candidate tests a sphere). With 2 to 3 contacts a sphere the chain
 // of loads of a contact counts: 1,048,576 spheres 154 us (215 when each lane
 // went through its own contacts), 1,000 spheres 18 us (51). A step that makes

@@ -211,7 +211,7 @@ sd_status launch_contacts_straddle(const ContactArgs& a, hipStream_t s);
 // keys_out and the positions in that order to posB, turns cell_start (the
 // previous order's cell starts, n_cells + 1 entries) into the new order's and
 // sets *next_count = 0. With *mcount > cap (= resort_cap(n)) it gives the step up instead
-// (step_ctl[0] = 1).
+// (ctl->given_up).
 // Most changed cells a re-sort takes: 1,024, and one sphere in 256 of larger
 // scenes up to 16,384. Ranking the movers grows with their square and the
 // radix sort it saves with n: at 4,194,304 spheres a re-sort of 1,000 movers

@@ -66,8 +66,9 @@ __global__ __launch_bounds__(256) void k_gather_soa(const float4* __restrict__ p
 }
 
 // Rows per chunk: about 1 MB of slot, so that the staging stays near 14 MB and
-// a chunk's transfer (20 us) covers its launch. Whole sphere states: 4,194,304
-// spheres 96 -> 4.6 ms (33 GB/s; the link does 56), 250,007 4.6 -> 0.40 ms,
+// a chunk's transfer (20 us) covers its launch. Whole sphere states into arrays
+// in use (pages touched for the first time: 4,194,304 spheres 111 -> 12 ms):
+// 4,194,304 spheres 96 -> 4.6 ms (33 GB/s; the link does 56), 250,007 4.6 -> 0.40 ms,
 // 65,536 0.55 -> 0.11 ms, 1,000 0.09 -> 0.03 ms, against copies of the rows to
 // pageable memory and a scatter by id on the host.
 constexpr int SPHERE_CHUNK = 32768;
