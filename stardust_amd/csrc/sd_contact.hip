@@ -733,7 +733,7 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
         }
         const float ox = p.x, oy = p.y, oz = p.z;
         integrate_sphere(c, p, v, w, fx, fy, fz, tx, ty, tz);
-        {
+        if (LISTS != LIST_NONE || a.list_new) {  // (a context without lists needs none)
             const float dx = p.x - ox, dyy = p.y - oy, dzz = p.z - oz;
             note_displacement(a.ctl, live ? dx * dx + dyy * dyy + dzz * dzz : 0.0f);
         }
@@ -767,8 +767,11 @@ __device__ __forceinline__ void contact_wave(const ContactArgs& a, int slot) {
 }
 
 
+// Six waves a SIMD for the kernels that only search (a batch's takes 81 registers
+// otherwise, one too many: 1.83M spheres of 128 scenes 195 us a step, 187 with one
+// spilled; beside a body step 2.00 ms, 1.98).
 template <int MODE, bool INDIRECT, bool STRADDLE, int LISTS>
-__global__ __launch_bounds__(256) void k_contacts(ContactArgs a) {
+__global__ __launch_bounds__(256, (LISTS == LIST_NONE && !STRADDLE ? 6 : 1)) void k_contacts(ContactArgs a) {
     static_assert(!STRADDLE || MODE == CONTACT_FUSED_BATCH, "k_contacts: straddling waves exist in batch mode only");
     static_assert(LISTS == LIST_NONE || INDIRECT, "k_contacts: only a context's steps have lists");
     if (MODE != CONTACT_FORCES) {

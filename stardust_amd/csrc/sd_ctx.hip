@@ -383,11 +383,11 @@ sd_status run_graph_pair(sd_ctx* c, bool full, int lists) {
 // attached (the bodies' part of a given-up step would be computed twice), or
 // where it cannot be had. A scene that fits without lists then steps without.
 void alloc_lists(sd_ctx* c) {
-    if (c->hulls) {
-        if (c->list_mem) (void)hipFree(c->list_mem);
-        c->list_mem = nullptr;
-    }
-    if (c->hulls || c->list_mem) return;
+    if (c->list_mem && !c->hulls) return;
+    if (c->list_mem) (void)hipFree(c->list_mem);
+    c->list_mem = nullptr;
+    c->list[0] = c->list[1] = nullptr;
+    if (c->hulls) return;
     const size_t n = (size_t)c->n, list = LIST_CAP * n * sizeof(int);
     if (hipMalloc((void**)&c->list_mem, 2 * list + n * sizeof(int) + 2 * n) != hipSuccess) {
         (void)hipGetLastError();

@@ -185,10 +185,10 @@ struct ContactArgs {
     // registers); launch_contacts_straddle runs them with per-lane parameters.
     const int* straddle;
     int n_straddle;
-    // fused modes: near lists (entry k of slot s at k * n + s; the old ones in
-    // the previous step's order, with newpos[old position] = position), what
-    // the step does with them (LIST_*), and the largest radius (per scene in
-    // batch mode)
+    // fused modes: near lists (list_new NULL: the context has none; entry k of
+    // slot s at k * n + s; the old ones in the previous step's order, with
+    // newpos[old position] = position), what the step does with them (LIST_*),
+    // and the largest radius (per scene in batch mode)
     int lists;
     const uint8_t* lcount_old;
     const int* list_old;
